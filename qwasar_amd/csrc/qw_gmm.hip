@@ -1,31 +1,579 @@
-// qw_gmm.hip -- the grouped (per-expert) 4-bit GEMM for prefill, on gfx950
-// MFMA (v_mfma_f32_16x16x32_f16), and its dense twin for the shared expert.
+// qw_gmm.hip -- the 4-bit products over many rows, on gfx950 MFMA: the dense
+// projection (qw_op_qmm_q4) and the grouped per-expert product of the
+// reference's op sequence (qw_op_qmm_q4_gather).  One kernel, two steps:
 //
-// Per workgroup: one tile of up to BM pairs routed to one expert (gathered
-// through perm) against a 64-row block of that expert's weights.  Four waves
-// each own 16 weight rows and all BM token rows.
+//   k_xstage  the activation rows once as f16 (and each quantisation group's
+//             sum), so that the product's many column blocks do not convert
+//             them again
+//   k_xgemm   the product
 //
-// Exactness of the weight operand.  A nibble q is fed to the MFMA as the f16
-// value 1024 + q, which is exact, built from the packed word with one shift
-// and one and-or per pair ((w >> 4j) & 0x000F000F | 0x64006400).  The MFMA
-// sums (1024 + q) * x over one quantisation group in fp32; the group's affine
-// map is applied afterwards on the fp32 partial:
+// Exactness of the weight operand.  A nibble q enters the MFMA as the f16
+// denormal q 2^-24 (nibbles 0, 2, 4, 6 of a word) or q 2^-20 (nibbles 1, 3,
+// 5, 7), which is the masked word itself: two ands, a shift, two ands a word
+// and no rounding (gfx950's f16 MFMA multiplies denormals exactly).  The
+// staged activations at the odd positions are 2^-4 of the others', so all
+// products of a group carry one scale.  The group's scale is applied to the
+// fp32 partial of its MFMAs:
 //
-//   sum_i (s q_i + b) x_i = s * C_g + (b - 1024 s) * X_g,
-//   C_g = sum_i (1024 + q_i) x_i,   X_g = sum_i x_i
+//   y = sum_g s_g C_g + sum_g b_g X_g,   C_g = sum q x,   X_g = sum x,
 //
-// so the weights enter with no rounding at all.  Activations are rounded to
-// f16 (relative error <= 2^-11 per element) -- the only approximation.
+// and the second sum is a product of its own: the biases (bf16, as stored)
+// against X_g cut into three bf16 parts (24 bits: exactly), 16 groups' parts
+// in two bf16 MFMAs.  So the weights enter with no rounding at all;
+// activations are rounded to f16 (relative error <= 2^-11 an element), the
+// only approximation.
 //
-// k order within an MFMA.  The shift-and-or above leaves a word's nibbles in
-// register order 0,4,1,5,2,6,3,7; the activation tile is written to LDS in
-// the same order within every 8-element block, so A and B agree.
+// k order within an MFMA.  The masks leave a word's nibbles in register order
+// 0,4,1,5,2,6,3,7; the stage stores every 8-element block in that order.
+//
+// What bounds it.  Dense, many rows: the vector unit's work beside the matrix
+// cores (per 64 k of a 16-column tile of a 64-row wave: 8 MFMAs of 16 cycles
+// against 16 multiply-adds for the scale and 10 operations for the masks; the
+// two units overlap by about half, as a loop of nothing else shows), so the
+// product runs at about half of a matrix library's f16 rate.  1024 x 3072 x
+// 10240: 96 us a call (670 TFLOP/s), where 64 x 64 tiles that converted the
+// activations in every column block and put 1024 + q through the MFMA took
+// 275.  Timing builds: without the loads of the stages 80 us, without their
+// arithmetic 50.  Experts with few pairs: requests to L1.  A load of 64 lanes
+// over 16 rows touches 16 lines, whatever it fetches, so the scales (and for
+// narrow tiles the biases) come as one flat run of the block's columns, and
+// the weights 128 bytes of a column a load where a tile is narrow: gate, up
+// and down of 512 experts of 640 x 2560, 6 pairs each, 1650 -> 420 us.
+// Both operands go straight to LDS (global_load_lds, 16-byte pieces, no
+// registers), NST - 1 stages ahead, one barrier a stage, two workgroups a CU.
+// Tried: every LDS read of a stage ahead of its MFMAs, and MFMAs interleaved
+// with the vector work by hand: no faster (90 and 93 us the kernel).
 #include "qw_device.h"
 #include "qw_kernels.h"
 
 typedef _Float16 qw_h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 qw_b8 __attribute__((ext_vector_type(8)));
 typedef float qw_f4 __attribute__((ext_vector_type(4)));
 
+#define QX_KPAD 256              // staged rows are padded with zeros to a multiple of this
+#define QX_SB 16                 // groups a block of the staged sums
+#define QX_SLOTS 512             // workgroups the chip holds at two a CU
+#define QX_WIDE_K 1024           // rows of at least this many elements are staged by a workgroup each
+#define QX_CHUNK_ROWS 8192       // rows a dense call stages at a time (bounds its scratch)
+
+// ---- staging -------------------------------------------------------------------
+
+// W waves a row (one under QX_WIDE_K elements, else the workgroup's four: a
+// lane's blocks of 8 stay in registers up to NI of them, so the row is read
+// once).  The row is scaled by one power of two 2^sh that puts its largest
+// magnitude in [2^14, 2^15), so no input overflows f16; ex gets 24 - sh, the
+// exponent the product's sums are scaled back by (24 from the denormal
+// nibbles).  xp holds a row's sums of the staged values 2^-24, 16 groups at a
+// time: [block][part 0..2, zeros][16].  1021 rows of 12288: a wave a row and
+// two reads took 24 us.
+template <int G, int W, int NI>
+__global__ __launch_bounds__(256) void k_xstage(_Float16 *__restrict__ ah, uint16_t *__restrict__ xp,
+                                                int *__restrict__ ex, const float *__restrict__ x, int rows, int k,
+                                                int kp, int nsb)
+{
+    constexpr int L = 64 * W;                                    // lanes a row
+    __shared__ float wm[4];
+    const int row = W == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x, lane = threadIdx.x & (L - 1);
+    if (W == 1 && row >= rows) return;
+    const int nb = k / 8, ng = k / G;
+    const float4 *xr = reinterpret_cast<const float4 *>(x + (size_t)row * k);
+    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 v[NI][2];
+    float m = 0.0f;
+    auto top = [&](float4 lo, float4 hi) {
+        m = fmaxf(m, fmaxf(fmaxf(fabsf(lo.x), fabsf(lo.y)), fmaxf(fabsf(lo.z), fabsf(lo.w))));
+        m = fmaxf(m, fmaxf(fmaxf(fabsf(hi.x), fabsf(hi.y)), fmaxf(fabsf(hi.z), fabsf(hi.w))));
+    };
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        // (every load issued, at a clamped place: a guarded one would be a branch and a wait)
+        const int b = min(lane + i * L, nb - 1);
+        v[i][0] = xr[2 * b];
+        v[i][1] = xr[2 * b + 1];
+    }
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        if (lane + i * L >= nb) v[i][0] = v[i][1] = z4;
+        top(v[i][0], v[i][1]);
+    }
+    for (int b = lane + NI * L; b < nb; b += L) top(xr[2 * b], xr[2 * b + 1]);
+    m = qw_wave_max(m);
+    if (W > 1) {
+        if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
+        __syncthreads();
+        m = fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3]));
+    }
+    int sh = 0;
+    if (m > 0.0f && m <= 3.40282346638528859812e+38f) {
+        sh = 15 - __builtin_amdgcn_frexp_expf(m);
+        sh = sh < -126 ? -126 : sh > 126 ? 126 : sh;
+    }
+    if (lane == 0) ex[row] = 24 - sh;
+    const float up = __builtin_ldexpf(1.0f, sh), up4 = __builtin_ldexpf(1.0f, sh - 4);
+    qw_h8 *hr = reinterpret_cast<qw_h8 *>(ah + (size_t)row * kp);
+    uint16_t *xr16 = xp + (size_t)row * nsb * 64;
+    // (kp / 8 is a multiple of 32, so a group's G / 8 lanes are in or out together)
+    auto block = [&](int b, float4 lo, float4 hi) {
+        const float f[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        _Float16 q[8];
+        float even = 0.0f, odd = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            q[j] = (_Float16)(f[j] * ((j & 1) ? up4 : up));
+            if (j & 1) odd += (float)q[j];
+            else even += (float)q[j];
+        }
+        hr[b] = qw_h8{q[0], q[4], q[1], q[5], q[2], q[6], q[3], q[7]};
+        const float sum = qw_xor_sum<G / 8>(__builtin_fmaf(odd, 16.0f, even));
+        const int g = b / (G / 8);
+        if (b % (G / 8) == 0 && g < ng) {
+            float r = sum * 0x1p-24f;
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+                const uint32_t hi16 = __float_as_uint(r) & 0xFFFF0000u;
+                xr16[(g / QX_SB) * 64 + p * QX_SB + g % QX_SB] = (uint16_t)(hi16 >> 16);
+                r -= __uint_as_float(hi16);
+            }
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+        if (lane + i * L < kp / 8) block(lane + i * L, v[i][0], v[i][1]);
+    for (int b = lane + NI * L; b < kp / 8; b += L) block(b, b < nb ? xr[2 * b] : z4, b < nb ? xr[2 * b + 1] : z4);
+    for (int i = lane; i < nsb * 64; i += L)
+        if ((i & 63) >= 3 * QX_SB || (i >> 6) * QX_SB + (i & 15) >= ng) xr16[i] = 0;
+}
+
+// ---- the product ---------------------------------------------------------------------
+
+struct QxArgs {
+    float *y;
+    const _Float16 *ah;      // [source rows, kp]
+    const uint16_t *xp;      // [source rows, nsb * 64]
+    const int *ex;           // [source rows]
+    const int32_t *perm, *tiles;
+    const uint32_t *w;
+    const uint16_t *s, *b;
+    int k, n, kp, nsb;
+    int K, x_by_pair;        // grouped: the source row of pair p is x_by_pair ? p : p / K
+    int rows;                // dense: rows
+    int nblk, nbw;           // column blocks, and how many of them a workgroup runs back to back
+    int kslice;              // k range of a blockIdx.y slice (whole stages and 16-group blocks; k: no split)
+    float *part;             // dense split-K: slice s writes part[s][rows][n]
+};
+
+// 16 bytes a lane from its own address straight into LDS at lds + 16 lane.
+// Written as asm because the compiler, which cannot tell the ring's stages
+// apart, waits for every such load before any LDS read; the waits on the
+// vector memory counter in k_xgemm are this kernel's own.
+__device__ __forceinline__ void qx_dma(uint32_t lds, const void *src)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+
+template <int N>
+__device__ __forceinline__ void qx_wait()
+{
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// A workgroup: WM x WN waves, each MT x NT tiles of 16 x 16; k in stages of
+// BK through a ring of NST in LDS.
+//
+// LDS layouts (a 16-byte piece is the unit a lane loads):
+//   activations  [BM][BK]: piece p of row r at p ^ (r % 8), so the 8 lanes
+//                that read one piece of 8 rows hit different banks
+//   weights      [BN][BK / 8 words]: pieces of 4 words, swizzled by the
+//                column for BK 128 and 256 alike
+//   scales       [BN][groups] bf16, as in memory; [BN][SGL] at a time where
+//                a row has more than SGL groups
+// The swizzles are in the addresses a lane loads from, since the loads fill
+// LDS in lane order.
+template <int G, int MT, int NT, int WM, int WN, int BK, int NST, int SGL, bool GATHER>
+__global__ __launch_bounds__(64 * WM * WN, 2) void k_xgemm(QxArgs a)
+{
+    constexpr int NW = WM * WN, BM = WM * MT * 16, BN = WN * NT * 16, THREADS = 64 * NW;
+    constexpr int APR = BK / 8, WPR = BK / 32;                   // pieces a row / a column
+    constexpr int ASZ = BM * BK * 2, WSZ = BN * BK / 2, STG = ASZ + WSZ;
+    constexpr int AI = ASZ / 1024 / NW, WT = WSZ / 1024;         // loads a stage: a wave's of A, all of W
+    constexpr int WI = (WT + NW - 1) / NW, WR = WT % NW;         // a wave's of W (waves from WR on one fewer)
+    static_assert(ASZ % (1024 * NW) == 0 && WSZ % 1024 == 0 && BK % 64 == 0 && (SGL * G) % BK == 0 && SGL % 8 == 0,
+                  "whole loads and whole stages");
+    static_assert((AI + WI) * (NST - 2) < 64, "the wait's counter");
+    __shared__ __align__(16) uint8_t ring[NST * STG];
+    __shared__ __align__(16) uint16_t Sc[(BN * SGL + 511) / 512 * 512];
+    __shared__ int rows_s[GATHER ? 2 * BM : 1];
+
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+    const int ln = lane & 15, kg = lane >> 4;
+    const int wm = wave / WN, wn = wave % WN;
+
+    // Workgroup b runs on XCD b % 8: each XCD takes a contiguous run of the
+    // items.  Grouped, an expert's column blocks are adjacent (they share its
+    // activation rows); dense, a column block's row tiles are (they share its
+    // weights).  The grouped grid is an upper bound: the run is cut from the
+    // tiles there are.
+    const int ntl = GATHER ? a.tiles[0] : (a.rows + BM - 1) / BM;
+    const int ngr = (a.nblk + a.nbw - 1) / a.nbw, items = ntl * ngr, per = items >> 3, rem = items & 7;
+    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    if (j >= per + (xcd < rem ? 1 : 0)) return;
+    const int v = xcd * per + min(xcd, rem) + j;
+    const int tile = GATHER ? v / ngr : v % ntl, nb0 = (GATHER ? v % ngr : v / ntl) * a.nbw;
+    const int nb1 = min(nb0 + a.nbw, a.nblk);
+
+    int expert = 0, first, len;
+    if (GATHER) {
+        expert = a.tiles[1 + 3 * tile];
+        first = a.tiles[2 + 3 * tile];
+        len = a.tiles[3 + 3 * tile];
+        // source and destination of each tile row; rows past the tile's read its first again
+        for (int m = t; m < BM; m += THREADS) {
+            const int p = a.perm[first + (m < len ? m : 0)];
+            rows_s[m] = a.x_by_pair ? p : p / a.K;
+            rows_s[BM + m] = p;
+        }
+        __syncthreads();
+    } else {
+        first = tile * BM;
+        len = min(BM, a.rows - first);
+    }
+    auto src_row = [&](int m) { return GATHER ? rows_s[m] : first + min(m, len - 1); };
+
+    const int k = a.k, n = a.n, words = k / 8, groups = k / G;
+    const int kb = (int)blockIdx.y * a.kslice, ke = min(k, kb + a.kslice), T = (ke - kb + BK - 1) / BK;
+    const uint32_t *wb = a.w + (size_t)expert * n * words;
+    const uint16_t *sb = a.s + (size_t)expert * n * groups;
+    const uint16_t *bb = a.b + (size_t)expert * n * groups;
+    // how the scales come (uniform): a flat copy of the block's columns, 8
+    // groups of a column a load, or one by one; the last two also the biases
+    const bool wide = groups % 8 == 0 && (((uintptr_t)sb | (uintptr_t)bb) & 15) == 0;
+    const int sld = min(groups, SGL);                            // groups a column in Sc
+    const bool flat = groups <= SGL && ((uintptr_t)sb & 15) == 0 && (n * (long)groups) % 8 == 0;
+
+    // ---- this lane's loads -----------------------------------------------------------
+    const _Float16 *asrc[AI];
+    const uint32_t *wrow[WI];
+    int wpc[WI];
+#pragma unroll
+    for (int i = 0; i < AI; i++) {
+        const int slot = (wave * AI + i) * 64 + lane, r = slot / APR, p = slot % APR;
+        asrc[i] = a.ah + (size_t)src_row(r) * a.kp + kb + 8 * (p ^ (r & 7));
+    }
+#pragma unroll
+    for (int i = 0; i < WI; i++) {
+        const int slot = ((wave + NW * i) * 64 + lane) % (BN * WPR), c = slot / WPR, p = slot % WPR;
+        wpc[i] = WPR == 2 ? p : WPR == 4 ? p ^ ((c >> 1) & 3) : p ^ (c & 7);
+    }
+    int n0;                                                      // the block's first column
+    const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)&ring[0];
+    const bool fewer = WR != 0 && wave >= WR;                    // this wave has one W load less
+    auto issue = [&](int i) {
+        const uint32_t st = ring0 + (uint32_t)(i % NST) * STG;
+        const int k0 = kb + i * BK;
+#pragma unroll
+        for (int u = 0; u < AI; u++) qx_dma(st + (wave * AI + u) * 1024, asrc[u] + i * BK);
+#pragma unroll
+        for (int u = 0; u < WI; u++) {
+            if (u == WI - 1 && fewer) break;
+            // a piece past the row's end (k not a multiple of BK) meets zeros of A: any piece of the row will do
+            const int pc = k0 / 32 + wpc[u];
+            qx_dma(st + ASZ + (wave + NW * u) * 1024, wrow[u] + 4 * (pc < words / 4 ? pc : 0));
+        }
+    };
+    auto landed = [&](int ahead) {       // all but the latest `ahead` stages' loads of this wave are in LDS
+        if (ahead >= 2 && NST >= 4) {
+            if (fewer) qx_wait<(NST >= 4 ? 2 : 0) * (AI + WI - 1)>();
+            else qx_wait<(NST >= 4 ? 2 : 0) * (AI + WI)>();
+        } else if (ahead == 1 && NST >= 3) {
+            if (fewer) qx_wait<AI + WI - 1>();
+            else qx_wait<AI + WI>();
+        } else {
+            qx_wait<0>();
+        }
+    };
+
+    // the narrow tiles' biases come to LDS too (in place of a stage)
+    static_assert(NST != 2 || STG >= (BN * SGL * 2 + 1023) / 1024 * 1024, "the biases' place");
+    const bool lds_bias = NST == 2 && flat && ((uintptr_t)bb & 15) == 0;
+    const uint32_t sc0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)&Sc[0];
+    // the block's columns of the scales or biases as one run; pieces past the
+    // bank's last column read its last 8 values again
+    auto load_flat = [&](uint32_t to, const uint16_t *from) {
+        const long end = (long)n * groups - 8;
+        for (int i = wave; i * 512 < BN * groups; i += NW)
+            qx_dma(to + i * 1024, from + min((long)n0 * groups + i * 512 + lane * 8, end));
+    };
+    auto load_bias = [&](uint32_t to) { load_flat(to, bb); };
+    auto load_scales = [&](int g0) {
+        if (flat) {
+            load_flat(sc0, sb);
+        } else if (wide) {
+            for (int i = wave; i * 512 < BN * SGL; i += NW) {
+                const int e = i * 512 + lane * 8, c = min(e / SGL, BN - 1), g = g0 + e % SGL;
+                qx_dma(sc0 + i * 1024, sb + (size_t)min(n0 + c, n - 1) * groups + (g < groups ? g : 0));
+            }
+        } else {
+            for (int i = t; i < BN * sld; i += THREADS) {
+                const int c = i / sld, g = g0 + i % sld;
+                Sc[i] = g < groups ? sb[(size_t)min(n0 + c, n - 1) * groups + g] : 0;
+            }
+        }
+    };
+    // a block's scales and first stages on their way
+    auto begin = [&](int nb) {
+        n0 = nb * BN;
+#pragma unroll
+        for (int i = 0; i < WI; i++) {
+            const int slot = ((wave + NW * i) * 64 + lane) % (BN * WPR), c = slot / WPR;
+            wrow[i] = wb + (size_t)min(n0 + c, n - 1) * words;
+        }
+        load_scales(kb / G);
+        for (int i = 0; i < min(NST - 1, T); i++) issue(i);
+    };
+    begin(nb0);
+    // the rows' exponents, all at once and before the stages (after them each was a trip to memory of its own)
+    int ex[MT][4];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) ex[mt][e] = a.ex[src_row((wm * MT + mt) * 16 + 4 * kg + e)];
+
+    // 16-row tiles of up to XS blocks of 16 groups keep their group sums for every block
+    constexpr int XS = MT == 1 ? 5 : 1;
+    const bool held = MT == 1 && a.nsb <= XS && kb == 0;
+    uint4 xa[XS][MT][2] = {};
+    if (lds_bias && held) {
+#pragma unroll
+        for (int u = 0; u < XS; u++)
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                const uint4 *p = reinterpret_cast<const uint4 *>(
+                    a.xp + (size_t)src_row((wm * MT + mt) * 16 + ln) * a.nsb * 64 + min(u, a.nsb - 1) * 64 + 8 * kg);
+                xa[u][mt][0] = p[0];
+                xa[u][mt][1] = p[4];
+            }
+    }
+
+    for (int nb = nb0; nb < nb1; nb++) {
+    qw_f4 acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) acc[mt][nt] = qw_f4{0.f, 0.f, 0.f, 0.f};
+
+    // ---- the biases' product, 16 groups at a time ------------------------------------
+    // from memory, under the first stages' trip
+    if (!lds_bias) {
+        const int g_end = (ke + G - 1) / G;
+        const uint16_t *xr[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) xr[mt] = a.xp + (size_t)src_row((wm * MT + mt) * 16 + ln) * a.nsb * 64 + 8 * kg;
+        for (int sblk = kb / G / QX_SB; sblk * QX_SB < g_end; sblk++) {
+            uint4 bf[NT], af[MT][2];
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const int c = min(n0 + (wn * NT + nt) * 16 + ln, n - 1), g = sblk * QX_SB + 8 * (kg & 1);
+                // (every load issued, at a clamped place; what is past the row's groups is zeroed after)
+                const uint16_t *p = bb + (size_t)c * groups;
+                if (wide) {
+                    bf[nt] = *reinterpret_cast<const uint4 *>(p + (g < groups ? g : 0));
+                    if (g >= groups) bf[nt] = make_uint4(0, 0, 0, 0);
+                } else if (groups % 4 == 0 && ((uintptr_t)bb & 7) == 0) {
+                    const uint2 u = *reinterpret_cast<const uint2 *>(p + min(g, groups - 4));
+                    const uint2 w = *reinterpret_cast<const uint2 *>(p + min(g + 4, groups - 4));
+                    bf[nt] = make_uint4(g < groups ? u.x : 0u, g < groups ? u.y : 0u, g + 4 < groups ? w.x : 0u,
+                                        g + 4 < groups ? w.y : 0u);
+                } else {
+                    uint32_t o[8];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) o[e] = p[min(g + e, groups - 1)];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) o[e] = g + e < groups ? o[e] : 0u;
+                    bf[nt] = make_uint4(o[0] | o[1] << 16, o[2] | o[3] << 16, o[4] | o[5] << 16, o[6] | o[7] << 16);
+                }
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                const uint4 *p = reinterpret_cast<const uint4 *>(xr[mt] + sblk * 64);
+                af[mt][0] = p[0];
+                af[mt][1] = p[4];
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++)
+                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(qw_b8, af[mt][h]),
+                                                                             __builtin_bit_cast(qw_b8, bf[nt]),
+                                                                             acc[mt][nt], 0, 0, 0);
+        }
+    }
+
+    // ---- the stages ----------------------------------------------------------------------
+    // A MFMA step is 32 k of one group: with 64-wide groups lane group kg
+    // holds k 16 kg .. 16 kg + 15 of the 64 (words and pieces 2 kg, 2 kg + 1,
+    // one a step); with 32-wide ones k 8 kg .. of each 32 (word 4 s + kg).
+    auto stage = [&](int i) {
+        const uint8_t *As = ring + (size_t)(i % NST) * STG, *Ws = As + ASZ;
+        const int gl = ((kb + i * BK) / G - (flat ? 0 : kb / G)) % SGL;   // the stage's first group in Sc
+        // (past the row's last group, where A is zero: the last one's again)
+        auto scale = [&](int c, int g) { return qw_bf16(Sc[c * sld + min(g, sld - 1)]); };
+#pragma unroll
+        for (int sub = 0; sub < BK / 64; sub++) {
+            qw_h8 af[MT][2];
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                const int p = sub * 8 + (G == 32 ? 4 * s + kg : 2 * kg + s);
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) {
+                    const int r = (wm * MT + mt) * 16 + ln;
+                    af[mt][s] = *reinterpret_cast<const qw_h8 *>(As + r * (BK * 2) + ((p ^ (r & 7)) * 16));
+                }
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const int c = (wn * NT + nt) * 16 + ln;
+                const int sw = WPR == 2 ? 0 : WPR == 4 ? (c >> 1) & 3 : c & 7;
+                const uint8_t *wr = Ws + c * (BK / 2);
+                uint32_t w[2];
+                if (G == 32) {
+#pragma unroll
+                    for (int s = 0; s < 2; s++)
+                        w[s] = *reinterpret_cast<const uint32_t *>(wr + ((sub * 2 + s) ^ sw) * 16 + kg * 4);
+                } else {
+                    const uint2 u = *reinterpret_cast<const uint2 *>(wr + ((sub * 2 + (kg >> 1)) ^ sw) * 16 + (kg & 1) * 8);
+                    w[0] = u.x;
+                    w[1] = u.y;
+                }
+                qw_h8 bf[2];
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    const uint32_t w8 = w[s] >> 8;
+                    const uint4 d = make_uint4(w[s] & 0x000F000Fu, w[s] & 0x00F000F0u, w8 & 0x000F000Fu, w8 & 0x00F000F0u);
+                    bf[s] = __builtin_bit_cast(qw_h8, d);
+                }
+                const qw_f4 z = {0.f, 0.f, 0.f, 0.f};
+                if (G == 32) {
+#pragma unroll
+                    for (int s = 0; s < 2; s++) {
+                        const float sc = scale(c, gl + sub * 2 + s);
+                        qw_f4 C[MT];
+#pragma unroll
+                        for (int mt = 0; mt < MT; mt++) C[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[mt][s], bf[s], z, 0, 0, 0);
+#pragma unroll
+                        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                            for (int e = 0; e < 4; e++) acc[mt][nt][e] = __builtin_fmaf(sc, C[mt][e], acc[mt][nt][e]);
+                    }
+                } else {
+                    const float sc = scale(c, gl + sub * 64 / G);
+                    qw_f4 C[MT];
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) C[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[mt][0], bf[0], z, 0, 0, 0);
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) C[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[mt][1], bf[1], C[mt], 0, 0, 0);
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[mt][nt][e] = __builtin_fmaf(sc, C[mt][e], acc[mt][nt][e]);
+                }
+            }
+        }
+    };
+    for (int i = 0; i < T; i++) {
+        if (!flat && i > 0 && (i * BK) % (SGL * G) == 0) {       // every wave is done with the last SGL groups' scales
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            load_scales((kb + i * BK) / G);
+            qx_wait<0>();
+        }
+        landed(min(NST - 2, T - 1 - i));
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        // stage i is in LDS, and every wave is done with stage i - 1, whose place stage i + NST - 1 takes
+        if (i + NST - 1 < T) issue(i + NST - 1);
+        else if (i + NST - 1 == T && lds_bias) load_bias(ring0 + (uint32_t)(T % NST) * STG);
+        stage(i);
+    }
+    // narrow tiles: the biases came to LDS as stage T, in one flat copy (read
+    // by every wave from memory they were as many requests as the weights)
+    if (lds_bias) {
+        qx_wait<0>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const uint16_t *Bs = reinterpret_cast<const uint16_t *>(ring + (size_t)(T % NST) * STG);
+        const int g_end = min(groups, (ke + G - 1) / G);
+#pragma unroll 1
+        for (int u = 0; u * QX_SB < g_end - kb / G; u++) {
+            const int sblk = kb / G / QX_SB + u, g = sblk * QX_SB + 8 * (kg & 1);
+            uint4 xf[MT][2];
+            if (held) {
+#pragma unroll
+                for (int q = 0; q < XS; q++)
+                    if (q == u) {
+#pragma unroll
+                        for (int mt = 0; mt < MT; mt++) { xf[mt][0] = xa[q][mt][0]; xf[mt][1] = xa[q][mt][1]; }
+                    }
+            } else {
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) {
+                    const uint4 *p = reinterpret_cast<const uint4 *>(
+                        a.xp + (size_t)src_row((wm * MT + mt) * 16 + ln) * a.nsb * 64 + sblk * 64 + 8 * kg);
+                    xf[mt][0] = p[0];
+                    xf[mt][1] = p[4];
+                }
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const uint16_t *p = Bs + ((wn * NT + nt) * 16 + ln) * groups;
+                uint32_t o[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) o[e] = p[min(g + e, groups - 1)];
+#pragma unroll
+                for (int e = 0; e < 8; e++) o[e] = g + e < g_end ? o[e] : 0u;
+                const uint4 bf = make_uint4(o[0] | o[1] << 16, o[2] | o[3] << 16, o[4] | o[5] << 16, o[6] | o[7] << 16);
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++)
+                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(qw_b8, xf[mt][h]),
+                                                                             __builtin_bit_cast(qw_b8, bf),
+                                                                             acc[mt][nt], 0, 0, 0);
+            }
+        }
+    }
+
+    // every wave is done with the ring and the scales: the next block's are
+    // on their way while this one's results leave
+    const int c0 = n0;
+    if (nb + 1 < nb1) {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        begin(nb + 1);
+    }
+    float *yo = !GATHER && a.part ? a.part + (size_t)blockIdx.y * a.rows * n : a.y;
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int m = (wm * MT + mt) * 16 + 4 * kg + e;
+            if (m >= len) continue;
+            float *yr = yo + (size_t)(GATHER ? rows_s[BM + m] : first + m) * n;
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const int c = c0 + (wn * NT + nt) * 16 + ln;
+                if (c < n) yr[c] = __builtin_ldexpf(acc[mt][nt][e], ex[mt][e]);
+            }
+        }
+    }
+}
+
+// ---- small dense products ------------------------------------------------------------
+//
+// Where the whole product is a few microseconds, the stage's launch costs more
+// than it saves (8 rows, 3072 x 512: 23.2 us a call against 25.7): one launch
+// that converts the activations as it stages them, four waves a workgroup, a
+// tile of BM rows against 64 columns.  A nibble enters as the f16 1024 + q
+// (exact); the group's map is applied to the fp32 partial:
+//   sum_i (s q_i + b) x_i = s C_g + (b - 1024 s) X_g,
+//   C_g = sum_i (1024 + q_i) x_i,   X_g = sum_i x_i.
 #define QW_GMM_BN 64
 #define QW_GMM_BK 128
 #define QW_GMM_THREADS 256
@@ -35,18 +583,16 @@ typedef float qw_f4 __attribute__((ext_vector_type(4)));
 struct QwGmmArgs {
     float *y;
     const float *x;
-    const int32_t *perm;
-    const int32_t *tiles;
     qwk_q4 m;
-    int k, n, K, x_by_pair, rows, nblk;
+    int k, n, rows, nblk;
     int kslice;      // k range of a blockIdx.y slice (k: no split)
-    float *part;     // dense split-K: slice s writes part[s][rows][n]
+    float *part;     // split-K: slice s writes part[s][rows][n]
 };
 
 union qw_h8u { qw_h8 h; uint32_t u[4]; uint4 v; };
 
-template <int G, int BM, bool DENSE>
-__global__ __launch_bounds__(QW_GMM_THREADS) void k_gather_gemm(QwGmmArgs a)
+template <int G, int BM>
+__global__ __launch_bounds__(QW_GMM_THREADS) void k_sgemm(QwGmmArgs a)
 {
     constexpr int MT = BM / 16;
     constexpr int GPS = (QW_GMM_BK / G) > 0 ? QW_GMM_BK / G : 1;   // groups per stage
@@ -61,24 +607,13 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_gather_gemm(QwGmmArgs a)
     const unsigned v = (total % 8u == 0u) ? (b % 8u) * (total / 8u) + b / 8u : b;
     const int tile = (int)(v / (unsigned)a.nblk), nb = (int)(v % (unsigned)a.nblk);
 
-    int expert, first, len;
-    if (DENSE) {
-        first = tile * BM;
-        if (first >= a.rows) return;
-        expert = 0;
-        len = min(BM, a.rows - first);
-    } else {
-        if (tile >= a.tiles[0]) return;
-        expert = a.tiles[1 + 3 * tile];
-        first = a.tiles[2 + 3 * tile];
-        len = a.tiles[3 + 3 * tile];
-    }
+    const int first = tile * BM, len = min(BM, a.rows - first);
+    if (len <= 0) return;
     const int k = a.k, n = a.n, words = k / 8, groups = k / G;
     const int n0 = nb * QW_GMM_BN;
     const int kb = (int)blockIdx.y * a.kslice, ke = min(k, kb + a.kslice);
-    const uint32_t *wb = a.m.w + (size_t)expert * n * words;
-    const uint16_t *sb = a.m.s + (size_t)expert * n * groups;
-    const uint16_t *bb = a.m.b + (size_t)expert * n * groups;
+    const uint32_t *wb = a.m.w;
+    const uint16_t *sb = a.m.s, *bb = a.m.b;
 
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int ln = lane & 15, lg = lane >> 4;
@@ -99,9 +634,7 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_gather_gemm(QwGmmArgs a)
             qw_h8u h;
             float bsum = 0.0f;
             if (m < len && bk * 8 < klen) {
-                const int p = DENSE ? first + m : a.perm[first + m];
-                const int xr = DENSE ? p : (a.x_by_pair ? p : p / a.K);
-                const float4 *xv = reinterpret_cast<const float4 *>(a.x + (size_t)xr * k + k0 + bk * 8);
+                const float4 *xv = reinterpret_cast<const float4 *>(a.x + (size_t)(first + m) * k + k0 + bk * 8);
                 const float4 lo = xv[0], hi = xv[1];
                 const float f[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
                 _Float16 q[8];
@@ -172,7 +705,7 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_gather_gemm(QwGmmArgs a)
         __syncthreads();
     }
 
-    float *yo = DENSE && a.part ? a.part + (size_t)blockIdx.y * a.rows * n : a.y;
+    float *yo = a.part ? a.part + (size_t)blockIdx.y * a.rows * n : a.y;
     if (col < n) {
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
@@ -180,8 +713,7 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_gather_gemm(QwGmmArgs a)
             for (int i = 0; i < 4; i++) {
                 const int m = mt * 16 + 4 * lg + i;
                 if (m < len) {
-                    const int row = DENSE ? first + m : a.perm[first + m];
-                    yo[(size_t)row * n + col] = acc[mt][i];
+                    yo[(size_t)(first + m) * n + col] = acc[mt][i];
                 }
             }
         }
@@ -198,30 +730,14 @@ __global__ void k_qmm_reduce(float *__restrict__ y, const float *__restrict__ pa
     }
 }
 
-template <int G, bool DENSE>
-static int gmm_bm(int bm, dim3 grid, hipStream_t s, const QwGmmArgs &a)
-{
-    const dim3 blk(QW_GMM_THREADS);
-    switch (bm) {
-    case 16: hipLaunchKernelGGL((k_gather_gemm<G, 16, DENSE>), grid, blk, 0, s, a); break;
-    case 32: hipLaunchKernelGGL((k_gather_gemm<G, 32, DENSE>), grid, blk, 0, s, a); break;
-    case 64: hipLaunchKernelGGL((k_gather_gemm<G, 64, DENSE>), grid, blk, 0, s, a); break;
-    default: return (int)hipErrorInvalidValue;
-    }
-    return (int)hipGetLastError();
-}
+// ---- plans -------------------------------------------------------------------------------
 
-template <bool DENSE>
-static int gmm_launch(hipStream_t s, const QwGmmArgs &a, int group, int bm, int ntiles, int splits = 1)
+static size_t qx_al(size_t b) { return (b + 255) & ~(size_t)255; }
+static int qx_kp(int k) { return (k + QX_KPAD - 1) / QX_KPAD * QX_KPAD; }
+static int qx_nsb(int k, int group) { return (k / group + QX_SB - 1) / QX_SB; }
+static size_t qx_stage_bytes(int rows, int k, int group)
 {
-    if (ntiles <= 0) return 0;
-    const dim3 grid((unsigned)(a.nblk * ntiles), (unsigned)splits);
-    switch (group) {
-    case 32: return gmm_bm<32, DENSE>(bm, grid, s, a);
-    case 64: return gmm_bm<64, DENSE>(bm, grid, s, a);
-    case 128: return gmm_bm<128, DENSE>(bm, grid, s, a);
-    default: return (int)hipErrorInvalidValue;
-    }
+    return qx_al((size_t)rows * qx_kp(k) * 2) + qx_al((size_t)rows * qx_nsb(k, group) * 128) + qx_al((size_t)rows * 4);
 }
 
 static bool gmm_shape_ok(const float *x, qwk_q4 m, int k, int n, int group)
@@ -230,22 +746,109 @@ static bool gmm_shape_ok(const float *x, qwk_q4 m, int k, int n, int group)
            k % group == 0 && ((uintptr_t)x & 15u) == 0 && ((uintptr_t)m.w & 15u) == 0;
 }
 
-extern "C" int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const int32_t *perm,
-                               const int32_t *tiles, qwk_q4 m, int k, int n, int K, int x_by_pair,
-                               int group, int bm, int max_tiles)
+// Stages `rows` rows at `work` and points the arguments at them.
+static void qx_stage(hipStream_t s, QxArgs &a, const float *x, int rows, int group, char *work)
 {
-    if (!gmm_shape_ok(x, m, k, n, group) || K < 1) return (int)hipErrorInvalidValue;
-    QwGmmArgs a = {y, x, perm, tiles, m, k, n, K, x_by_pair, 0, (n + QW_GMM_BN - 1) / QW_GMM_BN, k, nullptr};
-    return gmm_launch<false>(s, a, group, bm, max_tiles);
+    a.kp = qx_kp(a.k);
+    a.nsb = qx_nsb(a.k, group);
+    _Float16 *ah = reinterpret_cast<_Float16 *>(work);
+    uint16_t *xp = reinterpret_cast<uint16_t *>(work + qx_al((size_t)rows * a.kp * 2));
+    int *ex = reinterpret_cast<int *>(reinterpret_cast<char *>(xp) + qx_al((size_t)rows * a.nsb * 128));
+    a.ah = ah;
+    a.xp = xp;
+    a.ex = ex;
+    const bool wide = a.k >= QX_WIDE_K;
+    const dim3 grid(wide ? rows : (rows + 3) / 4), blk(256);
+#define QX_STAGE(GG)                                                                                                       \
+    if (!wide) hipLaunchKernelGGL((k_xstage<GG, 1, 2>), grid, blk, 0, s, ah, xp, ex, x, rows, a.k, a.kp, a.nsb);            \
+    else if (a.k <= 4096) hipLaunchKernelGGL((k_xstage<GG, 4, 2>), grid, blk, 0, s, ah, xp, ex, x, rows, a.k, a.kp, a.nsb); \
+    else hipLaunchKernelGGL((k_xstage<GG, 4, 6>), grid, blk, 0, s, ah, xp, ex, x, rows, a.k, a.kp, a.nsb)
+    if (group == 32) { QX_STAGE(32); }
+    else if (group == 64) { QX_STAGE(64); }
+    else { QX_STAGE(128); }
+#undef QX_STAGE
 }
 
-// Split-K for the dense product when the tiles alone would leave the chip
+// Column blocks a workgroup runs back to back: where k is short a block is
+// over in a few stages, and a workgroup's start (its tile's rows, the first
+// loads) would be most of it; kept to what still fills QX_SLOTS places.
+static int qx_nbw(int k, int nblk, long tiles)
+{
+    int w = k >= 2048 ? 1 : 2048 / (k < 256 ? 256 : k);
+    while (w > 1 && tiles * ((nblk + w - 1) / w) < QX_SLOTS) w--;
+    return w < nblk ? w : nblk;
+}
+
+// Few rows a tile: four waves side by side over 128 columns.
+template <int G, bool GATHER>
+static void qx_narrow(hipStream_t s, QxArgs &a, int bm, int ntiles, int splits)
+{
+    a.nblk = (a.n + 127) / 128;
+    a.nbw = qx_nbw(a.k, a.nblk, (long)ntiles * splits);
+    const long ngr = (a.nblk + a.nbw - 1) / a.nbw;
+    const dim3 grid((unsigned)((ngr * ntiles + 7) / 8 * 8), (unsigned)splits), blk(256);
+    if (bm == 16) hipLaunchKernelGGL((k_xgemm<G, 1, 2, 1, 4, 256, 2, 96, GATHER>), grid, blk, 0, s, a);
+    else if (bm == 32) hipLaunchKernelGGL((k_xgemm<G, 2, 2, 1, 4, 256, 2, 48, GATHER>), grid, blk, 0, s, a);
+    else hipLaunchKernelGGL((k_xgemm<G, 4, 2, 1, 4, 128, 2, 96, GATHER>), grid, blk, 0, s, a);
+}
+
+template <int G>
+static void qx_wide(hipStream_t s, QxArgs &a, int nt, int splits)
+{
+    a.nblk = (a.n + 32 * nt - 1) / (32 * nt);
+    const long ntiles = (a.rows + 127) / 128;
+    a.nbw = qx_nbw(a.k, a.nblk, ntiles * splits);
+    const long ngr = (a.nblk + a.nbw - 1) / a.nbw;
+    const dim3 grid((unsigned)((ngr * ntiles + 7) / 8 * 8), (unsigned)splits), blk(256);
+    switch (nt) {
+    case 2: hipLaunchKernelGGL((k_xgemm<G, 4, 2, 2, 2, 64, 3, 48, false>), grid, blk, 0, s, a); break;
+    case 3: hipLaunchKernelGGL((k_xgemm<G, 4, 3, 2, 2, 64, 3, 48, false>), grid, blk, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((k_xgemm<G, 4, 4, 2, 2, 64, 3, 48, false>), grid, blk, 0, s, a); break;
+    default: hipLaunchKernelGGL((k_xgemm<G, 4, 5, 2, 2, 64, 3, 48, false>), grid, blk, 0, s, a); break;
+    }
+}
+
+extern "C" size_t qwk_gather_gemm_work_bytes(int k, int pairs, int K, int x_by_pair, int group)
+{
+    if (k < 1 || pairs < 1 || K < 1 || group < 1) return 0;
+    return qx_stage_bytes(x_by_pair ? pairs : (pairs + K - 1) / K, k, group);
+}
+
+extern "C" int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const int32_t *perm,
+                               const int32_t *tiles, qwk_q4 m, int k, int n, int pairs, int K, int x_by_pair,
+                               int group, int bm, int max_tiles, void *work, size_t work_bytes)
+{
+    if (!gmm_shape_ok(x, m, k, n, group) || K < 1 || (bm != 16 && bm != 32 && bm != 64)) return (int)hipErrorInvalidValue;
+    if (max_tiles <= 0 || pairs <= 0) return 0;
+    if (!work || work_bytes < qwk_gather_gemm_work_bytes(k, pairs, K, x_by_pair, group)) return (int)hipErrorInvalidValue;
+    QxArgs a = {};
+    a.y = y; a.perm = perm; a.tiles = tiles; a.w = m.w; a.s = m.s; a.b = m.b;
+    a.k = k; a.n = n; a.K = K; a.x_by_pair = x_by_pair; a.kslice = k;
+    qx_stage(s, a, x, x_by_pair ? pairs : (pairs + K - 1) / K, group, static_cast<char *>(work));
+    if (group == 32) qx_narrow<32, true>(s, a, bm, max_tiles, 1);
+    else if (group == 64) qx_narrow<64, true>(s, a, bm, max_tiles, 1);
+    else qx_narrow<128, true>(s, a, bm, max_tiles, 1);
+    return (int)hipGetLastError();
+}
+
+// Small products' plan: split-K when the tiles alone would leave the chip
 // under two workgroups a CU: enough k slices for ~QW_QMM_SPLIT_WG workgroups,
 // each a whole number of QW_GMM_BK steps (so of quantisation groups) and no
-// shorter than QW_QMM_SPLIT_MIN_K.  The plan is a function of the shape only.
+// shorter than QW_QMM_SPLIT_MIN_K.
 #define QW_QMM_SPLIT_BELOW 512
 #define QW_QMM_SPLIT_WG 1024
 #define QW_QMM_SPLIT_MIN_K 512
+
+// Which products are small (both sides timed, us a call, this against the
+// staged form): 8 x 3072 x 3072 24.4 / 25.8, 20 x 1024 x 1024 23.0 / 24.9,
+// 33 x 3392 x 832 28.0 / 30.3, but 16 x 3072 x 10240 30.2 / 27.1 and 130 x
+// 2560 x 2560 40.7 / 34.5; a short k gives the stages little to overlap: 300
+// x 320 x 12288 28.8 / 30.2, 1021 x 320 x 12288 44.5 / 33.
+static bool qmm_small(int k, int n, int rows)
+{
+    const double macs = (double)rows * n * k;
+    return macs < 134217728.0 || (k <= 512 && macs < 2147483648.0);
+}
 
 static int qmm_bm(int rows) { return rows >= 64 ? 64 : (rows >= 32 ? 32 : 16); }
 
@@ -263,31 +866,116 @@ static int qmm_splits(int k, int n, int rows, int *kslice)
     return (k + ks - 1) / ks;
 }
 
-extern "C" size_t qwk_qmm_work_bytes(int k, int n, int rows)
+template <int G>
+static void qmm_small_launch(hipStream_t s, const QwGmmArgs &a, int splits)
 {
-    int ks;
-    const int sp = k > 0 && n > 0 && rows > 0 ? qmm_splits(k, n, rows, &ks) : 1;
-    return sp > 1 ? (size_t)sp * rows * n * sizeof(float) : 0;
+    const int bm = qmm_bm(a.rows);
+    const dim3 grid((unsigned)(a.nblk * ((a.rows + bm - 1) / bm)), (unsigned)splits), blk(QW_GMM_THREADS);
+    if (bm == 16) hipLaunchKernelGGL((k_sgemm<G, 16>), grid, blk, 0, s, a);
+    else if (bm == 32) hipLaunchKernelGGL((k_sgemm<G, 32>), grid, blk, 0, s, a);
+    else hipLaunchKernelGGL((k_sgemm<G, 64>), grid, blk, 0, s, a);
+}
+
+static void qmm_reduce(hipStream_t s, float *y, const float *part, long total, int splits)
+{
+    const long want = (total + 255) / 256;
+    hipLaunchKernelGGL(k_qmm_reduce, dim3((unsigned)(want < 4096 ? want : 4096)), dim3(256), 0, s, y, part, total, splits);
+}
+
+// The staged plan, a function of the shape only.  Up to 64 rows: one tile of
+// 16, 32 or 64 rows against 128 columns a workgroup; more: 128 rows against
+// 32 nt columns.  Where that leaves the chip's QX_SLOTS workgroup places
+// empty, k is cut into slices (of whole stages and whole 16-group blocks),
+// whose partial sums are added in slice order.  nt is the one that ends
+// first: rounds of workgroups, each as long as its stages' MFMAs plus what a
+// stage costs at any width, and the partials' trip through memory.
+struct QxPlan { int bm, nt, splits, kslice; };
+
+static QxPlan qx_plan(int k, int n, int rows, int group)
+{
+    QxPlan best = {};
+    double cost = 1e300;
+    const int bm = rows > 64 ? 128 : rows > 32 ? 64 : rows > 16 ? 32 : 16;
+    const long rt = (rows + bm - 1) / bm;
+    const int unit = QX_SB * group;                              // a slice is a multiple of this (and of any BK)
+    for (int nt = 2; nt <= (bm == 128 ? 5 : 2); nt++) {
+        const int bn = bm == 128 ? 32 * nt : 128;
+        const long tiles = rt * ((n + bn - 1) / bn);
+        const int units = (k + unit - 1) / unit;
+        for (int sp = 1; sp <= units && (sp == 1 || tiles * sp <= QX_SLOTS); sp++) {
+            const int ks = (units + sp - 1) / sp * unit, real = (k + ks - 1) / ks;
+            if (real != sp) continue;
+            const long rounds = (tiles * sp + QX_SLOTS - 1) / QX_SLOTS;
+            // in MFMA-stage units (64 k of a wave tile column): ~0.06 us
+            const double c = rounds * (((sp == 1 ? k : ks) / 64 + 8) * (nt + 1.0)) +
+                             (sp > 1 ? 30.0 + (double)rows * n * (sp + 1) * 4 / 4e6 / 0.06 : 0.0);
+            if (c < cost) {
+                cost = c;
+                best = QxPlan{bm, nt, sp, sp == 1 ? k : ks};
+            }
+        }
+    }
+    return best;
+}
+
+extern "C" size_t qwk_qmm_work_bytes(int k, int n, int rows, int group)
+{
+    if (k < 1 || n < 1 || rows < 1 || group < 1) return 0;
+    if (qmm_small(k, n, rows)) {
+        int ks;
+        const int sp = qmm_splits(k, n, rows, &ks);
+        return sp > 1 ? (size_t)sp * rows * n * sizeof(float) : 0;
+    }
+    const int r = rows < QX_CHUNK_ROWS ? rows : QX_CHUNK_ROWS;
+    const QxPlan p = qx_plan(k, n, r, group);
+    // (a last, shorter chunk may be split where whole ones are not)
+    const int tail = rows % QX_CHUNK_ROWS;
+    const QxPlan pt = tail && tail != r ? qx_plan(k, n, tail, group) : p;
+    const size_t pb = p.splits > 1 ? (size_t)p.splits * r * n * 4 : 0;
+    const size_t tb = tail && tail != r && pt.splits > 1 ? (size_t)pt.splits * tail * n * 4 : 0;
+    return qx_stage_bytes(r, k, group) + (pb > tb ? pb : tb);
 }
 
 extern "C" int qwk_qmm(hipStream_t s, float *y, const float *x, qwk_q4 m, int k, int n, int rows, int group,
                        void *work, size_t work_bytes)
 {
     if (!gmm_shape_ok(x, m, k, n, group) || rows < 1) return (int)hipErrorInvalidValue;
-    const int bm = qmm_bm(rows);
-    int ks;
-    int sp = qmm_splits(k, n, rows, &ks);
-    if (sp > 1 && (!work || work_bytes < qwk_qmm_work_bytes(k, n, rows) || ((uintptr_t)work & 15u))) {
-        sp = 1;
-        ks = k;
+    const size_t need = qwk_qmm_work_bytes(k, n, rows, group);
+    if (need > 0 && (!work || ((uintptr_t)work & 15u) || work_bytes < need)) return (int)hipErrorInvalidValue;
+    if (qmm_small(k, n, rows)) {
+        int ks;
+        const int sp = qmm_splits(k, n, rows, &ks);
+        const QwGmmArgs a = {y, x, m, k, n, rows, (n + QW_GMM_BN - 1) / QW_GMM_BN, ks,
+                             sp > 1 ? static_cast<float *>(work) : nullptr};
+        if (group == 32) qmm_small_launch<32>(s, a, sp);
+        else if (group == 64) qmm_small_launch<64>(s, a, sp);
+        else qmm_small_launch<128>(s, a, sp);
+        if (sp > 1) qmm_reduce(s, y, a.part, (long)rows * n, sp);
+        return (int)hipGetLastError();
     }
-    QwGmmArgs a = {y, x, nullptr, nullptr, m, k, n, 1, 1, rows, (n + QW_GMM_BN - 1) / QW_GMM_BN, ks,
-                   sp > 1 ? static_cast<float *>(work) : nullptr};
-    int rc = gmm_launch<true>(s, a, group, bm, (rows + bm - 1) / bm, sp);
-    if (rc || sp == 1) return rc;
-    const long total = (long)rows * n;
-    const long want = (total + 255) / 256;
-    hipLaunchKernelGGL(k_qmm_reduce, dim3((unsigned)(want < 4096 ? want : 4096)), dim3(256), 0, s, y,
-                       static_cast<const float *>(work), total, sp);
-    return (int)hipGetLastError();
+    for (int r0 = 0; r0 < rows; r0 += QX_CHUNK_ROWS) {
+        const int r = rows - r0 < QX_CHUNK_ROWS ? rows - r0 : QX_CHUNK_ROWS;
+        const QxPlan p = qx_plan(k, n, r, group);
+        QxArgs a = {};
+        a.y = y + (size_t)r0 * n;
+        a.w = m.w; a.s = m.s; a.b = m.b;
+        a.k = k; a.n = n; a.K = 1; a.x_by_pair = 1; a.rows = r; a.kslice = p.kslice;
+        char *part = static_cast<char *>(work) + qx_stage_bytes(r, k, group);
+        a.part = p.splits > 1 ? reinterpret_cast<float *>(part) : nullptr;
+        qx_stage(s, a, x + (size_t)r0 * k, r, group, static_cast<char *>(work));
+        if (p.bm == 128) {
+            if (group == 32) qx_wide<32>(s, a, p.nt, p.splits);
+            else if (group == 64) qx_wide<64>(s, a, p.nt, p.splits);
+            else qx_wide<128>(s, a, p.nt, p.splits);
+        } else {
+            const int nt = (r + p.bm - 1) / p.bm;
+            if (group == 32) qx_narrow<32, false>(s, a, p.bm, nt, p.splits);
+            else if (group == 64) qx_narrow<64, false>(s, a, p.bm, nt, p.splits);
+            else qx_narrow<128, false>(s, a, p.bm, nt, p.splits);
+        }
+        if (p.splits > 1) qmm_reduce(s, a.y, a.part, (long)r * n, p.splits);
+        const int rc = (int)hipGetLastError();
+        if (rc) return rc;
+    }
+    return 0;
 }

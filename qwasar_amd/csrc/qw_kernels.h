@@ -65,17 +65,19 @@ int qwk_q4mv_multi(hipStream_t s, const float *x, int k, int group, int count,
 
 /* The grouped (prefill) product: per tile of pairs routed to one expert,
  * y[perm[j], :] = W_e . in(perm[j]), in(p) = x row (x_by_pair ? p : p/K).
- * Tiles were cut at `bm` rows by qwk_moe_group; `max_tiles` bounds the grid. */
+ * Tiles were cut at `bm` rows by qwk_moe_group; `max_tiles` bounds the grid.
+ * work: qwk_gather_gemm_work_bytes(...) bytes for the staged activations. */
 int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const int32_t *perm,
-                    const int32_t *tiles, qwk_q4 m, int k, int n, int K, int x_by_pair,
-                    int group, int bm, int max_tiles);
+                    const int32_t *tiles, qwk_q4 m, int k, int n, int pairs, int K, int x_by_pair,
+                    int group, int bm, int max_tiles, void *work, size_t work_bytes);
+size_t qwk_gather_gemm_work_bytes(int k, int pairs, int K, int x_by_pair, int group);
 
 /* Dense prefill product y[rows, n] = x[rows, k] . W^T (the shared expert). */
-/* work: qwk_qmm_work_bytes(k, n, rows) bytes for the split-K partials (none
- * needed when it returns 0; with less, the product runs unsplit). */
+/* work: qwk_qmm_work_bytes(k, n, rows, group) bytes for the staged
+ * activations and the split-K partials. */
 int qwk_qmm(hipStream_t s, float *y, const float *x, qwk_q4 m, int k, int n, int rows, int group,
             void *work, size_t work_bytes);
-size_t qwk_qmm_work_bytes(int k, int n, int rows);
+size_t qwk_qmm_work_bytes(int k, int n, int rows, int group);
 
 /* A second weight bank for grouped tiles of expert `expert` (qwk_moe_group's
  * extra rows): its pairs p >= `pairs` read A row p - pairs when not

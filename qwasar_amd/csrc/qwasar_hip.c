@@ -534,8 +534,9 @@ void qw_op_qmm_q4(qw_cmd c, qw_ref y, qw_ref x, qw_ref w, qw_ref scales, qw_ref 
                   int32_t k, int32_t n, int32_t rows, int32_t group) {
     QW_OP(c);
     touch(c, x, 0); touch(c, w, 0); touch(c, scales, 0); touch(c, biases, 0); touch(c, y, 1);
-    const size_t wb = qwk_qmm_work_bytes(k, n, rows);
+    const size_t wb = qwk_qmm_work_bytes(k, n, rows, group);
     void *work = wb ? scratch(wb) : NULL;
+    if (wb && !work) { cmd_fail(c, hipErrorOutOfMemory, "qmm_q4: scratch of %zu bytes", wb); return; }
     launched(c, "qmm_q4", qwk_qmm(G.stream, dp(y), dp(x), q4(w, scales, biases), k, n, rows, group, work,
                                   work ? wb : 0));
 }
@@ -860,9 +861,12 @@ void qw_op_qmm_q4_gather(qw_cmd c, qw_ref y, qw_ref x, qw_ref perm, qw_ref tiles
     touch(c, x, 0); touch(c, perm, 0); touch(c, tiles, 0);
     touch(c, w, 0); touch(c, scales, 0); touch(c, biases, 0); touch(c, y, 1);
     const int32_t bm = qw_moe_tile_rows(pairs, E);
+    const size_t wb = qwk_gather_gemm_work_bytes(k, pairs, K, x_by_pair ? 1 : 0, group);
+    void *work = wb ? scratch(wb) : NULL;
+    if (wb && !work) { cmd_fail(c, hipErrorOutOfMemory, "qmm_q4_gather: scratch of %zu bytes", wb); return; }
     launched(c, "qmm_q4_gather", qwk_gather_gemm(G.stream, dp(y), dp(x), dp(perm), dp(tiles),
-                                                 q4(w, scales, biases), k, n, K, x_by_pair ? 1 : 0,
-                                                 group, bm, tiles_for(pairs, E, bm)));
+                                                 q4(w, scales, biases), k, n, pairs, K, x_by_pair ? 1 : 0,
+                                                 group, bm, tiles_for(pairs, E, bm), work, wb));
 }
 
 /* ---- the whole MoE layer ------------------------------------------------------ */
