@@ -205,7 +205,11 @@ void qw_op_gdn_gates(qw_cmd c, qw_ref g, qw_ref beta, qw_ref a, qw_ref b,
 /* The delta rule per value head over `rows` timesteps: S *= g; kv = S k;
  * S += k (v - kv) beta; y = S q.  state F32 [hv, dv, dk]; q, k [rows, hk, dk]
  * already l2-normed; v, y [rows, hv, dv]; value head h reads key head
- * h / (hv / hk).  dk = dv = 128 only (refused otherwise, as the reference's). */
+ * h / (hv / hk).  dk = dv = 128 only (refused otherwise, as the reference's).
+ * A call of under 256 steps, or with snapshots, takes the steps one by one
+ * (any split of a sequence into such calls gives the same bits); from 256 on
+ * without snapshots they are taken 32 at a time, the same sums in another
+ * order. */
 void qw_op_gated_delta(qw_cmd c, qw_ref y, qw_ref q, qw_ref k, qw_ref v,
                        qw_ref g, qw_ref beta, qw_ref state,
                        int32_t hk, int32_t hv, int32_t dk, int32_t dv, int32_t rows,

@@ -9,6 +9,8 @@
 //                         and, with PREP, q and k l2-normed and the gates
 //                         computed inside the kernel; with CONV (one decode
 //                         step) the conv too, for the channels it reads
+//   k_gdn_chunk_pre, k_gdn_chunk   the same recurrence in chunks of 32 steps,
+//                         for long calls
 //
 // The recurrence is serial in time but independent across the rows of each
 // head's [dv, dk] state.  A wave owns four value rows: each 16-lane row of
@@ -377,6 +379,435 @@ __global__ void __launch_bounds__(QG_THREADS) k_gated_delta(float *__restrict__ 
     sp[1] = su;
 }
 
+// ---- the recurrence in chunks ---------------------------------------------------
+//
+// A long call (QG_LONG_MIN_ROWS steps on, no snapshots) takes QG_C steps at a
+// time.  With P[t][i] the product of g over (i, t], G[t] the product of g up
+// to t in the chunk, S0 the state before it and u_t = beta_t (v_t - g_t S_{t-1} k_t):
+//   (I + L) U = beta (V - G K S0'),   L[t][i] = beta_t P[t][i] (k_t . k_i), i < t
+//   Y = G Q S0' + (P o Q K') U,       S = G[C-1] S0 + sum_i P[C-1][i] u_i k_i'
+// so the serial part is a few 16-wide products a chunk in place of QG_C
+// dependent steps.  k_gdn_chunk_pre does everything that does not need the
+// state, a workgroup a (key head, chunk): the norms, K K' and Q K', and for
+// each of the key head's value heads the gates, P by running products (never
+// a quotient or a difference of logarithms, which a strong decay would ruin)
+// and T = (I + L)^-1 by forward substitution.  k_gdn_chunk walks the chunks,
+// a workgroup 16 value rows of a head, every product on the fp32 matrix cores
+// (v_mfma_f32_16x16x4_f32: fp32 inputs and sums, as the serial form).
+// 2048 steps of 16 key and 48 value heads: 10 + 590 us serial (70 vector
+// operations a step on the CUs that hold two workgroups), 34 + 227 here; the
+// call with conv and output gate 682 -> 323.  Error against 64 bits over that
+// call: 1.5 to 1.6e-7 serial, 1.75e-7 here (y; the state 1.2e-7 either way).
+// What bounds it now: k_gdn_chunk's chain a chunk (56 MFMAs of 35 cycles a
+// wave and three hand-offs through LDS) on the CUs that hold two of the 384
+// workgroups, and its operands' bytes (K and Q read by 8 workgroups a head: a
+// build without the loads takes 165 us).
+// A step with a NaN or infinite input spoils the outputs of its whole chunk
+// (the zeros of T and Q K' above the diagonal multiply it), not only those
+// after it as in the serial form; the state is spoilt from there on in both.
+#define QG_C 32
+#define QG_LONG_MIN_ROWS 256     // below, the serial kernel (and its bits) stay
+#define QG_LONG_ROWS 4096        // steps a pair of launches takes: bounds the scratch
+#define QG_CS (QG_DK + 4)        // floats an LDS row of 128 takes: 16-byte reads of 8 rows hit different banks
+#define QG_TS (QG_C + 4)
+
+typedef float qg_f4 __attribute__((ext_vector_type(4)));
+
+// Scratch of one launch pair over `n` chunks.
+struct qg_long {
+    float *qn, *kn;          // [hk][n][2][8][64][4]: q and k, normed with PREP, in operand order
+    float *T, *QK;           // [hv][n][2][2][64][4]: QG_C x QG_C, in operand order
+    float4 *sc;              // [hv][n][QG_C]: beta, beta G, G, P[C-1]
+};
+static size_t qg_long_bytes(int hk, int hv, int rows, qg_long *w, char *base)
+{
+    const size_t n = (size_t)(rows + QG_C - 1) / QG_C;
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        char *p = base + off;
+        off += (bytes + 255) & ~(size_t)255;
+        return p;
+    };
+    qg_long l;
+    l.qn = reinterpret_cast<float *>(take(n * QG_C * hk * QG_DK * 4));
+    l.kn = reinterpret_cast<float *>(take(n * QG_C * hk * QG_DK * 4));
+    l.T = reinterpret_cast<float *>(take((size_t)hv * n * QG_C * QG_C * 4));
+    l.QK = reinterpret_cast<float *>(take((size_t)hv * n * QG_C * QG_C * 4));
+    l.sc = reinterpret_cast<float4 *>(take((size_t)hv * n * QG_C * 16));
+    if (w) *w = l;
+    return off;
+}
+
+// D += A B over 16 k: lane (ln, kg) holds A[ln][4 kg ..] and B[4 kg ..][ln],
+// and of D rows 4 kg .. 4 kg + 3 of column ln.  (Step s of the four takes
+// element s of every lane: the same k of A and B.)
+__device__ __forceinline__ qg_f4 qg_mm16(float4 a, float4 b, qg_f4 d)
+{
+    d = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, d, 0, 0, 0);
+    d = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, d, 0, 0, 0);
+    d = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, d, 0, 0, 0);
+    d = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, d, 0, 0, 0);
+    return d;
+}
+
+// Steps past the call's last are g = 1, beta = 0, q = k = 0: they leave the
+// state alone, and no output is written for them.  What k_gdn_chunk reads as
+// MFMA operands is stored in its lanes' order, so that its loads are whole
+// kilobytes (16 rows of 64 bytes a load were twice the lines).
+template <bool PREP>
+__global__ void __launch_bounds__(256) k_gdn_chunk_pre(qg_long w, const float *__restrict__ q,
+                                                       const float *__restrict__ k, const float *__restrict__ g,
+                                                       const float *__restrict__ beta, int hk, int hv, int rows,
+                                                       qg_prep pp)
+{
+    // q and k, then (in their place) a wave's L and masked Q K'
+    constexpr int NQ = 2 * QG_C * QG_CS, NL = 8 * QG_C * QG_TS;
+    __shared__ __align__(16) float lds[NQ > NL ? NQ : NL];
+    __shared__ __align__(16) float KK[QG_C][QG_TS], QK[QG_C][QG_TS];
+    float (*Ks)[QG_CS] = reinterpret_cast<float (*)[QG_CS]>(lds), (*Qs)[QG_CS] = Ks + QG_C;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 15, kg = lane >> 4;
+    const int c = blockIdx.x, hx = blockIdx.y, nch = gridDim.x, n = min(QG_C, rows - c * QG_C);
+
+    // q and k: 8 lanes a step, 16 values each
+    {
+        const int t = tid >> 3, e = tid & 7, tt = c * QG_C + min(t, n - 1);
+        const size_t o = ((size_t)tt * hk + hx) * QG_DK;
+        float4 vq[4], vk[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            vq[i] = reinterpret_cast<const float4 *>(q + o)[e + 8 * i];
+            vk[i] = reinterpret_cast<const float4 *>(k + o)[e + 8 * i];
+        }
+        float fq = t < n ? 1.0f : 0.0f, fk = fq;
+        if (PREP) {
+            // four chains of four and a tree: no longer a chain than the serial form's
+            float sq[4], sk[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                sq[i] = vq[i].x * vq[i].x;                        sk[i] = vk[i].x * vk[i].x;
+                sq[i] = __builtin_fmaf(vq[i].y, vq[i].y, sq[i]);  sk[i] = __builtin_fmaf(vk[i].y, vk[i].y, sk[i]);
+                sq[i] = __builtin_fmaf(vq[i].z, vq[i].z, sq[i]);  sk[i] = __builtin_fmaf(vk[i].z, vk[i].z, sk[i]);
+                sq[i] = __builtin_fmaf(vq[i].w, vq[i].w, sq[i]);  sk[i] = __builtin_fmaf(vk[i].w, vk[i].w, sk[i]);
+            }
+            const float aq = qw_xor_sum<8>((sq[0] + sq[1]) + (sq[2] + sq[3]));
+            const float ak = qw_xor_sum<8>((sk[0] + sk[1]) + (sk[2] + sk[3]));
+            fq *= 1.0f / sqrtf(aq / (float)QG_DK + pp.l2eps) * pp.q_scale;
+            fk *= 1.0f / sqrtf(ak / (float)QG_DK + pp.l2eps) * pp.k_scale;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            // (a select, not the factor 0: what a step past the last reads may be anything)
+            const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+            *reinterpret_cast<float4 *>(&Qs[t][4 * (e + 8 * i)]) =
+                t < n ? make_float4(vq[i].x * fq, vq[i].y * fq, vq[i].z * fq, vq[i].w * fq) : z;
+            *reinterpret_cast<float4 *>(&Ks[t][4 * (e + 8 * i)]) =
+                t < n ? make_float4(vk[i].x * fk, vk[i].y * fk, vk[i].z * fk, vk[i].w * fk) : z;
+        }
+    }
+    __syncthreads();
+    // out in operand order: [tile of 16 steps][j][lane], lane (ln, kg) the four from 16 j + 4 kg of step ln
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int t0 = 16 * (i >> 1), j = 4 * (i & 1) + wave;
+        const size_t o = (((size_t)hx * nch + c) * 16 + (t0 ? 8 : 0) + j) * 64 + lane;
+        reinterpret_cast<float4 *>(w.qn)[o] = *reinterpret_cast<const float4 *>(&Qs[t0 + ln][16 * j + 4 * kg]);
+        reinterpret_cast<float4 *>(w.kn)[o] = *reinterpret_cast<const float4 *>(&Ks[t0 + ln][16 * j + 4 * kg]);
+    }
+    // K K' and Q K', the tiles on and below the diagonal: (0, 0), (1, 0), (1, 1) of each
+    for (int u = wave; u < 6; u += 4) {
+        const int m = (u % 3) > 0 ? 16 : 0, i0 = (u % 3) > 1 ? 16 : 0;
+        const float *A = u < 3 ? &Ks[m + ln][0] : &Qs[m + ln][0], *B = &Ks[i0 + ln][0];
+        qg_f4 d[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) d[i] = qg_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < QG_DK; j += 64)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                d[i] = qg_mm16(*reinterpret_cast<const float4 *>(A + j + 16 * i + 4 * kg),
+                               *reinterpret_cast<const float4 *>(B + j + 16 * i + 4 * kg), d[i]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) (u < 3 ? KK : QK)[m + 4 * kg + e][i0 + ln] = (d[0][e] + d[1][e]) + (d[2][e] + d[3][e]);
+    }
+    __syncthreads();                                              // q and k are consumed
+    // a value head a wave: lane i has column i of P, L, the masked Q K' and T
+    float (*Ls)[QG_TS] = reinterpret_cast<float (*)[QG_TS]>(lds) + wave * 2 * QG_C, (*Ms)[QG_TS] = Ls + QG_C;
+    for (int r = wave; r < hv / hk; r += 4) {
+        const int h = hx * (hv / hk) + r, i = lane & 31;
+        const size_t hc = (size_t)h * nch + c;
+        float gi = 1.0f, bi = 0.0f;                               // step i's gate and beta
+        if (i < n) {
+            const size_t at = (size_t)(c * QG_C + i) * hv + h;
+            if (PREP) qg_gates(pp.a[at], pp.b[at], qw_bf16(pp.A_log[h]), qw_bf16(pp.dt_bias[h]), gi, bi);
+            else { gi = g[at]; bi = beta[at]; }
+        }
+        float p = 0.0f, gam = 1.0f;
+#pragma unroll 4
+        for (int t = 0; t < QG_C; t++) {
+            const float gt = qw_lane(gi, t), bt = qw_lane(bi, t);
+            if (t <= i) gam *= gt;
+            p = t == i ? 1.0f : t > i ? p * gt : 0.0f;
+            if (lane < QG_C) {
+                // (selects: what lies above the diagonal was never written)
+                Ls[t][i] = t > i ? bt * p * KK[t][i] : 0.0f;
+                Ms[t][i] = t >= i ? p * QK[t][i] : 0.0f;
+            }
+        }
+        if (lane < QG_C) w.sc[hc * QG_C + i] = make_float4(bi, bi * gam, gam, p);
+        __builtin_amdgcn_wave_barrier();
+        float x[QG_C];
+#pragma unroll
+        for (int t = 0; t < QG_C; t++) {
+            float a0 = t == i ? 1.0f : 0.0f, a1 = 0.0f;
+#pragma unroll
+            for (int j = 0; j < t; j += 4) {
+                const float4 l = *reinterpret_cast<const float4 *>(&Ls[t][j]);
+                a0 = __builtin_fmaf(-l.x, x[j], a0);
+                if (j + 1 < t) a1 = __builtin_fmaf(-l.y, x[j + 1], a1);
+                if (j + 2 < t) a0 = __builtin_fmaf(-l.z, x[j + 2], a0);
+                if (j + 3 < t) a1 = __builtin_fmaf(-l.w, x[j + 3], a1);
+            }
+            x[t] = a0 + a1;
+            if (lane < QG_C) Ls[t][i] = x[t];                     // T's row t takes L's place
+            __builtin_amdgcn_wave_barrier();
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int f = 0; f < 4; f++) {                             // [tile][j][lane], as q and k
+            const int t0 = 16 * (f >> 1), j = f & 1;
+            const size_t o = (hc * 4 + f) * 64 + lane;
+            reinterpret_cast<float4 *>(w.T)[o] = *reinterpret_cast<const float4 *>(&Ls[t0 + ln][16 * j + 4 * kg]);
+            reinterpret_cast<float4 *>(w.QK)[o] = *reinterpret_cast<const float4 *>(&Ms[t0 + ln][16 * j + 4 * kg]);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// A barrier for LDS that leaves the next chunk's loads in flight.
+__device__ __forceinline__ void qg_sync()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Wave w of four: rows (w & 1) 16 .. of the chunk, of K for waves 0 and 1
+// (which make U) and of Q for 2 and 3 (which make Y); and columns 32 w .. of
+// the state, as D tiles of S' (k rows, v columns), so that a lane's four are
+// a 16-byte piece of S[v][k].  QG_VT tiles of 16 value rows a workgroup: with
+// one, two workgroups share a CU and cover each other's barriers (2048 steps:
+// 243 us; with two, 316).
+#define QG_VT 1
+__global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restrict__ y, const float *__restrict__ v,
+                                                      float *state, int hk, int hv, int rows)
+{
+    __shared__ __align__(16) float Ss[16 * QG_VT][QG_CS], Ks[QG_C][QG_CS];
+    __shared__ __align__(16) float Rt[16 * QG_VT][QG_TS], Ut[16 * QG_VT][QG_TS], Up[16 * QG_VT][QG_TS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 15, kg = lane >> 4;
+    // the workgroups of a key head (which read its q and k) on one XCD
+    constexpr unsigned per = QG_DV / (16 * QG_VT);
+    const unsigned total = gridDim.x, b = blockIdx.x;
+    const unsigned id = total % 8u == 0u ? (b % 8u) * (total / 8u) + b / 8u : b;
+    const int h = (int)(id / per), v0 = 16 * QG_VT * (int)(id % per), hx = h / (hv / hk);
+    const int nch = (rows + QG_C - 1) / QG_C, t0 = 16 * (wave & 1);
+    const bool isq = wave >= 2;
+
+    float *sp = state + ((size_t)h * QG_DV + v0 + ln) * QG_DK + 32 * wave + 4 * kg;
+    qg_f4 S[QG_VT][2];
+#pragma unroll
+    for (int z = 0; z < QG_VT; z++)
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            S[z][u] = *reinterpret_cast<const qg_f4 *>(sp + z * 16 * QG_DK + 16 * u);
+            *reinterpret_cast<qg_f4 *>(&Ss[16 * z + ln][32 * wave + 16 * u + 4 * kg]) = S[z][u];
+        }
+    // a chunk's operands, fetched a chunk ahead: 16 rows of K or Q, the rows'
+    // scalars, T or the masked Q K' and (waves 0 and 1) V
+    const float4 *kq = reinterpret_cast<const float4 *>(isq ? w.qn : w.kn) + ((size_t)hx * nch * 16 + t0 / 2) * 64 + lane;
+    const float4 *tq = reinterpret_cast<const float4 *>(isq ? w.QK : w.T) + ((size_t)h * nch * 4 + t0 / 8) * 64 + lane;
+    const float4 *sc = w.sc + (size_t)h * nch * QG_C + t0 + 4 * kg;
+    float4 fa[8], ft[2], fs[4];
+    float fv[QG_VT][4] = {}, fg;
+    auto fetch = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) fa[j] = kq[((size_t)c * 16 + j) * 64];
+#pragma unroll
+        for (int j = 0; j < 2; j++) ft[j] = tq[((size_t)c * 4 + j) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; e++) fs[e] = sc[(size_t)c * QG_C + e];
+        if (!isq) {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int z = 0; z < QG_VT; z++)
+                    fv[z][e] = v[((size_t)min(c * QG_C + t0 + 4 * kg + e, rows - 1) * hv + h) * QG_DV + v0 + 16 * z + ln];
+        }
+        fg = w.sc[((size_t)h * nch + c) * QG_C + QG_C - 1].z;     // G[C - 1]
+    };
+    fetch(0);
+    qg_sync();
+    for (int c = 0; c < nch; c++) {
+        float4 a[8], tm[2], s4[4];
+        float vv[QG_VT][4];
+#pragma unroll
+        for (int j = 0; j < 8; j++) a[j] = fa[j];
+#pragma unroll
+        for (int j = 0; j < 2; j++) tm[j] = ft[j];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            s4[e] = fs[e];
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++) vv[z][e] = fv[z][e];
+        }
+        const float gc = fg;
+        if (c + 1 < nch) fetch(c + 1);
+        if (!isq) {
+#pragma unroll
+            for (int j = 0; j < 8; j++) *reinterpret_cast<float4 *>(&Ks[t0 + ln][16 * j + 4 * kg]) = a[j];
+        }
+        // K S0' or Q S0': four chains a tile, met in a tree (one chain of 32 sums rounds more than the serial form)
+        qg_f4 d[QG_VT];
+        {
+            qg_f4 dd[QG_VT][4];
+            float4 sb[QG_VT][8];
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+#pragma unroll
+                for (int z = 0; z < QG_VT; z++)
+                    sb[z][j] = *reinterpret_cast<const float4 *>(&Ss[16 * z + ln][16 * j + 4 * kg]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++) dd[z][0] = dd[z][1] = dd[z][2] = dd[z][3] = qg_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 8; j += 4)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+#pragma unroll
+                        for (int z = 0; z < QG_VT; z++)
+                            dd[z][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&a[j + i])[e],
+                                                                           reinterpret_cast<const float *>(&sb[z][j + i])[e],
+                                                                           dd[z][i], 0, 0, 0);
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) d[z][e] = (dd[z][0][e] + dd[z][1][e]) + (dd[z][2][e] + dd[z][3][e]);
+        }
+        if (!isq) {
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++) {
+                qg_f4 r;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const bool in = c * QG_C + t0 + 4 * kg + e < rows;
+                    r[e] = in ? __builtin_fmaf(s4[e].x, vv[z][e], -(s4[e].y * d[z][e])) : 0.0f;
+                }
+                *reinterpret_cast<qg_f4 *>(&Rt[16 * z + ln][t0 + 4 * kg]) = r;
+            }
+        }
+        qg_sync();
+        // X over the chunk's 32 steps against T's or the masked Q K's 16 rows (upper right tile zero)
+        auto over = [&](const float (*X)[QG_TS], qg_f4 (&o)[QG_VT]) __attribute__((always_inline)) {
+            float4 x0[QG_VT], x1[QG_VT];
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++) {
+                x0[z] = *reinterpret_cast<const float4 *>(&X[16 * z + ln][4 * kg]);
+                x1[z] = *reinterpret_cast<const float4 *>(&X[16 * z + ln][16 + 4 * kg]);
+            }
+            qg_f4 p[QG_VT];
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++) p[z] = qg_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int z = 0; z < QG_VT; z++) {
+                    o[z] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&tm[0])[e],
+                                                                reinterpret_cast<const float *>(&x0[z])[e], o[z], 0, 0, 0);
+                    if (t0)
+                        p[z] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&tm[1])[e],
+                                                                    reinterpret_cast<const float *>(&x1[z])[e], p[z], 0, 0, 0);
+                }
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[z][e] += p[z][e];
+        };
+        if (!isq) {
+            // U = T R
+            qg_f4 u[QG_VT];
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++) u[z] = qg_f4{0.f, 0.f, 0.f, 0.f};
+            over(Rt, u);
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++) {
+                qg_f4 up;
+#pragma unroll
+                for (int e = 0; e < 4; e++) up[e] = u[z][e] * s4[e].w;
+                *reinterpret_cast<qg_f4 *>(&Ut[16 * z + ln][t0 + 4 * kg]) = u[z];
+                *reinterpret_cast<qg_f4 *>(&Up[16 * z + ln][t0 + 4 * kg]) = up;
+            }
+        }
+        qg_sync();
+        // S' = G[C-1] S0' + K' (P U)
+        {
+            float4 bu[QG_VT][2], ka[2][2];
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) bu[z][i] = *reinterpret_cast<const float4 *>(&Up[16 * z + ln][16 * i + 4 * kg]);
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const int kc = 32 * wave + 16 * u + ln, r = 16 * i + 4 * kg;
+                    ka[u][i] = make_float4(Ks[r][kc], Ks[r + 1][kc], Ks[r + 2][kc], Ks[r + 3][kc]);
+                }
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++)
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) S[z][u][e] *= gc;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int u = 0; u < 2; u++)
+#pragma unroll
+                        for (int z = 0; z < QG_VT; z++)
+                            S[z][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&ka[u][i])[e],
+                                                                          reinterpret_cast<const float *>(&bu[z][i])[e],
+                                                                          S[z][u], 0, 0, 0);
+        }
+        if (isq) {
+            // Y = G Q S0' + (P o Q K') U
+            qg_f4 o[QG_VT];
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[z][e] = s4[e].z * d[z][e];
+            over(Ut, o);
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int t = c * QG_C + t0 + 4 * kg + e;
+                    if (t < rows) y[((size_t)t * hv + h) * QG_DV + v0 + 16 * z + ln] = o[z][e];
+                }
+        }
+#pragma unroll
+        for (int z = 0; z < QG_VT; z++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) *reinterpret_cast<qg_f4 *>(&Ss[16 * z + ln][32 * wave + 16 * u + 4 * kg]) = S[z][u];
+        qg_sync();
+    }
+#pragma unroll
+    for (int z = 0; z < QG_VT; z++)
+#pragma unroll
+        for (int u = 0; u < 2; u++) *reinterpret_cast<qg_f4 *>(sp + z * 16 * QG_DK + 16 * u) = S[z][u];
+}
+
 // ---- launchers ----------------------------------------------------------------
 
 extern "C" int qwk_conv1d_causal_silu(hipStream_t s, float *y, const float *x, float *state, const uint16_t *w,
@@ -416,8 +847,16 @@ extern "C" int qwk_gdn_gates(hipStream_t s, float *g, float *beta, const float *
     return (int)hipGetLastError();
 }
 
-extern "C" size_t qwk_gated_delta_work(int hk, int hv, int rows, int prep)
+// Whether a call takes the chunks, and its scratch: a function of the shape.
+static bool qg_is_long(int hk, int hv, int rows, int n_snap)
 {
+    return rows >= QG_LONG_MIN_ROWS && n_snap == 0 && hk >= 1 && hv >= hk && hv % hk == 0;
+}
+
+extern "C" size_t qwk_gated_delta_work(int hk, int hv, int rows, int prep, int n_snap)
+{
+    if (qg_is_long(hk, hv, rows, n_snap))
+        return qg_long_bytes(hk, hv, rows < QG_LONG_ROWS ? rows : QG_LONG_ROWS, nullptr, nullptr);
     if (!prep || rows < QG_PRE_MIN_ROWS || hk < 1 || hv < 1) return 0;
     return ((size_t)rows * hk * 2 + (size_t)rows * hv * 2) * sizeof(float);
 }
@@ -432,10 +871,31 @@ extern "C" int qwk_gated_delta(hipStream_t s, float *y, const float *q, const fl
         return hipErrorInvalidValue;
     if (rows == 0) return 0;
     const dim3 grid(hv * (QG_DV / QG_ROWS_PER_WG));
+    if (work && qg_is_long(hk, hv, rows, n_snap)) {
+        for (int r0 = 0; r0 < rows; r0 += QG_LONG_ROWS) {
+            const int r = rows - r0 < QG_LONG_ROWS ? rows - r0 : QG_LONG_ROWS;
+            const size_t oq = (size_t)r0 * hk * QG_DK, ov = (size_t)r0 * hv * QG_DV, og = (size_t)r0 * hv;
+            qg_long w;
+            qg_long_bytes(hk, hv, r, &w, static_cast<char *>(work));
+            const dim3 pre((r + QG_C - 1) / QG_C, hk);
+            if (prep) {
+                const qg_prep pp = { prep->a + og, prep->b + og, prep->A_log, prep->dt_bias, prep->l2eps, prep->q_scale,
+                                     prep->k_scale, nullptr, nullptr };
+                hipLaunchKernelGGL(k_gdn_chunk_pre<true>, pre, dim3(256), 0, s, w, q + oq, k + oq, nullptr, nullptr, hk,
+                                   hv, r, pp);
+            } else {
+                const qg_prep pp = {};
+                hipLaunchKernelGGL(k_gdn_chunk_pre<false>, pre, dim3(256), 0, s, w, q + oq, k + oq, g + og, beta + og,
+                                   hk, hv, r, pp);
+            }
+            hipLaunchKernelGGL(k_gdn_chunk, dim3(hv * (QG_DV / (16 * QG_VT))), dim3(256), 0, s, w, y + ov, v + ov, state, hk, hv, r);
+        }
+        return (int)hipGetLastError();
+    }
     if (prep) {
         qg_prep pp = { prep->a, prep->b, prep->A_log, prep->dt_bias, prep->l2eps, prep->q_scale, prep->k_scale,
                        nullptr, nullptr };
-        if (work && qwk_gated_delta_work(hk, hv, rows, 1) > 0) {
+        if (work && rows >= QG_PRE_MIN_ROWS) {
             pp.nrm = static_cast<float *>(work);
             pp.gb = pp.nrm + (size_t)rows * hk * 2;
             const int nbv = (rows * hk * 2 + 3) / 4, nbg = (rows * hv + 255) / 256;

@@ -272,9 +272,11 @@ int qwk_gdn_gates(hipStream_t s, float *g, float *beta, const float *a, const fl
                   const uint16_t *A_log, const uint16_t *dt_bias, int hv, int rows);
 /* prep NULL: q, k normed and g, beta given; else g and beta are unused.
  * work: qwk_gated_delta_work() bytes of device memory (NULL when that is 0):
- * a long prepared call computes its norms and gates there first, in
- * parallel, instead of a chunk at a time inside the recurrence. */
-size_t qwk_gated_delta_work(int hk, int hv, int rows, int prep);
+ * a prepared call of 64 steps on computes its norms and gates there first, in
+ * parallel, instead of a chunk at a time inside the recurrence; a call of 256
+ * on without snapshots works in chunks of 32 steps (qw_gdn.hip) and keeps
+ * their operands there. */
+size_t qwk_gated_delta_work(int hk, int hv, int rows, int prep, int n_snap);
 int qwk_gated_delta(hipStream_t s, float *y, const float *q, const float *k, const float *v,
                     const float *g, const float *beta, float *state, int hk, int hv, int dk, int dv,
                     int rows, float *snap, int n_snap, int snap_stride, const qwk_gdn_prep *prep, void *work);

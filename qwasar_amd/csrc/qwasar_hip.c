@@ -1210,7 +1210,7 @@ static void gated_delta(qw_cmd c, qw_ref y, qw_ref q, qw_ref k, qw_ref v, qw_ref
     } else {
         touch(c, g, 0); touch(c, beta, 0);
     }
-    const size_t wb = qwk_gated_delta_work(hk, hv, rows, prep != NULL);
+    const size_t wb = qwk_gated_delta_work(hk, hv, rows, prep != NULL, n_snap > 0 ? n_snap : 0);
     void *work = wb ? scratch(wb) : NULL;
     if (wb && !work) { cmd_fail(c, hipErrorOutOfMemory, "gated_delta: scratch of %zu bytes", wb); return; }
     launched(c, prep ? "gated_delta_prep" : "gated_delta",

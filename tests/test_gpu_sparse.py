@@ -490,3 +490,56 @@ def test_rms_norm_gated_sigmoid(gpu):
     gpu.run(c, "rms norm gated sigmoid")
     want = sparse.rms_norm_gated_sigmoid(x, w, gate, dim, rows, EPS)
     assert np.allclose(yb.read(np.float32, (rows, dim)), want, rtol=3e-6, atol=1e-7)
+
+
+# ---- the delta rule in chunks (256 steps on) --------------------------------------------
+
+@pytest.mark.parametrize("hk,hv,rows,decay", [
+    (16, 48, 256, "usual"),      # whole chunks of 32, the model's heads
+    (2, 4, 257, "usual"),        # one step into a last chunk
+    (1, 5, 287, "none"),         # g = 1: nothing is forgotten; more value heads a key head than waves
+    (3, 3, 300, "strong"),       # g down to zero: running products, no quotients
+    (1, 2, 4130, "usual"),       # past one pair of launches' steps
+])
+def test_gated_delta_chunks(gpu, hk, hv, rows, decay):
+    """The chunked form against the oracle's serial one, with the op's usual
+    bar (rel-L2 5e-6 on outputs and state); per step as well where nothing
+    decays, so that no step hides behind the rest."""
+    q, k, v, g, beta, s0 = delta_inputs(hk, hv, rows, 11 + rows)
+    if decay == "none":
+        g[:] = 1.0
+        beta[:] = 0.5
+    elif decay == "strong":
+        g[:] = np.random.default_rng(3).choice(np.float32([0.0, 1e-30, 1e-3, 0.5, 1.0]), g.shape)
+    y, s1, _ = gpu_delta(gpu, q, k, v, g, beta, s0, hk, hv, rows)
+    wy, ws, _ = sparse.gated_delta(q, k, v, g, beta, s0, hk, hv, 128, 128, rows)
+    assert rel_l2(y, wy) < 5e-6 and rel_l2(s1, ws) < 5e-6, (rel_l2(y, wy), rel_l2(s1, ws))
+    for t in (0, 1, 31, 32, 63, rows - 2, rows - 1):
+        # a single step's output: 128 dims a head, the bound above with the scatter of fewer terms
+        assert rel_l2(y[t], wy[t]) < 2e-5, f"step {t}"
+
+
+@pytest.mark.parametrize("hk,hv,rows", [(16, 48, 270), (2, 6, 320)])
+def test_gated_delta_prep_chunks(gpu, hk, hv, rows):
+    """Prepared: norms and gates ahead of the chunks; snapshots asked for
+    keep the serial form (and its bits with shorter calls)."""
+    dk = dv = 128
+    q, k, v = rnd((rows, hk, dk), 241), rnd((rows, hk, dk), 242), rnd((rows, hv, dv), 243)
+    a, b = rnd((rows, hv), 244, -4, 4), rnd((rows, hv), 245, -4, 4)
+    s0 = rnd((hv, dv, dk), 246) * np.float32(0.05)
+    Al, dt = np.ascontiguousarray(np.resize(FX["A_log"], hv)), np.ascontiguousarray(np.resize(FX["dt_bias"], hv))
+    eps, qs, ks = 1e-6 / dk, 1.0 / dk, 1.0 / np.sqrt(dk)
+    B = gpu.Buf
+    qb, kb, vb, ab, bb, Ab, db = B.of(q), B.of(k), B.of(v), B.of(a), B.of(b), B.of(Al), B.of(dt)
+    prep = gpu.qw_gdn_prep(ab.ref(), bb.ref(), Ab.ref(), db.ref(), eps, qs, ks)
+    s1, s2, y1, y2 = B.of(s0), B.of(s0), B(v.nbytes), B(v.nbytes)
+    snap = B(hv * dv * dk * 4)
+    c = gpu.qw_cmd_begin()
+    gpu.qw_op_gated_delta_prep(c, y1.ref(), qb.ref(), kb.ref(), vb.ref(), prep, s1.ref(), hk, hv, dk, dv, rows,
+                               gpu.NULL_REF, 0, 0)
+    gpu.qw_op_gated_delta_prep(c, y2.ref(), qb.ref(), kb.ref(), vb.ref(), prep, s2.ref(), hk, hv, dk, dv, rows,
+                               snap.ref(), 1, hv * dv * dk)
+    gpu.run(c, "gated delta prep, chunks")
+    wy, ws, _ = sparse.gated_delta_prep(q, k, v, a, b, Al, dt, eps, qs, ks, s0, hk, hv, dk, dv, rows)
+    for yb, sb in ((y1, s1), (y2, s2)):
+        assert rel_l2(yb.read(np.float32, v.shape), wy) < 5e-6 and rel_l2(sb.read(np.float32, s0.shape), ws) < 5e-6
