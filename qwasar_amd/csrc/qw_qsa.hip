@@ -9,14 +9,15 @@
 // the first 64 dims at the block's first position -- lanes j and j+32, one
 // swizzle apart.
 //
-// Score (phase 2): the keys are transposed through LDS so that a thread owns
+// Score: up to 16 query heads of up to 128 dims on the fp32 matrix cores
+// (k_qsa_scores_mx, below); else (k_qsa_scores phase 2) the keys are transposed through LDS so that a thread owns
 // one block's key in registers; the row's query heads sit in LDS and are read
 // as broadcast float4s.  Thread (wave w, lane l) scores block l against heads
 // w, w+4, ...: per head a serial fma chain over the dims, the positive dots
 // summed in head order; the four waves' partials meet as (p0 + p1) + (p2 +
-// p3), then / sqrt(d).  The arithmetic does not depend on how many rows or
-// blocks a call has, and the pooled path runs the same phase 2 on stored keys,
-// so scores and pooled scores agree bit for bit.
+// p3), then / sqrt(d).  Either way the arithmetic does not depend on how many
+// rows or blocks a call has, and the pooled path runs the same sums on stored
+// keys, so scores and pooled scores agree bit for bit.
 //
 // Selection (k_qsa_select): a workgroup of 1024 threads per query.  Scores
 // map to 32-bit keys that order as the floats do (-0 as +0; -FLT_MAX, -inf
@@ -191,94 +192,128 @@ __global__ void __launch_bounds__(QS_THREADS) __attribute__((amdgpu_waves_per_eu
     qs_score_rows<D>(scores, qn, kl, ql, part, b0, r0, rows, nq, d, ratio, base_pos, max_blocks);
 }
 
-// The same scores on the fp32 matrix cores (nq <= 16, D <= 128, many rows).
-// v_mfma_f32_16x16x1_4b_f32 adds a 16x16 outer product to its accumulator in
-// each of four blocks, one rounding per element: element (i, j) of a block
-// takes fmaf(a_i, b_j, c), so D of them in dim order are phase 2's chain
-// (from 0, dims ascending), bit for bit.  Lane l feeds B column l % 16 of
-// block l / 16 with its own block's key -- block b0 + l, held in registers
-// for the whole tile -- and A row l % 16 of every block with one query row's
-// head hd(l % 16), hd(i) = 4 (i % 4) + i / 4 (heads past nq zero: a zero dot,
-// never summed).  Accumulator e of lane l is then block column 16 (e / 4) +
-// l % 16 against A row 4 (l / 16) + e % 4, head l / 16 + 4 (e % 4): the lanes
-// of group g = l / 16 hold heads g, g + 4, g + 8, g + 12 in e order, the
-// heads phase 2's wave g sums, in its order.  Two xor shuffles (16, then 32)
-// form (p0 + p1) + (p2 + p3) (each pair's sum the same bits whichever lane
-// adds it), and lane l writes block b0 + l.  A workgroup scores its 64 blocks
-// against QM_ROWS rows, eight at a time: the eight rows' heads are staged in
-// LDS (over the block keys, once those are in registers), each wave runs two
-// rows' chains interleaved.
+// The scores on the fp32 matrix cores (nq <= 16, D <= 128).  The query heads
+// are the rows of an MFMA tile (heads past nq zero: a zero dot, never summed)
+// and 16 blocks its columns, so one query row fills the instruction
+// (v_mfma_f32_16x16x4_f32) and a decode step takes the same kernel, and the
+// same bits, as a chunk's rows.  Lane (ln, kg) holds dims 16 j + 4 kg .. + 3
+// of head ln (A) and of block ln (B), element e feeding step e of the four, so
+// both sides list the same dims.  A lane's accumulators are block ln's dots
+// with heads 4 kg .. 4 kg + 3: their positive ones are summed in order, then
+// over kg by two xor shuffles.
+// A workgroup has NW waves of 16 TB blocks, whose keys stay in registers
+// while it walks its rows; the rows' heads pass through LDS eight rows at a
+// time (one row alone is read straight from memory).
+// 512 rows at 16K: 127 us with K = 1 MFMAs (the serial chain's order, half
+// the rate), 102 here; one row of 8192 blocks: 10.0 us with a thread a block,
+// 4.1 here.  What bounds it: many rows, the fp32 MFMA's issue (35 cycles each,
+// 60 of the 102) and the staging between groups of rows; one row, the trip to
+// memory.
 #define QM_ROWS 32
-#define QM_GROUP 8                                 // rows staged at once: 2 a wave
-template <int D, bool POOLED>
-__global__ void __launch_bounds__(QS_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) k_qsa_scores_mx(
+#define QM_GROUP 8                                 // rows staged at once
+template <int D, bool POOLED, int TB, int NW, bool ONE>
+__global__ void __launch_bounds__(64 * NW, ONE ? 1 : 2) k_qsa_scores_mx(
     float *__restrict__ scores, const float *__restrict__ qn, const float *__restrict__ src,
     const uint16_t *__restrict__ kw, const float *__restrict__ inv_freq, int rows, int nq, int d, int ratio,
     int base_pos, int max_blocks, float eps)
 {
-    typedef float f16v __attribute__((ext_vector_type(4 * 4)));
-    constexpr int QST = 16 * (D + 4);                          // floats a staged row
-    __shared__ float4 lds4[(QM_GROUP * QST > QS_BLK * (D + 4) ? QM_GROUP * QST : QS_BLK * (D + 4)) / 4];
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    static_assert(POOLED || (16 * TB * NW == QS_BLK && 64 * NW == QS_THREADS), "direct keys: qs_keys_to_lds's workgroup");
+    constexpr int QST = 16 * (D + 4), NJ = D / 16;             // floats a staged row; float4s a lane a head
+    constexpr int LQ = ONE ? 0 : QM_GROUP * QST, LK = POOLED ? 0 : QS_BLK * (D + 4), LN = LQ > LK ? LQ : LK;
+    __shared__ float4 lds4[LN / 4 + 1];
     float *lds = reinterpret_cast<float *>(lds4);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int b0 = blockIdx.x * QS_BLK, r0 = blockIdx.y * QM_ROWS;
-    const int rend = min(r0 + QM_ROWS, rows);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 15, kg = lane >> 4;
+    const int b0 = blockIdx.x * (16 * TB * NW), r0 = blockIdx.y * QM_ROWS;
+    const int rend = min(r0 + QM_ROWS, rows), wb = b0 + wave * 16 * TB;
     const int nb_hi = (base_pos + rend) / ratio;
     if (nb_hi <= b0) return;                                   // uniform
-    qs_keys_to_lds<D, POOLED>(lds, src, kw, inv_freq, b0, nb_hi, d, ratio, eps);
-    __syncthreads();
-    float kr[D];
+    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 key[TB][NJ];
+    if (POOLED) {
+        // every load issued, at a clamped place; dims past d zeroed after (d % 32 == 0: whole float4s)
 #pragma unroll
-    for (int i = 0; i < D; i += 4) {
-        const float4 v = *reinterpret_cast<const float4 *>(lds + lane * (D + 4) + i);
-        kr[i] = v.x; kr[i + 1] = v.y; kr[i + 2] = v.z; kr[i + 3] = v.w;
+        for (int t = 0; t < TB; t++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                key[t][j] = *reinterpret_cast<const float4 *>(src + (size_t)min(wb + 16 * t + ln, nb_hi - 1) * d +
+                                                              min(16 * j + 4 * kg, d - 4));
+    } else {
+        qs_keys_to_lds<D, false>(lds, src, kw, inv_freq, b0, nb_hi, d, ratio, eps);
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TB; t++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                key[t][j] = *reinterpret_cast<const float4 *>(lds + (wave * 16 * TB + 16 * t + ln) * (D + 4) + 16 * j + 4 * kg);
+    }
+    float4 one[ONE ? NJ : 1];
+    if (ONE) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+            one[j] = *reinterpret_cast<const float4 *>(qn + ((size_t)r0 * nq + min(ln, nq - 1)) * d + min(16 * j + 4 * kg, d - 4));
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+            if (ln >= nq || 16 * j + 4 * kg >= d) one[j] = z4;
+    }
+    if (POOLED) {
+#pragma unroll
+        for (int t = 0; t < TB; t++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                if (16 * j + 4 * kg >= d) key[t][j] = z4;
     }
     const float rs = sqrtf((float)d);
-    const int g = lane >> 4;
-    const float *qa = lds + (2 * wave) * QST + (lane & 15) * (D + 4), *qb = qa + QST;
+    auto score = [&](const float4 (&a)[NJ], int r) __attribute__((always_inline)) {
+        f4v acc[TB];
+#pragma unroll
+        for (int t = 0; t < TB; t++) acc[t] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const float av[4] = {a[j].x, a[j].y, a[j].z, a[j].w};
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int t = 0; t < TB; t++) {
+                    const float kv[4] = {key[t][j].x, key[t][j].y, key[t][j].z, key[t][j].w};
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], kv[e], acc[t], 0, 0, 0);
+                }
+        }
+        float mine = 0.0f;
+#pragma unroll
+        for (int t = 0; t < TB; t++) {
+            float p = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (acc[t][e] > 0.0f) p += acc[t][e];
+            p = p + __shfl_xor(p, 16, 64);
+            p = p + __shfl_xor(p, 32, 64);
+            if (t == kg) mine = p;
+        }
+        const int b = wb + 16 * kg + ln;
+        if (kg < TB && b < (base_pos + r + 1) / ratio) scores[(size_t)r * max_blocks + b] = mine / rs;
+    };
+    if (ONE) {
+        if constexpr (ONE) score(one, r0);
+        return;
+    }
     for (int g0 = r0; g0 < rend; g0 += QM_GROUP) {
         const int gl = min(g0 + QM_GROUP, rend);
         if ((base_pos + gl) / ratio <= b0) continue;           // uniform: no row of the group sees these blocks
         __syncthreads();                                       // the keys are in registers / the last group is done
-        // stage: A row i of staged row t holds head hd(i) (4 x 4 transpose: its own inverse)
-        for (int q = tid; q < QM_GROUP * 16 * (D / 4); q += QS_THREADS) {
-            const int t = q / (16 * (D / 4)), i = (q / (D / 4)) % 16, j = 4 * (q % (D / 4));
-            const int h = 4 * (i % 4) + i / 4, r = g0 + t;
-            float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (int i = tid; i < QM_GROUP * 16 * (D / 4); i += 64 * NW) {
+            const int t = i / (16 * (D / 4)), h = (i / (D / 4)) % 16, j = 4 * (i % (D / 4)), r = g0 + t;
+            float4 v = z4;
             if (r < gl && h < nq && j < d) v = *reinterpret_cast<const float4 *>(qn + ((size_t)r * nq + h) * d + j);
-            *reinterpret_cast<float4 *>(lds + t * QST + i * (D + 4) + j) = v;
+            *reinterpret_cast<float4 *>(lds + t * QST + h * (D + 4) + j) = v;
         }
         __syncthreads();
-        f16v acc0 = {}, acc1 = {};
+        for (int r = g0; r < gl; r++) {
+            float4 a[NJ];
 #pragma unroll
-        for (int k = 0; k < D; k += 4) {
-            const float4 a0 = *reinterpret_cast<const float4 *>(qa + k), a1 = *reinterpret_cast<const float4 *>(qb + k);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x1f32(a0.x, kr[k], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x1f32(a1.x, kr[k], acc1, 0, 0, 0);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x1f32(a0.y, kr[k + 1], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x1f32(a1.y, kr[k + 1], acc1, 0, 0, 0);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x1f32(a0.z, kr[k + 2], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x1f32(a1.z, kr[k + 2], acc1, 0, 0, 0);
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x1f32(a0.w, kr[k + 3], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x1f32(a1.w, kr[k + 3], acc1, 0, 0, 0);
-        }
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const int r = g0 + 2 * wave + u;
-            const f16v &acc = u ? acc1 : acc0;
-            float mine = 0.0f;
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                float p = 0.0f;
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-                    if (acc[4 * c + t] > 0.0f) p += acc[4 * c + t];
-                const float x = p + __shfl_xor(p, 16, 64);
-                const float sc = x + __shfl_xor(x, 32, 64);
-                if (c == g) mine = sc;
-            }
-            const int b = b0 + lane;
-            if (r < gl && b < (base_pos + r + 1) / ratio) scores[(size_t)r * max_blocks + b] = mine / rs;
+            for (int j = 0; j < NJ; j++)
+                a[j] = *reinterpret_cast<const float4 *>(lds + (r - g0) * QST + ln * (D + 4) + 16 * j + 4 * kg);
+            score(a, r);
         }
     }
 }
@@ -807,6 +842,265 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
     }
 }
 
+// ---- masked attention on the matrix cores -------------------------------------------
+//
+// The same split of the work (a workgroup a row, kv head and split) for many
+// query heads a kv head, where k_attn_masked's multiply-adds bind it (G = 12:
+// 26 GFLOP of fp32 vector work for 512 rows of 2052 positions, 850 us).  Both
+// products run on f16 MFMAs with nothing rounded to 16 bits: the caches are
+// f16 as they are, and each fp32 operand is cut into three f16 parts (33
+// bits), a part a MFMA, summed in fp32:
+//   q   scaled a head by the power of two that puts its largest magnitude in
+//       [2^14, 2^15); the parts stay in LDS for the row
+//   p   the softmax weights 2^(s - m), at most 2^8 (below), times 2^6
+// The scores are computed transposed, S'[position][head] = K q': a lane then
+// holds its head's weights for positions 4 kg .. 4 kg + 3 of two tiles of 16,
+// which is an A operand of the second product as it stands if the MFMA's k
+// slots 8 kg .. are taken to be those positions.  V's operand must list the
+// same positions of one dim a lane: a lane loads 8 dims (16 bytes) of each of
+// its 8 positions and takes column t of that 8 x 8 block, by v_perm, as tile
+// t's operand, so tile t holds dims 8 n + t.  No value passes through LDS.
+// A wave takes 32 positions a pass and keeps its own softmax state; the
+// reference maximum moves only when a score passes it by 8 (a weight is then
+// at most 2^8 of the state's unit), so the sums are seldom rescaled.  The four
+// waves' states meet in LDS at the end, as (w0 + w1) + (w2 + w3).
+// 512 rows of 2052 positions at 16K, 24 / 2 heads: 850 -> 185 us, and closer
+// to 64 bits (2.5e-7 against 4.3e-7).  What bounds it: the gathered rows, 1 KB
+// a position and kv head, 2.1 GB for that call: 11.6 TB/s through the L1s.
+typedef _Float16 qa_h8 __attribute__((ext_vector_type(8)));
+typedef float qa_f4 __attribute__((ext_vector_type(4)));
+#define QAM_HEADS 16                      // a MFMA tile of heads (G of them real)
+#define QAM_QST (QA_D + 8)                // halfs a head's row takes in LDS
+#define QAM_OST (QA_D + 4)                // floats
+#define QAM_STEP 32                       // positions a wave takes a pass
+#define QAM_P_EXP 6
+#define QAM_SLACK 8.0f
+
+// x as three f16 parts, x = a + b + c to 33 bits (fewer near f16's smallest)
+__device__ __forceinline__ void qa_split(float x, _Float16 &a, _Float16 &b, _Float16 &c)
+{
+    a = (_Float16)x;
+    float r = x - (float)a;
+    b = (_Float16)r;
+    r = r - (float)b;
+    c = (_Float16)r;
+}
+
+template <int G>
+__global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, const float *__restrict__ gate,
+                                                    const float *__restrict__ q, const uint16_t *__restrict__ kc,
+                                                    const uint16_t *__restrict__ vc, const uint32_t *__restrict__ list,
+                                                    int q_heads, int kv_heads, int max_ctx, float scale, int cap,
+                                                    int nsplit, float *__restrict__ part)
+{
+    constexpr int QB = 3 * QAM_HEADS * QAM_QST * 2, OB = 4 * QAM_HEADS * QAM_OST * 4;
+    __shared__ __align__(16) uint8_t lds[QB > OB ? QB : OB];
+    __shared__ float qf[QAM_HEADS];                   // a head's score factor
+    __shared__ float wm[4][QAM_HEADS], wl[4][QAM_HEADS];
+    _Float16 (*qp)[QAM_HEADS][QAM_QST] = reinterpret_cast<_Float16 (*)[QAM_HEADS][QAM_QST]>(lds);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 15, kg = lane >> 4;
+    const int split = blockIdx.x % nsplit, rk = blockIdx.x / nsplit;
+    const int row = rk / kv_heads, kvh = rk % kv_heads;
+    const uint32_t *lr = list + (size_t)row * (1 + cap);
+    const int per = ((cap + QA_P - 1) / QA_P + nsplit - 1) / nsplit;
+    const int j_lo = min(split * per * QA_P, cap), j_cap = min(j_lo + per * QA_P, cap);
+    const int j_hi = min(j_cap, (int)min(lr[0], (uint32_t)cap));
+
+    // the heads, a wave four: lane l dims 4 l ..
+#pragma unroll
+    for (int u = 0; u < QAM_HEADS / 4; u++) {
+        const int g = 4 * u + wave;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (g < G) v = reinterpret_cast<const float4 *>(q + ((size_t)row * q_heads + (size_t)kvh * G + g) * QA_D)[lane];
+        const float mx = qw_wave_max(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+        int sh = 0;
+        if (mx > 0.0f && mx <= FLT_MAX) {
+            sh = 15 - __builtin_amdgcn_frexp_expf(mx);
+            sh = sh < -100 ? -100 : sh > 100 ? 100 : sh;
+        }
+        const float f[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            _Float16 a, b, c;
+            qa_split(__builtin_ldexpf(f[i], sh), a, b, c);
+            qp[0][g][4 * lane + i] = a;
+            qp[1][g][4 * lane + i] = b;
+            qp[2][g][4 * lane + i] = c;
+        }
+        if (lane == 0) qf[g] = __builtin_ldexpf(scale * QA_LOG2E, -sh);
+    }
+    __syncthreads();
+
+    const uint16_t *kbase = kc + (size_t)kvh * max_ctx * QA_D + 8 * kg;      // K: dims 32 s + 8 kg of position ln
+    const uint16_t *vbase = vc + (size_t)kvh * max_ctx * QA_D + 8 * ln;      // V: dims 8 ln (and 128 on) of 8 positions
+    const float fac = qf[ln];
+    float m = -FLT_MAX, l = 0.0f;
+    qa_f4 acc[16];
+#pragma unroll
+    for (int t = 0; t < 16; t++) acc[t] = qa_f4{0.f, 0.f, 0.f, 0.f};
+
+    // list entries of a pass from j0 (past the range: its last, whose weight is then zero)
+    auto at = [&](int j) { return min(lr[1 + min(j, j_hi - 1)], (uint32_t)(max_ctx - 1)); };
+    uint32_t ki[2], vi[8];
+    auto entries = [&](int j0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < 2; t++) ki[t] = at(j0 + 16 * t + ln);
+#pragma unroll
+        for (int i = 0; i < 8; i++) vi[i] = at(j0 + 16 * (i >> 2) + 4 * kg + (i & 3));
+    };
+    uint4 kv[2][8];
+    auto load_k = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const uint4 *p = reinterpret_cast<const uint4 *>(kbase + (size_t)ki[t] * QA_D);
+#pragma unroll
+            for (int s = 0; s < 8; s++) kv[t][s] = p[4 * s];
+        }
+    };
+    int j0 = j_lo + QAM_STEP * wave;
+    if (j0 < j_hi) {
+        entries(j0);
+        load_k();
+    }
+    for (; j0 < j_hi; j0 += 4 * QAM_STEP) {
+        // Half of the values' dims are requested ahead of the scores, half
+        // after them (in the keys' registers), the next pass's keys ahead of
+        // the second half's product.
+        uint4 v0[8], v1[8];
+        const uint16_t *vp[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) vp[i] = vbase + (size_t)vi[i] * QA_D;
+        entries(j0 + 4 * QAM_STEP);                            // the next pass's, ahead of this one's values
+#pragma unroll
+        for (int i = 0; i < 8; i++) v0[i] = *reinterpret_cast<const uint4 *>(vp[i]);
+        // scores: the first parts in one sum, the others in another
+        qa_f4 hi[2], lo[2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) hi[t] = lo[t] = qa_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            qa_h8 b[3];
+#pragma unroll
+            for (int p = 0; p < 3; p++) b[p] = *reinterpret_cast<const qa_h8 *>(&qp[p][ln][32 * s + 8 * kg]);
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const qa_h8 a = __builtin_bit_cast(qa_h8, kv[t][s]);
+                hi[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[0], hi[t], 0, 0, 0);
+                lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[2], lo[t], 0, 0, 0);
+                lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[1], lo[t], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; i++) v1[i] = *reinterpret_cast<const uint4 *>(vp[i] + 128);
+        float sc[8], cm = -FLT_MAX;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int j = j0 + 16 * (i >> 2) + 4 * kg + (i & 3);
+            sc[i] = j < j_hi ? (hi[i >> 2][i & 3] + lo[i >> 2][i & 3]) * fac : -FLT_MAX;
+            cm = fmaxf(cm, sc[i]);
+        }
+        cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
+        cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
+        const bool up = cm > m + QAM_SLACK;                    // (at first m + 8 is -FLT_MAX itself)
+        if (__ballot(up)) {
+            const float mn = up ? cm : m, f = qa_exp2(m - mn);
+            m = mn;
+            l *= f;
+            float fr[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) fr[e] = __shfl(f, 4 * kg + e, 64);
+#pragma unroll
+            for (int t = 0; t < 16; t++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[t][e] *= fr[e];
+        }
+        qa_h8 pa[3];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float p = qa_exp2(sc[i] - m);
+            l += p;
+            _Float16 a, b, c;
+            qa_split(p * (float)(1 << QAM_P_EXP), a, b, c);
+            pa[0][i] = a;
+            pa[1][i] = b;
+            pa[2][i] = c;
+        }
+        auto values = [&](const uint4 (&vv)[8], int t0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                // column t of the lane's 8 positions x 8 dims
+                uint32_t c[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t x = reinterpret_cast<const uint32_t *>(&vv[2 * i])[t / 2];
+                    const uint32_t y = reinterpret_cast<const uint32_t *>(&vv[2 * i + 1])[t / 2];
+                    c[i] = __builtin_amdgcn_perm(y, x, t & 1 ? 0x07060302u : 0x05040100u);
+                }
+                const qa_h8 b = __builtin_bit_cast(qa_h8, make_uint4(c[0], c[1], c[2], c[3]));
+                qa_f4 &o = acc[t0 + t];
+                o = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[0], b, o, 0, 0, 0);
+                o = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[1], b, o, 0, 0, 0);
+                o = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[2], b, o, 0, 0, 0);
+            }
+        };
+        values(v0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        load_k();
+        __builtin_amdgcn_sched_barrier(0);
+        values(v1, 8);
+    }
+    // the waves' states meet
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (kg == 0) { wm[wave][ln] = m; wl[wave][ln] = l; }
+    __syncthreads();                                           // (q is no longer read)
+    float (*os)[QAM_HEADS][QAM_OST] = reinterpret_cast<float (*)[QAM_HEADS][QAM_OST]>(lds);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int g = 4 * kg + e;
+        const float M = fmaxf(fmaxf(wm[0][g], wm[1][g]), fmaxf(wm[2][g], wm[3][g]));
+        const float f = qa_exp2(wm[wave][g] - M);
+#pragma unroll
+        for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int t = 8 * hf + 4 * u;
+                *reinterpret_cast<float4 *>(&os[wave][g][128 * hf + 8 * ln + 4 * u]) =
+                    make_float4(acc[t][e] * f, acc[t + 1][e] * f, acc[t + 2][e] * f, acc[t + 3][e] * f);
+            }
+    }
+    __syncthreads();
+    float *pr = part ? part + (size_t)blockIdx.x * G * (QA_D + 2) : nullptr;
+    for (int i = tid; i < G * (QA_D / 4); i += 256) {
+        const int g = i / (QA_D / 4), d = 4 * (i % (QA_D / 4));
+        const float M = fmaxf(fmaxf(wm[0][g], wm[1][g]), fmaxf(wm[2][g], wm[3][g]));
+        const float L = (wl[0][g] * qa_exp2(wm[0][g] - M) + wl[1][g] * qa_exp2(wm[1][g] - M)) +
+                        (wl[2][g] * qa_exp2(wm[2][g] - M) + wl[3][g] * qa_exp2(wm[3][g] - M));
+        const float4 a = *reinterpret_cast<const float4 *>(&os[0][g][d]), b = *reinterpret_cast<const float4 *>(&os[1][g][d]);
+        const float4 c = *reinterpret_cast<const float4 *>(&os[2][g][d]), e = *reinterpret_cast<const float4 *>(&os[3][g][d]);
+        constexpr float dn = 1.0f / (float)(1 << QAM_P_EXP);
+        float o[4] = {((a.x + b.x) + (c.x + e.x)) * dn, ((a.y + b.y) + (c.y + e.y)) * dn,
+                      ((a.z + b.z) + (c.z + e.z)) * dn, ((a.w + b.w) + (c.w + e.w)) * dn};
+        if (nsplit == 1) {
+            const size_t ob = ((size_t)row * q_heads + (size_t)kvh * G + g) * QA_D + d;
+            float4 gv = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (gate) gv = *reinterpret_cast<const float4 *>(gate + ob);
+            const float gg[4] = {gv.x, gv.y, gv.z, gv.w};
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                o[u] = L > 0.0f ? o[u] / L : 0.0f;
+                if (gate) o[u] *= 1.0f / (1.0f + expf(-gg[u]));
+                out[ob + u] = o[u];
+            }
+        } else {
+            if (d == 0) { pr[g] = M; pr[G + g] = L; }
+#pragma unroll
+            for (int u = 0; u < 4; u++) pr[2 * G + g * QA_D + d + u] = o[u];
+        }
+    }
+}
+
 // The splits of one (row, kv head, head), combined in split order: their
 // maxima and sums go to LDS first, then thread t adds dim t of every split's
 // output with all its loads in flight at once.
@@ -870,8 +1164,6 @@ __global__ void __launch_bounds__(256) k_attn_merge(float *__restrict__ out, con
 
 // ---- launchers ----------------------------------------------------------------------
 
-#define QS_MX_MIN_ROWS 16                  // rows from which the scores take the matrix cores
-
 static bool qs_shape_ok(int d, int rotary_dim) { return rotary_dim == QS_ROTARY && d >= 64 && d % 32 == 0 && d <= 256; }
 
 template <bool POOLED>
@@ -883,14 +1175,26 @@ static int qs_launch_scores(hipStream_t s, float *scores, const float *qn, const
     if (blocks == 0) return 0;
     const dim3 grid((blocks + QS_BLK - 1) / QS_BLK, (rows + QS_ROWS - 1) / QS_ROWS);
     const int D = d <= 64 ? 64 : d <= 128 ? 128 : d <= 192 ? 192 : 256;
-    if (rows >= QS_MX_MIN_ROWS && nq <= 16 && D <= 128) {
-        const dim3 gm((blocks + QS_BLK - 1) / QS_BLK, (rows + QM_ROWS - 1) / QM_ROWS);
-        if (D == 64)
-            hipLaunchKernelGGL((k_qsa_scores_mx<64, POOLED>), gm, dim3(QS_THREADS), 0, s, scores, qn, src, kw, inv_freq,
-                               rows, nq, d, ratio, base_pos, max_blocks, eps);
-        else
-            hipLaunchKernelGGL((k_qsa_scores_mx<128, POOLED>), gm, dim3(QS_THREADS), 0, s, scores, qn, src, kw, inv_freq,
-                               rows, nq, d, ratio, base_pos, max_blocks, eps);
+    if (nq <= 16 && D <= 128) {
+        // one row of stored keys: a wave a workgroup, so that 8192 blocks are
+        // 512 workgroups; from 64 rows on two tiles a wave share a row's heads
+        const unsigned gy = (unsigned)((rows + QM_ROWS - 1) / QM_ROWS);
+#define QS_MX(DD, TB, NW, ONE)                                                                                         \
+    hipLaunchKernelGGL((k_qsa_scores_mx<DD, POOLED, TB, NW, ONE>), dim3((blocks + 16 * TB * NW - 1) / (16 * TB * NW), gy), \
+                       dim3(64 * NW), 0, s, scores, qn, src, kw, inv_freq, rows, nq, d, ratio, base_pos, max_blocks, eps)
+#define QS_MXD(DD)                                                                                                     \
+    if constexpr (POOLED) {                                                                                            \
+        if (rows == 1) QS_MX(DD, 1, 1, true);                                                                          \
+        else if (rows < 64) QS_MX(DD, 1, 4, false);                                                                    \
+        else QS_MX(DD, 2, 4, false);                                                                                   \
+    } else {                                                                                                           \
+        if (rows == 1) QS_MX(DD, 1, 4, true);                                                                          \
+        else QS_MX(DD, 1, 4, false);                                                                                   \
+    }
+        if (D == 64) { QS_MXD(64) }
+        else { QS_MXD(128) }
+#undef QS_MXD
+#undef QS_MX
         return (int)hipGetLastError();
     }
     const size_t lds = ((size_t)QS_BLK * (D + 4) + 4 * QS_BLK + (size_t)nq * D) * sizeof(float);
@@ -988,15 +1292,33 @@ extern "C" size_t qwk_attn_masked_work_bytes(int rows, int q_heads, int kv_heads
 }
 
 template <int G>
+static void qa_merge(hipStream_t s, float *out, const float *gate, const float *part, int rows, int q_heads,
+                     int kv_heads, int ns)
+{
+    hipLaunchKernelGGL(k_attn_merge<G>, dim3(rows * kv_heads * G), dim3(256), 0, s, out, gate, part, q_heads,
+                       kv_heads, ns);
+}
+
+template <int G>
 static void qa_launch(hipStream_t s, float *out, const float *gate, const float *q, const uint16_t *kc,
                       const uint16_t *vc, const uint32_t *list, int rows, int q_heads, int kv_heads, int max_ctx,
                       float scale, int cap, int ns, float *part)
 {
+    // the matrix cores from 8 heads a kv head on, where a split gives every
+    // wave of a workgroup a pass of 32 positions (a decode step's splits are
+    // one pass long: three waves would idle)
+    const int per = ((cap + QA_P - 1) / QA_P + ns - 1) / ns;
+    if constexpr (G >= 8) {
+        if (per * QA_P >= 4 * QAM_STEP) {
+            hipLaunchKernelGGL(k_attn_mx<G>, dim3(rows * kv_heads * ns), dim3(256), 0, s, out, gate, q, kc, vc, list,
+                               q_heads, kv_heads, max_ctx, scale, cap, ns, part);
+            if (ns > 1) qa_merge<G>(s, out, gate, part, rows, q_heads, kv_heads, ns);
+            return;
+        }
+    }
     hipLaunchKernelGGL(k_attn_masked<G>, dim3(rows * kv_heads * ns), dim3(256), 0, s, out, gate, q, kc, vc, list,
                        q_heads, kv_heads, max_ctx, scale, cap, ns, part);
-    if (ns > 1)
-        hipLaunchKernelGGL(k_attn_merge<G>, dim3(rows * kv_heads * G), dim3(256), 0, s, out, gate, part, q_heads,
-                           kv_heads, ns);
+    if (ns > 1) qa_merge<G>(s, out, gate, part, rows, q_heads, kv_heads, ns);
 }
 
 extern "C" int qwk_attn_masked(hipStream_t s, float *out, const float *gate, const float *q, const uint16_t *kc,

@@ -543,3 +543,79 @@ def test_gated_delta_prep_chunks(gpu, hk, hv, rows):
     wy, ws, _ = sparse.gated_delta_prep(q, k, v, a, b, Al, dt, eps, qs, ks, s0, hk, hv, dk, dv, rows)
     for yb, sb in ((y1, s1), (y2, s2)):
         assert rel_l2(yb.read(np.float32, v.shape), wy) < 5e-6 and rel_l2(sb.read(np.float32, s0.shape), ws) < 5e-6
+
+
+# ---- masked attention on the matrix cores (8 query heads a kv head on) ---------------------
+
+@pytest.mark.parametrize("rows,qh,kvh,base,topk", [
+    (130, 24, 2, 200, 64),       # one split a row: lists of 201 to 260 positions, a ragged last pass
+    (129, 16, 2, 5, 64),         # lists of 6 to 134: under a wave's 32, one, a few waves idle
+    (260, 16, 1, 700, 32),       # 16 heads a kv head
+    (40, 24, 2, 3000, 512),      # splits of several passes, merged
+    (256, 8, 1, 0, 512),         # from position 0: a list of one
+])
+def test_attn_masked_matrix_cores(gpu, rows, qh, kvh, base, topk):
+    attn_case(gpu, rows, qh, kvh, base, topk, 4, 300 + rows + qh, gated=True)
+
+
+def test_attn_masked_matrix_cores_ranges(gpu):
+    """Heads of 1e4 and 1e-4 beside each other, a zero head, scores that climb
+    through the list (the running maximum moves many times) and one row whose
+    weight is all on its last position.  Bar: the weights are exponentials of
+    fp32 scores s, so an error of 2^-23 |s| in s (up to 60 here) is 7e-6 of a
+    weight: 2e-5 of the O(1) values."""
+    D, qh, kvh, rows, n = 256, 24, 2, 140, 300
+    q = rnd((rows, qh, D), 401)
+    kc = rnd((kvh, n, D), 402)
+    kc[:, :, 0] = np.linspace(-1, 1, n)[None, :]
+    q[:, :, 0] = 200.0
+    q[1, 3] *= 1e-4
+    q[1, 5] *= 0.25
+    q[2, 7] = 0.0
+    q[3] *= -1.0
+    kc[:, n - 1, 1] = 8.0
+    q[4, :, 1] = 120.0
+    kb16, vb16 = sparse.f16_bits(kc.astype(np.float32)), sparse.f16_bits(rnd((kvh, n, D), 403))
+    lst = np.zeros((rows, 1 + n), np.uint32)
+    lst[:, 0] = n
+    lst[:, 1:] = np.arange(n)
+    lst[5, 0] = 0                                  # nothing listed: zeros
+    B = gpu.Buf
+    topk, ratio = n // 4 - 1, 4
+    assert gpu.qw_qsa_list_cap(topk, ratio) == n
+    qb, kb, vb, lb, ob = B.of(q), B.of(kb16), B.of(vb16), B.of(lst), B(rows * qh * D * 4)
+    c = gpu.qw_cmd_begin()
+    gpu.qw_op_attn_masked(c, ob.ref(), qb.ref(), kb.ref(), vb.ref(), lb.ref(), rows, qh, kvh, D, n, n - rows,
+                          1.0 / 16.0, topk, ratio)
+    gpu.run(c, "attn masked")
+    got = ob.read(np.float32, (rows, qh, D))
+    k64 = np.asarray(kb16).view(np.float16).astype(np.float64).reshape(kvh, n, D)
+    v64 = np.asarray(vb16).view(np.float16).astype(np.float64).reshape(kvh, n, D)
+    G = qh // kvh
+    for r in range(rows):
+        for h in range(qh):
+            if r == 5:
+                assert (got[r, h] == 0).all()
+                continue
+            s = k64[h // G] @ q[r, h].astype(np.float64) / 16.0
+            w = np.exp(s - s.max())
+            want = (w / w.sum()) @ v64[h // G]
+            assert np.abs(got[r, h] - want).max() < 2e-5, (r, h, np.abs(got[r, h] - want).max())
+
+
+@pytest.mark.parametrize("nq,d,base,rows", [(16, 128, 900, 75), (7, 96, 3, 130)])
+def test_qsa_scores_many_rows_match_rowwise(gpu, nq, d, base, rows):
+    """From 64 rows on a wave scores two tiles of 16 blocks: the bits of one
+    row at a time (a wave a tile), at the first, a middle and the last rows;
+    blocks that end inside a tile, fewer heads than a tile's rows."""
+    ratio = 4
+    mb = (base + rows) // ratio + 3
+    kw = FX["k_norm"] if d == 128 else synth.to_bf16(1.0 + 0.1 * rnd(d, d + nq))
+    qn, ik, inv = rnd((rows, nq, d), 71 + d), rnd((mb * ratio, d), 72 + d), rope_inv()
+    for pooled in (False, True):
+        got, _ = gpu_scores(gpu, qn, ik, kw, inv, rows, nq, d, ratio, base, mb, pooled=pooled)
+        for r in (0, 1, 31, 32, 63, 64, rows - 1):
+            one, _ = gpu_scores(gpu, qn[r:r + 1], ik, kw, inv, 1, nq, d, ratio, base + r, mb, pooled=pooled)
+            nb = (base + r + 1) // ratio
+            assert same_bits(got[r, :nb], one[0, :nb]), f"row {r}"
+            assert np.isnan(got[r, nb:]).all()
