@@ -181,120 +181,187 @@ __global__ __launch_bounds__(64) void k_dmat_tiled(float *__restrict__ y, const 
 // v_mfma_f32_16x16x1f32, is four independent 16x16 outer products
 // D_b = C_b + a_b b_b^T, each element one fused multiply-add -- fmaf(a, b, c)
 // -- so a chunk's chain (from 0, k in index order) is 64 MFMAs on one
-// accumulator.  A workgroup owns 64 rows x 64 outputs; wave w owns rows
-// 16 w .. 16 w + 15 against all 64 outputs as the instruction's four blocks
-// (block b: outputs 16 b ..): lane l feeds block l / 16 with x[row l % 16][k]
-// and w[output l % 16][k].  The operands pass through LDS QW_DM_NC chunks at a
-// time (coalesced loads, the next stage requested while this one runs); a
-// wave runs the stage's chunk chains interleaved -- independent, so the
-// matrix pipe always has one ready -- and adds their partials to its running
-// total in chunk order (total = p_0, then total + p_c: the order above).
-// k % 64 == 0.
+// accumulator; chunk partials are added in chunk order (total = p_0, then
+// total + p_c: the order above).  k % 64 == 0.
+//
+// A workgroup owns RT tiles of 16 rows against 64 outputs, the instruction's
+// four blocks.  Wave w runs row tile w / NC and chunk NC s + w % NC of stage s
+// (NC = 4 / RT chunks a stage); a stage's partials meet in LDS and each wave
+// adds those of RT of its row tile's four output blocks to its totals.
+//
+// Bound by the chain: the instruction takes 38 cycles and a wave a SIMD has
+// only itself to hide what stands between two of them.  So
+//  - x (fp32) and w (bf16) go from memory straight to LDS, three stages in
+//    flight; piece p (16 bytes) of row r lies at p ^ (r % 8), which keeps the
+//    reads of 8 rows in different banks (the swizzle is in the address that a
+//    lane loads from);
+//  - the next stage's operands go to registers while this one's chain runs
+//    (LDS reads ahead of the chain waited for all of them at its start: 101 us
+//    against 89 at 2048 rows of the shape below);
+//  - lane group b holds the x of pieces 4 q + b and the MFMA hands it to all
+//    four blocks (cbsz 2, abid b): a quarter of the reads and registers;
+//  - weights are widened eight at a time before eight MFMAs run back to back
+//    (a conversion between every two of them: 69 cycles an MFMA, now 57).
+// k 3072, 512 outputs, 32-512 / 1024 / 2048 / 4096 rows: 25 / 44 / 75 / 127 us;
+// 64 rows a workgroup through registers, the form before, 76 / 76 / 76 / 129.
 typedef float qr_f16v __attribute__((ext_vector_type(16)));
 #define QW_DM_T 64
-#define QW_DM_NC 2                                 // chunks a stage (4 measured slower)
-#define QW_DM_KS (64 * QW_DM_NC + 4)               // floats a row of a stage (+ pad)
-__global__ __launch_bounds__(256) void k_dmat_mfma(float *__restrict__ y, const float *__restrict__ x,
-                                                   const uint16_t *__restrict__ w, int k, int n, int rows)
+__device__ __forceinline__ void qd_dma(uint32_t lds, const void *src)
 {
-    extern __shared__ float4 dm_lds[];
-    float *xs = reinterpret_cast<float *>(dm_lds), *ws = xs + QW_DM_T * QW_DM_KS;
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, blk = lane >> 4, i = lane & 15;
-    // Workgroup b runs on XCD b % 8: each XCD takes a contiguous range of
-    // tiles in (row tile, column tile) order, so the column tiles of one row
-    // tile share its token rows in that XCD's L2
-    const int nct = (n + QW_DM_T - 1) / QW_DM_T, ntt = nct * ((rows + QW_DM_T - 1) / QW_DM_T);
-    const int lt = (blockIdx.x & 7) * ((ntt + 7) / 8) + (blockIdx.x >> 3);
+    // (asm: the compiler would wait for every such load before any LDS read;
+    // the kernel's own waits follow)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+template <int RT>
+__global__ __launch_bounds__(256, 1) void k_dmat_mfma(float *__restrict__ y, const float *__restrict__ x,
+                                                     const uint16_t *__restrict__ w, int k, int n, int rows)
+{
+    constexpr int NC = 4 / RT, SK = 64 * NC, R = 16 * RT, NST = 3;
+    constexpr int XP = SK / 4, WP = SK / 8;                       // pieces a row of x, of w
+    constexpr int XSZ = R * SK * 4, WSZ = QW_DM_T * SK * 2, STG = XSZ + WSZ;
+    constexpr int XI = XSZ / 4096, WI = WSZ / 4096;               // loads a wave a stage
+    static_assert(XSZ % 4096 == 0 && WSZ % 4096 == 0 && (XI + WI) * 2 < 64, "whole loads, the wait's counter");
+    __shared__ __align__(16) uint8_t ring[NST * STG];
+    __shared__ float4 ps[NC > 1 ? 4 : 1][4][64];                  // [wave][output block][lane]: a stage's partials
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, blk = lane >> 4, i = lane & 15;
+    const int rt = wave / NC, ch = wave % NC;
+    const int nct = (n + QW_DM_T - 1) / QW_DM_T, ntt = nct * ((rows + R - 1) / R);
+    const int lt = (blockIdx.x & 7) * ((ntt + 7) / 8) + (blockIdx.x >> 3);   // (an XCD's tiles are contiguous)
     if (lt >= ntt) return;
-    const int r0 = lt / nct * QW_DM_T, o0 = lt % nct * QW_DM_T;
-    const int nch = k / 64, rounds = (nch + QW_DM_NC - 1) / QW_DM_NC;
-    constexpr int SK = 64 * QW_DM_NC;                    // k a stage
-    constexpr int XF4 = QW_DM_T * SK / 4 / 256, WU4 = QW_DM_T * SK / 8 / 256;
-    // staging: x [64 rows][SK] as float4s, w [64 outputs][SK] bf16 as uint4s,
-    // consecutive threads along a row
-    float4 xr[XF4];
-    uint4 wr[WU4];
-    auto fetch = [&](int rd) {
-        const int k0 = SK * rd, kl = min(SK, k - k0);
+    const int r0 = lt / nct * R, o0 = lt % nct * QW_DM_T;
+    const int nch = k / 64, rounds = (nch + NC - 1) / NC;
+    const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)&ring[0];
+    const float *xrow[XI];
+    const uint16_t *wrow[WI];
+    int xpc[XI], wpc[WI];
 #pragma unroll
-        for (int j = 0; j < XF4; j++) {
-            const int q = t + 256 * j, row = q / (SK / 4), c4 = q % (SK / 4);
-            const int gr = min(r0 + row, rows - 1);
-            xr[j] = 4 * c4 < kl ? reinterpret_cast<const float4 *>(x + (size_t)gr * k + k0)[c4]
-                                : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (int j = 0; j < WU4; j++) {
-            const int q = t + 256 * j, o = q / (SK / 8), c8 = q % (SK / 8);
-            const int go = min(o0 + o, n - 1);
-            wr[j] = 8 * c8 < kl ? reinterpret_cast<const uint4 *>(w + (size_t)go * k + k0)[c8] : make_uint4(0, 0, 0, 0);
-        }
-    };
-    auto stash = [&]() {
-#pragma unroll
-        for (int j = 0; j < XF4; j++) {
-            const int q = t + 256 * j, row = q / (SK / 4), c4 = q % (SK / 4);
-            *reinterpret_cast<float4 *>(xs + row * QW_DM_KS + 4 * c4) = xr[j];
-        }
-#pragma unroll
-        for (int j = 0; j < WU4; j++) {
-            const int q = t + 256 * j, o = q / (SK / 8), c8 = q % (SK / 8);
-            const uint32_t v[4] = {wr[j].x, wr[j].y, wr[j].z, wr[j].w};
-            float f[8];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                f[2 * e] = __uint_as_float(v[e] << 16);
-                f[2 * e + 1] = __uint_as_float(v[e] & 0xFFFF0000u);
-            }
-            float4 *d = reinterpret_cast<float4 *>(ws + o * QW_DM_KS + 8 * c8);
-            d[0] = make_float4(f[0], f[1], f[2], f[3]);
-            d[1] = make_float4(f[4], f[5], f[6], f[7]);
-        }
-    };
-    const qr_f16v zero = {};
-    qr_f16v tot = zero;
-    fetch(0);
-    const float *xa = xs + (16 * wave + i) * QW_DM_KS, *wa = ws + (16 * blk + i) * QW_DM_KS;
-    for (int rd = 0; rd < rounds; rd++) {
-        __syncthreads();                            // the previous stage is consumed
-        stash();
-        __syncthreads();
-        if (rd + 1 < rounds) fetch(rd + 1);
-        const int nc = min(QW_DM_NC, nch - QW_DM_NC * rd);
-        qr_f16v acc[QW_DM_NC];
-#pragma unroll
-        for (int c = 0; c < QW_DM_NC; c++) acc[c] = zero;
-#pragma unroll 2
-        for (int kk = 0; kk < 64; kk += 4) {
-            float4 av[QW_DM_NC], bv[QW_DM_NC];
-#pragma unroll
-            for (int c = 0; c < QW_DM_NC; c++) {
-                av[c] = *reinterpret_cast<const float4 *>(xa + 64 * c + kk);
-                bv[c] = *reinterpret_cast<const float4 *>(wa + 64 * c + kk);
-            }
-#pragma unroll
-            for (int c = 0; c < QW_DM_NC; c++) acc[c] = __builtin_amdgcn_mfma_f32_16x16x1f32(av[c].x, bv[c].x, acc[c], 0, 0, 0);
-#pragma unroll
-            for (int c = 0; c < QW_DM_NC; c++) acc[c] = __builtin_amdgcn_mfma_f32_16x16x1f32(av[c].y, bv[c].y, acc[c], 0, 0, 0);
-#pragma unroll
-            for (int c = 0; c < QW_DM_NC; c++) acc[c] = __builtin_amdgcn_mfma_f32_16x16x1f32(av[c].z, bv[c].z, acc[c], 0, 0, 0);
-#pragma unroll
-            for (int c = 0; c < QW_DM_NC; c++) acc[c] = __builtin_amdgcn_mfma_f32_16x16x1f32(av[c].w, bv[c].w, acc[c], 0, 0, 0);
-        }
-#pragma unroll
-        for (int c = 0; c < QW_DM_NC; c++)
-            if (c < nc) {
-#pragma unroll
-                for (int e = 0; e < 16; e++) tot[e] = rd == 0 && c == 0 ? acc[c][e] : tot[e] + acc[c][e];
-            }
+    for (int j = 0; j < XI; j++) {
+        const int slot = (wave * XI + j) * 64 + lane, r = slot / XP;
+        xrow[j] = x + (size_t)min(r0 + r, rows - 1) * k;
+        xpc[j] = slot % XP ^ (r & 7);
     }
-    // block b's values of this lane: rows 4 (lane / 16) + e of the wave's 16,
-    // output 16 b + lane % 16
 #pragma unroll
-    for (int e = 0; e < 16; e++) {
-        const int b = e >> 2;
-        const int row = r0 + 16 * wave + 4 * (lane >> 4) + (e & 3), o = o0 + 16 * b + (lane & 15);
-        if (row < rows && o < n) y[(size_t)row * n + o] = tot[e];
+    for (int j = 0; j < WI; j++) {
+        const int slot = (wave * WI + j) * 64 + lane, o = slot / WP;
+        wrow[j] = w + (size_t)min(o0 + o, n - 1) * k;
+        wpc[j] = slot % WP ^ (o & 7);
+    }
+    auto issue = [&](int s) {      // (past the row's end a piece of its start: no wave's chunk)
+        const uint32_t st = ring0 + (uint32_t)(s % NST) * STG;
+#pragma unroll
+        for (int j = 0; j < XI; j++) {
+            const int p = s * XP + xpc[j];
+            qd_dma(st + (wave * XI + j) * 1024, xrow[j] + 4 * (p < k / 4 ? p : 0));
+        }
+#pragma unroll
+        for (int j = 0; j < WI; j++) {
+            const int p = s * WP + wpc[j];
+            qd_dma(st + XSZ + (wave * WI + j) * 1024, wrow[j] + 8 * (p < k / 8 ? p : 0));
+        }
+    };
+    float tot[RT][4];
+    auto meet = [&](int s) {       // stage s's partials, in chunk order
+        const int nc = min(NC, nch - NC * s);
+#pragma unroll
+        for (int u = 0; u < RT; u++) {
+            float4 p[NC];
+#pragma unroll
+            for (int c = 0; c < NC; c++) p[c] = ps[NC > 1 ? rt * NC + c : 0][ch * RT + u][lane];
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+                if (c < nc) {
+                    const float v[4] = {p[c].x, p[c].y, p[c].z, p[c].w};
+#pragma unroll
+                    for (int e = 0; e < 4; e++) tot[u][e] = s == 0 && c == 0 ? v[e] : tot[u][e] + v[e];
+                }
+        }
+    };
+    const int xr = 16 * rt + i, wr = 16 * blk + i;
+    float4 a[2][4];      // x: lane group blk holds the k of pieces 4 q + blk, which the MFMA hands to all four
+    uint4 b[2][8];       // w: piece j
+    auto takea = [&](int s, int q) {
+        return *reinterpret_cast<const float4 *>(ring + (s % NST) * STG + xr * (SK * 4) + (((16 * ch + 4 * q + blk) ^ (xr & 7)) * 16));
+    };
+    auto takeb = [&](int s, int j) {
+        return *reinterpret_cast<const uint4 *>(ring + (s % NST) * STG + XSZ + wr * (SK * 2) + (((8 * ch + j) ^ (wr & 7)) * 16));
+    };
+    auto widen = [](uint4 q, float *v) {
+        const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            v[2 * e] = __uint_as_float(u[e] << 16);
+            v[2 * e + 1] = __uint_as_float(u[e] & 0xFFFF0000u);
+        }
+    };
+    auto stage = [&](int s, const float4 *ra, const uint4 *rb, float4 *na, uint4 *nb) {
+        // stage s + 1 is in LDS (the one after it stays in flight) and the last stage's partials are written
+        __builtin_amdgcn_s_waitcnt(0xC07F);              // lgkmcnt(0) where the compiler sees it: it adds no waits below
+        if (s + 2 < rounds) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(XI + WI) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + 3 < rounds) issue(s + 3);
+        if (NC > 1 && s > 0) meet(s - 1);
+        const int sn = min(s + 1, rounds - 1);           // (the last stage reads itself again)
+        qr_f16v acc = {};
+#define QD_K8(j, b0)                                                                                                    \
+{                                                                                                                       \
+    const float4 av = ra[(j) / 2];                                                                                      \
+    float wn[8];                                                                                                        \
+    if ((j) < 7) widen(rb[((j) + 1) & 7], wn);                                                                          \
+    nb[j] = takeb(sn, j);                                                                                               \
+    if ((j) % 2 == 0) na[(j) / 2] = takea(sn, (j) / 2);                                                                 \
+    __builtin_amdgcn_sched_barrier(0);                                                                                  \
+    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(av.x, wv[0], acc, 2, b0, 0);                                             \
+    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(av.y, wv[1], acc, 2, b0, 0);                                             \
+    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(av.z, wv[2], acc, 2, b0, 0);                                             \
+    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(av.w, wv[3], acc, 2, b0, 0);                                             \
+    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(av.x, wv[4], acc, 2, b0 + 1, 0);                                         \
+    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(av.y, wv[5], acc, 2, b0 + 1, 0);                                         \
+    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(av.z, wv[6], acc, 2, b0 + 1, 0);                                         \
+    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(av.w, wv[7], acc, 2, b0 + 1, 0);                                         \
+    __builtin_amdgcn_sched_barrier(0);                                                                                  \
+    if ((j) < 7) for (int e = 0; e < 8; e++) wv[e] = wn[e];                                                             \
+}
+        float wv[8];
+        widen(rb[0], wv);
+        QD_K8(0, 0) QD_K8(1, 2) QD_K8(2, 0) QD_K8(3, 2) QD_K8(4, 0) QD_K8(5, 2) QD_K8(6, 0) QD_K8(7, 2)
+#undef QD_K8
+        if constexpr (NC > 1) {
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (NC * s + ch < nch) {
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    ps[wave][c][lane] = make_float4(acc[4 * c], acc[4 * c + 1], acc[4 * c + 2], acc[4 * c + 3]);
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) tot[c][e] = s == 0 ? acc[4 * c + e] : tot[c][e] + acc[4 * c + e];
+        }
+    };
+    for (int s = 0; s < min(3, rounds); s++) issue(s);
+    if (rounds > 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * (XI + WI)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < 8; j++) b[0][j] = takeb(0, j);
+#pragma unroll
+    for (int q = 0; q < 4; q++) a[0][q] = takea(0, q);
+    for (int s = 0; s < rounds; s += 2) {
+        stage(s, a[0], b[0], a[1], b[1]);
+        if (s + 1 < rounds) stage(s + 1, a[1], b[1], a[0], b[0]);
+    }
+    if constexpr (NC > 1) {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        meet(rounds - 1);
+    }
+#pragma unroll
+    for (int u = 0; u < RT; u++) {
+        const int o = o0 + 16 * (ch * RT + u) + i;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int row = r0 + 16 * rt + 4 * blk + e;
+            if (row < rows && o < n) y[(size_t)row * n + o] = tot[u][e];
+        }
     }
 }
 
@@ -502,16 +569,17 @@ extern "C" int qwk_dmat_bf16(hipStream_t s, float *y, const float *x, const uint
     }
     if (vec && n >= 8 && qw_few_ok(x, w, k, rows)) return qw_launch_few(s, y, nullptr, x, w, nullptr, k, n, rows);
     if (vec && k % 64 == 0 && rows >= QW_DT && n >= QW_DM_T) {
-        const int lds = 2 * QW_DM_T * QW_DM_KS * (int)sizeof(float);
-        static bool attr = false;
-        if (!attr) {
-            attr = true;
-            (void)hipFuncSetAttribute((const void *)k_dmat_mfma, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-            (void)hipGetLastError();
-        }
-        const int ntt = ((n + QW_DM_T - 1) / QW_DM_T) * ((rows + QW_DM_T - 1) / QW_DM_T);
-        hipLaunchKernelGGL(k_dmat_mfma, dim3((ntt + 7) / 8 * 8), dim3(256), lds,
-                           s, y, x, w, k, n, rows);
+        // The fewest rows a workgroup that leave no more workgroups than the
+        // chip has CUs (one each: LDS).  n 512, k 3072, us at 16 / 32 / 64
+        // rows a workgroup: 512 rows 25 / 42 / 73, 768 rows 47 / 43 / 73,
+        // 1536 rows 71 / 82 / 73, 2048 rows 93 / 84 / 75, 4096 rows 181 / 164 / 127.
+        const int ct = (n + QW_DM_T - 1) / QW_DM_T;
+        auto tiles = [&](int r) { return ct * ((rows + r - 1) / r); };
+        const int rt = tiles(16) <= 256 ? 1 : tiles(32) <= 256 ? 2 : 4;
+        const dim3 grid((tiles(16 * rt) + 7) / 8 * 8);
+        if (rt == 1) hipLaunchKernelGGL(k_dmat_mfma<1>, grid, dim3(256), 0, s, y, x, w, k, n, rows);
+        else if (rt == 2) hipLaunchKernelGGL(k_dmat_mfma<2>, grid, dim3(256), 0, s, y, x, w, k, n, rows);
+        else hipLaunchKernelGGL(k_dmat_mfma<4>, grid, dim3(256), 0, s, y, x, w, k, n, rows);
         return (int)hipGetLastError();
     }
     if (vec && k % 64 == 0 && rows >= QW_DT) {

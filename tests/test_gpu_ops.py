@@ -142,6 +142,24 @@ def test_dmat_bf16_order_r_bit_exact(gpu, k, n, rows):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), "router logits not bit-exact (order R)"
 
 
+@pytest.mark.parametrize("k,n,rows", [(64, 64, 32), (192, 65, 49), (320, 512, 512), (192, 512, 545), (64, 512, 1024),
+                                      (448, 130, 1500), (64, 515, 1025), (192, 512, 1090)])
+def test_dmat_bf16_row_tiles_bit_exact(gpu, k, n, rows):
+    """16, 32 and 64 rows a workgroup: chunks that leave the last stage partly
+    empty, one stage only, and ragged row and output tiles."""
+    w = synth.to_bf16(rnd((n, k), 15 + k, 0.02))
+    x = rnd((rows, k), 19 + n).astype(np.float32)
+    x[rows // 2] = 0.0
+    B = gpu.Buf
+    wb, xb, yb = B.of(w), B.of(x), B(rows * n * 4)
+    c = gpu.qw_cmd_begin()
+    gpu.qw_op_dmat_bf16(c, yb.ref(), xb.ref(), wb.ref(), k, n, rows)
+    gpu.run(c, "dmat")
+    want = ref.dmat_bf16(x, w, k, n, rows)
+    got = yb.read(np.float32, (rows, n))
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), "not bit-exact (order R)"
+
+
 # ---- decode banks ------------------------------------------------------------
 
 @pytest.mark.parametrize("G", [64, 32])
