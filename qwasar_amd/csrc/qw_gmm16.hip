@@ -211,9 +211,15 @@ __global__ __launch_bounds__(G16_THREADS, BM == 64 ? 1 : 2) void k_gmm16(Gmm16Ar
         nitems = 1;
     }
     const int tile = xcd * tpx + tl;
-    // NT weight tiles of 16 a wave: the item's BNT weight rows
-    auto body = [&](auto ntc) {
-    constexpr int NT = decltype(ntc)::value, NH = NT / 2, BNT = NT * 16 * (G16_THREADS / 64);
+    // NT weight tiles of 16 a wave: the item's BNT weight rows; MT row tiles
+    // of 16: those that hold rows of the tile.  An expert of a 2048-token
+    // chunk has about 40 rows, of a 512-token one about 10, and the empty row
+    // tiles' MFMAs and LDS reads stood beside the conversions on the same
+    // SIMDs (of the gate / up launch's cycles at 2048 tokens the matrix unit
+    // now runs 23%, the vector unit 45%): a layer of 512 tokens with skewed
+    // experts 288 -> 279 us, of 2048 1% at most (runs differ by as much).
+    auto body = [&](auto ntc, auto mtc) {
+    constexpr int NT = decltype(ntc)::value, NH = NT / 2, BNT = NT * 16 * (G16_THREADS / 64), MT = decltype(mtc)::value;
     int expert, first, len;
     if (DENSE) {
         first = tile * BM;
@@ -375,9 +381,9 @@ __global__ __launch_bounds__(G16_THREADS, BM == 64 ? 1 : 2) void k_gmm16(Gmm16Ar
     // barrier that publishes a block leaves them in flight)
     constexpr int NBL = NT * (WPL == 2 ? 1 : WPL / 4);
 
-    g16_f4 acc[BM / 16][NT];
+    g16_f4 acc[MT][NT];
 #pragma unroll
-    for (int mt = 0; mt < BM / 16; mt++)
+    for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) acc[mt][nt] = g16_f4{0.f, 0.f, 0.f, 0.f};
     uint32_t lo = 0x64006400u, hi = 0x54005400u;
@@ -409,10 +415,10 @@ __global__ __launch_bounds__(G16_THREADS, BM == 64 ? 1 : 2) void k_gmm16(Gmm16Ar
         __builtin_amdgcn_sched_barrier(0);
         if (bstart) fetch_sb(beta + 1, (beta + 1) & 1);
         __builtin_amdgcn_sched_barrier(0);
-        auto lda = [&](int st, g16_h8 (&o)[BM / 16]) {
+        auto lda = [&](int st, g16_h8 (&o)[MT]) {
             const int ah = kg * KPL + 8 * st;
 #pragma unroll
-            for (int mt = 0; mt < BM / 16; mt++) o[mt] = *reinterpret_cast<const g16_h8 *>(&As[q][mt * 16 + ln][ah]);
+            for (int mt = 0; mt < MT; mt++) o[mt] = *reinterpret_cast<const g16_h8 *>(&As[q][mt * 16 + ln][ah]);
         };
         auto dqs = [&](int st, g16_h8 (&o)[NT]) {
             const int g = NGL == 1 ? 0 : st * 8 / G;
@@ -423,7 +429,7 @@ __global__ __launch_bounds__(G16_THREADS, BM == 64 ? 1 : 2) void k_gmm16(Gmm16Ar
                 o[nt] = __builtin_bit_cast(g16_h8, g16_u4{d[0], d[1], d[2], d[3]});
             }
         };
-        g16_h8 af[2][BM / 16], bf[2][NT];
+        g16_h8 af[2][MT], bf[2][NT];
         lda(0, af[0]);
         dqs(0, bf[0]);
 #pragma unroll
@@ -434,7 +440,7 @@ __global__ __launch_bounds__(G16_THREADS, BM == 64 ? 1 : 2) void k_gmm16(Gmm16Ar
                 dqs(st + 1, bf[cu ^ 1]);
             }
 #pragma unroll
-            for (int mt = 0; mt < BM / 16; mt++)
+            for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                 for (int nt = 0; nt < NT; nt++)
                     acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[cu][mt], bf[cu][nt], acc[mt][nt], 0, 0, 0);
@@ -448,7 +454,7 @@ __global__ __launch_bounds__(G16_THREADS, BM == 64 ? 1 : 2) void k_gmm16(Gmm16Ar
         if (c == nch - 1) {
             // the item is done: out, y = F acc, with SWIGLU silu(F g) * (F u)
 #pragma unroll
-            for (int mt = 0; mt < BM / 16; mt++)
+            for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const int m = mt * 16 + 4 * kg + e;
@@ -523,8 +529,19 @@ __global__ __launch_bounds__(G16_THREADS, BM == 64 ? 1 : 2) void k_gmm16(Gmm16Ar
         }
     }
     };
-    if (half) body(std::integral_constant<int, 2>{});
-    else body(std::integral_constant<int, 4>{});
+    auto rows_of = [&](auto mtc) {
+        if (half) body(std::integral_constant<int, 2>{}, mtc);
+        else body(std::integral_constant<int, 4>{}, mtc);
+    };
+    if constexpr (BM == 64 && !DENSE && KC == 256) {
+        const int len = a.tiles[3 + 3 * tile], mt = rh == 0 ? min(len, 32) : len;
+        if (mt <= 16) rows_of(std::integral_constant<int, 1>{});
+        else if (mt <= 32) rows_of(std::integral_constant<int, 2>{});
+        else if (mt <= 48) rows_of(std::integral_constant<int, 3>{});
+        else rows_of(std::integral_constant<int, 4>{});
+    } else {
+        rows_of(std::integral_constant<int, BM / 16>{});
+    }
 }
 
 // ---- the batch decode's gate / up: one stream a wave ------------------------------

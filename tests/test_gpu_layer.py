@@ -207,6 +207,17 @@ def test_prefill_shared_expert_grouped(gpu, split):
     lb.free()
 
 
+@pytest.mark.parametrize("rows", [66, 128, 257, 380, 470])
+def test_prefill_row_tile_heights(gpu, rows):
+    """32 experts of 8, 16, 32, 47 and 59 rows on average: products over one,
+    two, three and four row tiles of 16, their last rows ragged."""
+    L = synth.make_layer(325, H=512, E=32, K=4, I=128, SI=128, group=64, split=True, tag="pfrt.")
+    x = synth.make_x(326 + rows, rows, L.H, name="pfrt.x")
+    lb = gpu.LayerBufs(L)
+    check(run_layer(gpu, lb, x), ref.moe_forward(L, x), 1e-3)
+    lb.free()
+
+
 @pytest.mark.parametrize("split", [True, False])
 @pytest.mark.parametrize("si", [128, 256])
 def test_decode_shared_slices_ahead(gpu, split, si):
