@@ -253,6 +253,14 @@ def test_attn_masked_split_merge(gpu, rows, qh, kvh, base):
         attn_case(gpu, rows, qh, kvh, base, 512, 4, 90 + qh + rows, gated=True)
 
 
+@pytest.mark.parametrize("rows,qh,kvh,base,topk", [(1, 4, 1, 40, 9), (1, 16, 2, 70, 17), (2, 8, 2, 130, 24),
+                                                   (1, 8, 1, 200, 40), (1, 2, 1, 5000, 1040)])
+def test_attn_masked_merge_split_counts(gpu, rows, qh, kvh, base, topk):
+    """Two, three, four to seven and 128 splits: quarters of the merge with no
+    split, one, and all 32."""
+    attn_case(gpu, rows, qh, kvh, base, topk, 4, 190 + qh + rows, gated=rows == 1)
+
+
 # ---- gated DeltaNet ----------------------------------------------------------------
 
 @pytest.mark.parametrize("channels,rows,n_snap", [(1024, 1, 1), (1024, 7, 7), (10240, 3, 3), (1024, 2, 2),
