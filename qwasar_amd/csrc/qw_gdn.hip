@@ -395,9 +395,12 @@ __global__ void __launch_bounds__(QG_THREADS) k_gated_delta(float *__restrict__ 
 // a workgroup 16 value rows of a head, every product on the fp32 matrix cores
 // (v_mfma_f32_16x16x4_f32: fp32 inputs and sums, as the serial form).
 // 2048 steps of 16 key and 48 value heads: 10 + 590 us serial (70 vector
-// operations a step on the CUs that hold two workgroups), 34 + 227 here; the
-// call with conv and output gate 682 -> 323.  Error against 64 bits over that
-// call: 1.5 to 1.6e-7 serial, 1.75e-7 here (y; the state 1.2e-7 either way).
+// operations a step on the CUs that hold two workgroups), 40 + 235 here; the
+// call with conv and output gate 686 -> 335.  Error against 64 bits over calls
+// of 600 and 2048 steps: y 1.50 to 1.51e-7 serial, 1.48 to 1.51e-7 here, the
+// state 1.19 to 1.33e-7 and 1.09 to 1.22e-7.  That takes short chains from zero
+// met in trees, and the norms' factors and the gates' products in 64 bits
+// (without: y 1.75e-7, 34 + 227 us).
 // What bounds it now: k_gdn_chunk's chain a chunk (56 MFMAs of 35 cycles a
 // wave and three hand-offs through LDS) on the CUs that hold two of the 384
 // workgroups, and its operands' bytes (K and Q read by 8 workgroups a head: a
@@ -450,6 +453,15 @@ __device__ __forceinline__ qg_f4 qg_mm16(float4 a, float4 b, qg_f4 d)
     return d;
 }
 
+// Lane t's double in every lane.
+__device__ __forceinline__ double qg_lane(double v, int t)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, t);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), t);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
 // Steps past the call's last are g = 1, beta = 0, q = k = 0: they leave the
 // state alone, and no output is written for them.  What k_gdn_chunk reads as
 // MFMA operands is stored in its lanes' order, so that its loads are whole
@@ -480,19 +492,24 @@ __global__ void __launch_bounds__(256) k_gdn_chunk_pre(qg_long w, const float *_
         }
         float fq = t < n ? 1.0f : 0.0f, fk = fq;
         if (PREP) {
-            // four chains of four and a tree: no longer a chain than the serial form's
-            float sq[4], sk[4];
+            // (a row's factor in 64 bits: its error is common to the row, where the sums' are not)
+            double aq = 0.0, ak = 0.0;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                sq[i] = vq[i].x * vq[i].x;                        sk[i] = vk[i].x * vk[i].x;
-                sq[i] = __builtin_fmaf(vq[i].y, vq[i].y, sq[i]);  sk[i] = __builtin_fmaf(vk[i].y, vk[i].y, sk[i]);
-                sq[i] = __builtin_fmaf(vq[i].z, vq[i].z, sq[i]);  sk[i] = __builtin_fmaf(vk[i].z, vk[i].z, sk[i]);
-                sq[i] = __builtin_fmaf(vq[i].w, vq[i].w, sq[i]);  sk[i] = __builtin_fmaf(vk[i].w, vk[i].w, sk[i]);
+                const float cq[4] = {vq[i].x, vq[i].y, vq[i].z, vq[i].w}, ck[4] = {vk[i].x, vk[i].y, vk[i].z, vk[i].w};
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+                    aq = __builtin_fma((double)cq[m], (double)cq[m], aq);
+                    ak = __builtin_fma((double)ck[m], (double)ck[m], ak);
+                }
             }
-            const float aq = qw_xor_sum<8>((sq[0] + sq[1]) + (sq[2] + sq[3]));
-            const float ak = qw_xor_sum<8>((sk[0] + sk[1]) + (sk[2] + sk[3]));
-            fq *= 1.0f / sqrtf(aq / (float)QG_DK + pp.l2eps) * pp.q_scale;
-            fk *= 1.0f / sqrtf(ak / (float)QG_DK + pp.l2eps) * pp.k_scale;
+#pragma unroll
+            for (int o = 1; o < 8; o <<= 1) {
+                aq += __shfl_xor(aq, o, 64);
+                ak += __shfl_xor(ak, o, 64);
+            }
+            fq *= (float)((double)pp.q_scale / sqrt(aq / QG_DK + (double)pp.l2eps));
+            fk *= (float)((double)pp.k_scale / sqrt(ak / QG_DK + (double)pp.l2eps));
         }
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -517,17 +534,14 @@ __global__ void __launch_bounds__(256) k_gdn_chunk_pre(qg_long w, const float *_
     for (int u = wave; u < 6; u += 4) {
         const int m = (u % 3) > 0 ? 16 : 0, i0 = (u % 3) > 1 ? 16 : 0;
         const float *A = u < 3 ? &Ks[m + ln][0] : &Qs[m + ln][0], *B = &Ks[i0 + ln][0];
-        qg_f4 d[4];
+        qg_f4 d[8];
 #pragma unroll
-        for (int i = 0; i < 4; i++) d[i] = qg_f4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < 8; i++)
+            d[i] = qg_mm16(*reinterpret_cast<const float4 *>(A + 16 * i + 4 * kg),
+                           *reinterpret_cast<const float4 *>(B + 16 * i + 4 * kg), qg_f4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-        for (int j = 0; j < QG_DK; j += 64)
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                d[i] = qg_mm16(*reinterpret_cast<const float4 *>(A + j + 16 * i + 4 * kg),
-                               *reinterpret_cast<const float4 *>(B + j + 16 * i + 4 * kg), d[i]);
-#pragma unroll
-        for (int e = 0; e < 4; e++) (u < 3 ? KK : QK)[m + 4 * kg + e][i0 + ln] = (d[0][e] + d[1][e]) + (d[2][e] + d[3][e]);
+        for (int e = 0; e < 4; e++) (u < 3 ? KK : QK)[m + 4 * kg + e][i0 + ln] = ((d[0][e] + d[1][e]) + (d[2][e] + d[3][e])) +
+                                                                                     ((d[4][e] + d[5][e]) + (d[6][e] + d[7][e]));
     }
     __syncthreads();                                              // q and k are consumed
     // a value head a wave: lane i has column i of P, L, the masked Q K' and T
@@ -535,25 +549,32 @@ __global__ void __launch_bounds__(256) k_gdn_chunk_pre(qg_long w, const float *_
     for (int r = wave; r < hv / hk; r += 4) {
         const int h = hx * (hv / hk) + r, i = lane & 31;
         const size_t hc = (size_t)h * nch + c;
-        float gi = 1.0f, bi = 0.0f;                               // step i's gate and beta
+        // step i's gate and beta; the gate and its running products in 64
+        // bits (a product of 32 factors is off by 32 of their errors)
+        double gi = 1.0;
+        float bi = 0.0f;
         if (i < n) {
             const size_t at = (size_t)(c * QG_C + i) * hv + h;
-            if (PREP) qg_gates(pp.a[at], pp.b[at], qw_bf16(pp.A_log[h]), qw_bf16(pp.dt_bias[h]), gi, bi);
-            else { gi = g[at]; bi = beta[at]; }
+            if (PREP) {
+                const double u = (double)pp.a[at] + (double)qw_bf16(pp.dt_bias[h]);
+                gi = exp(-exp((double)qw_bf16(pp.A_log[h])) * (u > 20.0 ? u : log1p(exp(u))));
+                bi = (float)(1.0 / (1.0 + exp(-(double)pp.b[at])));
+            } else { gi = (double)g[at]; bi = beta[at]; }
         }
-        float p = 0.0f, gam = 1.0f;
+        double p = 0.0, gam = 1.0;
 #pragma unroll 4
         for (int t = 0; t < QG_C; t++) {
-            const float gt = qw_lane(gi, t), bt = qw_lane(bi, t);
+            const double gt = qg_lane(gi, t);
+            const float bt = qw_lane(bi, t);
             if (t <= i) gam *= gt;
-            p = t == i ? 1.0f : t > i ? p * gt : 0.0f;
+            p = t == i ? 1.0 : t > i ? p * gt : 0.0;
             if (lane < QG_C) {
                 // (selects: what lies above the diagonal was never written)
-                Ls[t][i] = t > i ? bt * p * KK[t][i] : 0.0f;
-                Ms[t][i] = t >= i ? p * QK[t][i] : 0.0f;
+                Ls[t][i] = t > i ? (float)(bt * p * KK[t][i]) : 0.0f;
+                Ms[t][i] = t >= i ? (float)(p * QK[t][i]) : 0.0f;
             }
         }
-        if (lane < QG_C) w.sc[hc * QG_C + i] = make_float4(bi, bi * gam, gam, p);
+        if (lane < QG_C) w.sc[hc * QG_C + i] = make_float4(bi, (float)(bi * gam), (float)gam, (float)p);
         __builtin_amdgcn_wave_barrier();
         float x[QG_C];
 #pragma unroll
@@ -663,10 +684,11 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
 #pragma unroll
             for (int j = 0; j < 8; j++) *reinterpret_cast<float4 *>(&Ks[t0 + ln][16 * j + 4 * kg]) = a[j];
         }
-        // K S0' or Q S0': four chains a tile, met in a tree (one chain of 32 sums rounds more than the serial form)
+        // K S0' or Q S0': eight chains a tile, met in a tree (here and below a
+        // long chain, or one that starts on a large value, rounds more than the serial form)
         qg_f4 d[QG_VT];
         {
-            qg_f4 dd[QG_VT][4];
+            qg_f4 dd[QG_VT][8];
             float4 sb[QG_VT][8];
 #pragma unroll
             for (int j = 0; j < 8; j++)
@@ -675,22 +697,24 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
                     sb[z][j] = *reinterpret_cast<const float4 *>(&Ss[16 * z + ln][16 * j + 4 * kg]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++) dd[z][0] = dd[z][1] = dd[z][2] = dd[z][3] = qg_f4{0.f, 0.f, 0.f, 0.f};
+            for (int z = 0; z < QG_VT; z++)
 #pragma unroll
-            for (int j = 0; j < 8; j += 4)
+                for (int j = 0; j < 8; j++) dd[z][j] = qg_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 8; j++)
 #pragma unroll
                 for (int e = 0; e < 4; e++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-#pragma unroll
-                        for (int z = 0; z < QG_VT; z++)
-                            dd[z][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&a[j + i])[e],
-                                                                           reinterpret_cast<const float *>(&sb[z][j + i])[e],
-                                                                           dd[z][i], 0, 0, 0);
+                    for (int z = 0; z < QG_VT; z++)
+                        dd[z][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&a[j])[e],
+                                                                       reinterpret_cast<const float *>(&sb[z][j])[e],
+                                                                       dd[z][j], 0, 0, 0);
 #pragma unroll
             for (int z = 0; z < QG_VT; z++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) d[z][e] = (dd[z][0][e] + dd[z][1][e]) + (dd[z][2][e] + dd[z][3][e]);
+                for (int e = 0; e < 4; e++)
+                    d[z][e] = ((dd[z][0][e] + dd[z][1][e]) + (dd[z][2][e] + dd[z][3][e])) +
+                              ((dd[z][4][e] + dd[z][5][e]) + (dd[z][6][e] + dd[z][7][e]));
         }
         if (!isq) {
 #pragma unroll
@@ -713,23 +737,24 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
                 x0[z] = *reinterpret_cast<const float4 *>(&X[16 * z + ln][4 * kg]);
                 x1[z] = *reinterpret_cast<const float4 *>(&X[16 * z + ln][16 + 4 * kg]);
             }
-            qg_f4 p[QG_VT];
+            qg_f4 p[QG_VT][4];
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++) p[z] = qg_f4{0.f, 0.f, 0.f, 0.f};
+            for (int z = 0; z < QG_VT; z++) p[z][0] = p[z][1] = p[z][2] = p[z][3] = qg_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int e = 0; e < 4; e++)
 #pragma unroll
                 for (int z = 0; z < QG_VT; z++) {
-                    o[z] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&tm[0])[e],
-                                                                reinterpret_cast<const float *>(&x0[z])[e], o[z], 0, 0, 0);
+                    p[z][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&tm[0])[e],
+                                                                       reinterpret_cast<const float *>(&x0[z])[e], p[z][e & 1], 0, 0, 0);
                     if (t0)
-                        p[z] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&tm[1])[e],
-                                                                    reinterpret_cast<const float *>(&x1[z])[e], p[z], 0, 0, 0);
+                        p[z][2 + (e & 1)] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&tm[1])[e],
+                                                                                 reinterpret_cast<const float *>(&x1[z])[e],
+                                                                                 p[z][2 + (e & 1)], 0, 0, 0);
                 }
 #pragma unroll
             for (int z = 0; z < QG_VT; z++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) o[z][e] += p[z][e];
+                for (int e = 0; e < 4; e++) o[z][e] += (p[z][0][e] + p[z][1][e]) + (p[z][2][e] + p[z][3][e]);
         };
         if (!isq) {
             // U = T R
@@ -761,12 +786,9 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
                     const int kc = 32 * wave + 16 * u + ln, r = 16 * i + 4 * kg;
                     ka[u][i] = make_float4(Ks[r][kc], Ks[r + 1][kc], Ks[r + 2][kc], Ks[r + 3][kc]);
                 }
+            qg_f4 ds[QG_VT][2];
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) S[z][u][e] *= gc;
+            for (int z = 0; z < QG_VT; z++) ds[z][0] = ds[z][1] = qg_f4{0.f, 0.f, 0.f, 0.f};
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < 2; i++)
@@ -776,9 +798,15 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
                     for (int u = 0; u < 2; u++)
 #pragma unroll
                         for (int z = 0; z < QG_VT; z++)
-                            S[z][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&ka[u][i])[e],
-                                                                          reinterpret_cast<const float *>(&bu[z][i])[e],
-                                                                          S[z][u], 0, 0, 0);
+                            ds[z][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&ka[u][i])[e],
+                                                                           reinterpret_cast<const float *>(&bu[z][i])[e],
+                                                                           ds[z][u], 0, 0, 0);
+#pragma unroll
+            for (int z = 0; z < QG_VT; z++)
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) S[z][u][e] = __builtin_fmaf(S[z][u][e], gc, ds[z][u][e]);
         }
         if (isq) {
             // Y = G Q S0' + (P o Q K') U
