@@ -204,8 +204,8 @@ __global__ void __launch_bounds__(QS_THREADS) __attribute__((amdgpu_waves_per_eu
 // A workgroup has NW waves of 16 TB blocks, whose keys stay in registers
 // while it walks its rows; the rows' heads pass through LDS eight rows at a
 // time (one row alone is read straight from memory).
-// 512 rows at 16K: 127 us with K = 1 MFMAs (the serial chain's order, half
-// the rate), 102 here; one row of 8192 blocks: 10.0 us with a thread a block,
+// 512 rows at 16K: 127 us with K = 1 MFMAs in the serial chain's order, 102
+// here; one row of 8192 blocks: 10.0 us with a thread a block,
 // 4.1 here.  What bounds it: many rows, the fp32 MFMA's issue (35 cycles each,
 // 60 of the 102) and the staging between groups of rows; one row, the trip to
 // memory.
