@@ -395,8 +395,8 @@ __global__ void __launch_bounds__(QG_THREADS) k_gated_delta(float *__restrict__ 
 // a workgroup 16 value rows of a head, every product on the fp32 matrix cores
 // (v_mfma_f32_16x16x4_f32: fp32 inputs and sums, as the serial form).
 // 2048 steps of 16 key and 48 value heads: 10 + 590 us serial (70 vector
-// operations a step on the CUs that hold two workgroups), 40 + 235 here; the
-// call with conv and output gate 686 -> 335.  Error against 64 bits over calls
+// operations a step on the CUs that hold two workgroups), 39 + 268 here; the
+// call with conv and output gate 690 -> 370.  Error against 64 bits over calls
 // of 600 and 2048 steps: y 1.50 to 1.51e-7 serial, 1.48 to 1.51e-7 here, the
 // state 1.19 to 1.33e-7 and 1.09 to 1.22e-7.  That takes short chains from zero
 // met in trees, and the norms' factors and the gates' products in 64 bits
@@ -405,9 +405,11 @@ __global__ void __launch_bounds__(QG_THREADS) k_gated_delta(float *__restrict__ 
 // wave and three hand-offs through LDS) on the CUs that hold two of the 384
 // workgroups, and its operands' bytes (K and Q read by 8 workgroups a head: a
 // build without the loads takes 165 us).
-// A step with a NaN or infinite input spoils the outputs of its whole chunk
-// (the zeros of T and Q K' above the diagonal multiply it), not only those
-// after it as in the serial form; the state is spoilt from there on in both.
+// A NaN or infinity must not reach the chunk's earlier steps through the zeros
+// of T and Q K' above the diagonal, so a value row's first step with one is
+// kept (`bad`): R and U are zero from there on as operands of those products,
+// and the row's outputs from there on are NaN, its state what it comes to
+// (34 us of the 268).
 #define QG_C 32
 #define QG_LONG_MIN_ROWS 256     // below, the serial kernel (and its bits) stay
 #define QG_LONG_ROWS 4096        // steps a pair of launches takes: bounds the scratch
@@ -622,6 +624,7 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
 {
     __shared__ __align__(16) float Ss[16 * QG_VT][QG_CS], Ks[QG_C][QG_CS];
     __shared__ __align__(16) float Rt[16 * QG_VT][QG_TS], Ut[16 * QG_VT][QG_TS], Up[16 * QG_VT][QG_TS];
+    __shared__ int bad[2][16 * QG_VT];       // by the chunk's parity
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 15, kg = lane >> 4;
     // the workgroups of a key head (which read its q and k) on one XCD
     constexpr unsigned per = QG_DV / (16 * QG_VT);
@@ -663,6 +666,8 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
         }
         fg = w.sc[((size_t)h * nch + c) * QG_C + QG_C - 1].z;     // G[C - 1]
     };
+    if (tid < 32 * QG_VT) (&bad[0][0])[tid] = QG_C;
+    auto finite = [](float x) { return (__float_as_uint(x) & 0x7F800000u) != 0x7F800000u; };
     fetch(0);
     qg_sync();
     for (int c = 0; c < nch; c++) {
@@ -725,6 +730,12 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
                     const bool in = c * QG_C + t0 + 4 * kg + e < rows;
                     r[e] = in ? __builtin_fmaf(s4[e].x, vv[z][e], -(s4[e].y * d[z][e])) : 0.0f;
                 }
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (!finite(r[e])) {
+                        atomicMin(&bad[c & 1][16 * z + ln], t0 + 4 * kg + e);
+                        r[e] = 0.0f;
+                    }
                 *reinterpret_cast<qg_f4 *>(&Rt[16 * z + ln][t0 + 4 * kg]) = r;
             }
         }
@@ -756,6 +767,7 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
 #pragma unroll
                 for (int e = 0; e < 4; e++) o[z][e] += (p[z][0][e] + p[z][1][e]) + (p[z][2][e] + p[z][3][e]);
         };
+        if (tid >= 256 - 16 * QG_VT) bad[(c + 1) & 1][tid - (256 - 16 * QG_VT)] = QG_C;   // the next chunk's
         if (!isq) {
             // U = T R
             qg_f4 u[QG_VT];
@@ -765,8 +777,17 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
 #pragma unroll
             for (int z = 0; z < QG_VT; z++) {
                 qg_f4 up;
+                const int fb = bad[c & 1][16 * z + ln];
 #pragma unroll
-                for (int e = 0; e < 4; e++) up[e] = u[z][e] * s4[e].w;
+                for (int e = 0; e < 4; e++) {
+                    const int t = t0 + 4 * kg + e;
+                    if (t >= fb) u[z][e] = __builtin_nanf("");
+                    up[e] = u[z][e] * s4[e].w;
+                    if (!finite(u[z][e])) {
+                        atomicMin(&bad[c & 1][16 * z + ln], t);
+                        u[z][e] = 0.0f;
+                    }
+                }
                 *reinterpret_cast<qg_f4 *>(&Ut[16 * z + ln][t0 + 4 * kg]) = u[z];
                 *reinterpret_cast<qg_f4 *>(&Up[16 * z + ln][t0 + 4 * kg]) = up;
             }
@@ -821,7 +842,8 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const int t = c * QG_C + t0 + 4 * kg + e;
-                    if (t < rows) y[((size_t)t * hv + h) * QG_DV + v0 + 16 * z + ln] = o[z][e];
+                    const float yv = t0 + 4 * kg + e >= bad[c & 1][16 * z + ln] ? __builtin_nanf("") : o[z][e];
+                    if (t < rows) y[((size_t)t * hv + h) * QG_DV + v0 + 16 * z + ln] = yv;
                 }
         }
 #pragma unroll

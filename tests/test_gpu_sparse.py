@@ -527,6 +527,31 @@ def test_gated_delta_chunks(gpu, hk, hv, rows, decay):
         assert rel_l2(y[t], wy[t]) < 2e-5, f"step {t}"
 
 
+@pytest.mark.parametrize("what,at", [("v", 100), ("v", 64), ("v", 95), ("k", 75), ("q", 33)])
+def test_gated_delta_chunks_not_finite(gpu, what, at):
+    """A NaN or infinity at one step: the steps before it keep the clean
+    call's bits, and from it on what the serial form loses is not finite."""
+    hk, hv, rows = 1, 2, 290
+    q, k, v, g, beta, s0 = delta_inputs(hk, hv, rows, 5)
+    y0, s_clean, _ = gpu_delta(gpu, q, k, v, g, beta, s0, hk, hv, rows)
+    if what == "v":
+        v[at, 1, 37] = np.inf if at == 95 else np.nan
+    else:
+        {"k": k, "q": q}[what][at, 0, 5] = np.nan
+    y1, s1, _ = gpu_delta(gpu, q, k, v, g, beta, s0, hk, hv, rows)
+    assert same_bits(y1[:at], y0[:at]), "earlier steps"
+    lost = np.zeros(y0.shape, bool)
+    slost = np.zeros(s1.shape, bool)
+    if what == "v":
+        lost[at:, 1, 37], slost[1, 37] = True, True
+    elif what == "k":
+        lost[at:], slost[:] = True, True
+    else:
+        lost[at] = True
+    assert np.array_equal(~np.isfinite(y1), lost) and same_bits(y1[~lost], y0[~lost])
+    assert np.array_equal(~np.isfinite(s1), slost) and same_bits(s1[~slost], s_clean[~slost])
+
+
 @pytest.mark.parametrize("hk,hv,rows", [(16, 48, 270), (2, 6, 320)])
 def test_gated_delta_prep_chunks(gpu, hk, hv, rows):
     """Prepared: norms and gates ahead of the chunks; snapshots asked for
