@@ -247,8 +247,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_xgemm(QxArgs a)
     // how the scales come (uniform): a flat copy of the block's columns, 8
     // groups of a column a load, or one by one; the last two also the biases
     const bool wide = groups % 8 == 0 && (((uintptr_t)sb | (uintptr_t)bb) & 15) == 0;
-    const int sld = min(groups, SGL);                            // groups a column in Sc
     const bool flat = groups <= SGL && ((uintptr_t)sb & 15) == 0 && (n * (long)groups) % 8 == 0;
+    // groups a column in Sc; one by one no more than a split product's slice has
+    const int sld = GATHER || flat || wide ? min(groups, SGL) : min(min(groups, SGL), a.kslice / G);
 
     // ---- this lane's loads -----------------------------------------------------------
     const _Float16 *asrc[AI];
@@ -313,9 +314,34 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_xgemm(QxArgs a)
                 qx_dma(sc0 + i * 1024, sb + (size_t)min(n0 + c, n - 1) * groups + (g < groups ? g : 0));
             }
         } else {
-            for (int i = t; i < BN * sld; i += THREADS) {
-                const int c = i / sld, g = g0 + i % sld;
-                Sc[i] = g < groups ? sb[(size_t)min(n0 + c, n - 1) * groups + g] : 0;
+            if constexpr (GATHER) {
+                // (only a bank off a 16-byte boundary, or an odd one of more than SGL groups)
+                for (int i = t; i < BN * sld; i += THREADS) {
+                    const int c = i / sld, g = g0 + i % sld;
+                    Sc[i] = g < groups ? sb[(size_t)min(n0 + c, n - 1) * groups + g] : 0;
+                }
+            } else {
+                // LB in flight: one at a time, 128 columns of 96 groups were 48
+                // trips to memory in a row (16 x 4160 x 6144, groups of 32: 42.8
+                // -> 32.4 us a call).  Their places are stepped to: with a
+                // division each, calls that never come here ran up to 7% longer
+                constexpr int LB = MT * NT > 12 ? 4 : 8;
+                const int dc = THREADS / sld, dg = THREADS % sld;
+                int c = t / sld, g = t % sld;
+                for (int i0 = t; i0 < BN * sld; i0 += LB * THREADS) {
+                    uint16_t v[LB];
+#pragma unroll
+                    for (int u = 0; u < LB; u++) {
+                        const uint16_t x = sb[(size_t)min(n0 + c, n - 1) * groups + min(g0 + g, groups - 1)];
+                        v[u] = g0 + g < groups ? x : 0;
+                        c += dc;
+                        g += dg;
+                        if (g >= sld) { g -= sld; c++; }
+                    }
+#pragma unroll
+                    for (int u = 0; u < LB; u++)
+                        if (i0 + u * THREADS < BN * sld) Sc[i0 + u * THREADS] = v[u];
+                }
             }
         }
     };

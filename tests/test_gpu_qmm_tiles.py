@@ -124,3 +124,23 @@ def test_grouped_product_edges(gpu, E, K, rows, k, n, G, by_pair):
         if p.size:
             w = x[p if by_pair else p // K].astype(np.float64) @ q.dequant(e * n, n).astype(np.float64).T
             assert rel_l2(y[p], w) < 4e-4, f"expert {e}"
+
+
+@pytest.mark.parametrize("rows,k,n,G", [
+    (16, 4160, 6144, 32),      # 130 groups in slices of 16: a window no wider than the slice
+    (24, 5632, 1536, 32),      # 176: the same, 8 a load
+    (40, 4160, 6140, 32),
+    (1000, 3392, 10230, 64),   # 53 groups, unsplit: two windows of 48
+])
+def test_staged_product_scale_windows(gpu, rows, k, n, G):
+    """Scales that come by the window, few or one at a time."""
+    q = synth.make_q4(rows + k, "window", n, k, G)
+    x = np.random.default_rng(rows).uniform(-1, 1, (rows, k)).astype(np.float32)
+    B = gpu.Buf
+    wb, sb, bb, xb, yb = B.of(q.w), B.of(q.s), B.of(q.b), B.of(x), B(rows * n * 4)
+    c = gpu.qw_cmd_begin()
+    gpu.qw_op_qmm_q4(c, yb.ref(), xb.ref(), wb.ref(), sb.ref(), bb.ref(), k, n, rows, G)
+    gpu.run(c, "qmm")
+    y, w = yb.read(np.float32, (rows, n)), want(q, x)
+    for c0 in range(0, n, 128):
+        assert rel_l2(y[:, c0:c0 + 128], w[:, c0:c0 + 128]) < 4e-4, f"columns from {c0}"
