@@ -46,12 +46,15 @@
 #include "qw_device.h"
 #include "qw_kernels.h"
 
+#include <climits>
+
 typedef _Float16 qw_h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 qw_b8 __attribute__((ext_vector_type(8)));
 typedef float qw_f4 __attribute__((ext_vector_type(4)));
 
 #define QX_KPAD 256              // staged rows are padded with zeros to a multiple of this
 #define QX_SB 16                 // groups a block of the staged sums
+#define QX_SLICE 8               // a slice of k is a multiple of this many groups
 #define QX_SLOTS 512             // workgroups the chip holds at two a CU
 #define QX_WIDE_K 1024           // rows of at least this many elements are staged by a workgroup each
 #define QX_CHUNK_ROWS 8192       // rows a dense call stages at a time (bounds its scratch)
@@ -158,7 +161,7 @@ struct QxArgs {
     int K, x_by_pair;        // grouped: the source row of pair p is x_by_pair ? p : p / K
     int rows;                // dense: rows
     int nblk, nbw;           // column blocks, and how many of them a workgroup runs back to back
-    int kslice;              // k range of a blockIdx.y slice (whole stages and 16-group blocks; k: no split)
+    int kslice;              // k range of a blockIdx.y slice (whole stages, a multiple of QX_SLICE groups; k: no split)
     float *part;             // dense split-K: slice s writes part[s][rows][n]
 };
 
@@ -241,6 +244,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_xgemm(QxArgs a)
 
     const int k = a.k, n = a.n, words = k / 8, groups = k / G;
     const int kb = (int)blockIdx.y * a.kslice, ke = min(k, kb + a.kslice), T = (ke - kb + BK - 1) / BK;
+    // the slice's groups; it starts and ends at a multiple of 8 (or at the row's end), so a lane's 8 biases are in or out
+    const int gb = GATHER ? 0 : kb / G, ge = GATHER ? groups : (ke + G - 1) / G;
     const uint32_t *wb = a.w + (size_t)expert * n * words;
     const uint16_t *sb = a.s + (size_t)expert * n * groups;
     const uint16_t *bb = a.b + (size_t)expert * n * groups;
@@ -390,31 +395,31 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_xgemm(QxArgs a)
     // ---- the biases' product, 16 groups at a time ------------------------------------
     // from memory, under the first stages' trip
     if (!lds_bias) {
-        const int g_end = (ke + G - 1) / G;
         const uint16_t *xr[MT];
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) xr[mt] = a.xp + (size_t)src_row((wm * MT + mt) * 16 + ln) * a.nsb * 64 + 8 * kg;
-        for (int sblk = kb / G / QX_SB; sblk * QX_SB < g_end; sblk++) {
+        for (int sblk = gb / QX_SB; sblk * QX_SB < ge; sblk++) {
             uint4 bf[NT], af[MT][2];
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
                 const int c = min(n0 + (wn * NT + nt) * 16 + ln, n - 1), g = sblk * QX_SB + 8 * (kg & 1);
-                // (every load issued, at a clamped place; what is past the row's groups is zeroed after)
+                // (every load issued, at a clamped place; what is not of the slice's groups is zeroed after)
+                const bool in = g >= gb && g < ge;
                 const uint16_t *p = bb + (size_t)c * groups;
                 if (wide) {
                     bf[nt] = *reinterpret_cast<const uint4 *>(p + (g < groups ? g : 0));
-                    if (g >= groups) bf[nt] = make_uint4(0, 0, 0, 0);
+                    if (!in) bf[nt] = make_uint4(0, 0, 0, 0);
                 } else if (groups % 4 == 0 && ((uintptr_t)bb & 7) == 0) {
                     const uint2 u = *reinterpret_cast<const uint2 *>(p + min(g, groups - 4));
                     const uint2 w = *reinterpret_cast<const uint2 *>(p + min(g + 4, groups - 4));
-                    bf[nt] = make_uint4(g < groups ? u.x : 0u, g < groups ? u.y : 0u, g + 4 < groups ? w.x : 0u,
-                                        g + 4 < groups ? w.y : 0u);
+                    const bool hi = in && g + 4 < groups;
+                    bf[nt] = make_uint4(in ? u.x : 0u, in ? u.y : 0u, hi ? w.x : 0u, hi ? w.y : 0u);
                 } else {
                     uint32_t o[8];
 #pragma unroll
                     for (int e = 0; e < 8; e++) o[e] = p[min(g + e, groups - 1)];
 #pragma unroll
-                    for (int e = 0; e < 8; e++) o[e] = g + e < groups ? o[e] : 0u;
+                    for (int e = 0; e < 8; e++) o[e] = in && g + e < groups ? o[e] : 0u;
                     bf[nt] = make_uint4(o[0] | o[1] << 16, o[2] | o[3] << 16, o[4] | o[5] << 16, o[6] | o[7] << 16);
                 }
             }
@@ -526,15 +531,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_xgemm(QxArgs a)
         qx_wait<0>();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         const uint16_t *Bs = reinterpret_cast<const uint16_t *>(ring + (size_t)(T % NST) * STG);
-        const int g_end = min(groups, (ke + G - 1) / G);
 #pragma unroll 1
-        for (int u = 0; u * QX_SB < g_end - kb / G; u++) {
-            const int sblk = kb / G / QX_SB + u, g = sblk * QX_SB + 8 * (kg & 1);
+        for (int sblk = gb / QX_SB; sblk * QX_SB < ge; sblk++) {
+            const int g = sblk * QX_SB + 8 * (kg & 1);
             uint4 xf[MT][2];
             if (held) {
 #pragma unroll
                 for (int q = 0; q < XS; q++)
-                    if (q == u) {
+                    if (q == sblk) {
 #pragma unroll
                         for (int mt = 0; mt < MT; mt++) { xf[mt][0] = xa[q][mt][0]; xf[mt][1] = xa[q][mt][1]; }
                     }
@@ -554,7 +558,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_xgemm(QxArgs a)
 #pragma unroll
                 for (int e = 0; e < 8; e++) o[e] = p[min(g + e, groups - 1)];
 #pragma unroll
-                for (int e = 0; e < 8; e++) o[e] = g + e < g_end ? o[e] : 0u;
+                for (int e = 0; e < 8; e++) o[e] = g >= gb && g + e < ge ? o[e] : 0u;
                 const uint4 bf = make_uint4(o[0] | o[1] << 16, o[2] | o[3] << 16, o[4] | o[5] << 16, o[6] | o[7] << 16);
 #pragma unroll
                 for (int h = 0; h < 2; h++)
@@ -865,11 +869,12 @@ extern "C" int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const in
 #define QW_QMM_SPLIT_WG 1024
 #define QW_QMM_SPLIT_MIN_K 512
 
-// Which products are small (both sides timed, us a call, this against the
-// staged form): 8 x 3072 x 3072 24.4 / 25.8, 20 x 1024 x 1024 23.0 / 24.9,
-// 33 x 3392 x 832 28.0 / 30.3, but 16 x 3072 x 10240 30.2 / 27.1 and 130 x
-// 2560 x 2560 40.7 / 34.5; a short k gives the stages little to overlap: 300
-// x 320 x 12288 28.8 / 30.2, 1021 x 320 x 12288 44.5 / 33.
+// Which products are small: under 2^27 multiply-adds, or a short k, which
+// gives the stages little to overlap.  us a call, this against the staged
+// form: 9 x 3072 x 3072 24.9 / 27.2, 20 x 1024 x 1024 23.0 / 24.9, 56 x 320 x
+// 12288 20.3 / 22.6, but 112 x 3072 x 1024 30.8 / 28.9, 512 x 320 x 12288 38.2
+// / 32.5.  (16 x 3072 x 3072 would be 25.4 / 26.7 still; but the staged form
+// scales a row, so that no input overflows f16, and keeps what it has.)
 static bool qmm_small(int k, int n, int rows)
 {
     const double macs = (double)rows * n * k;
@@ -908,40 +913,79 @@ static void qmm_reduce(hipStream_t s, float *y, const float *part, long total, i
     hipLaunchKernelGGL(k_qmm_reduce, dim3((unsigned)(want < 4096 ? want : 4096)), dim3(256), 0, s, y, part, total, splits);
 }
 
-// The staged plan, a function of the shape only.  Up to 64 rows: one tile of
-// 16, 32 or 64 rows against 128 columns a workgroup; more: 128 rows against
-// 32 nt columns.  Where that leaves the chip's QX_SLOTS workgroup places
-// empty, k is cut into slices (of whole stages and whole 16-group blocks),
-// whose partial sums are added in slice order.  nt is the one that ends
-// first: rounds of workgroups, each as long as its stages' MFMAs plus what a
-// stage costs at any width, and the partials' trip through memory.
+// The staged plan, a function of the shape only: tiles of 16, 32 or 64 rows
+// against 128 columns, or of 128 rows against 32 nt, and where that leaves the
+// chip's QX_SLOTS workgroup places empty k cut into slices (of whole stages
+// and QX_SLICE groups), whose partial sums are added in slice order.  The plan
+// is the one that ends first by the times below: what 64 k cost a workgroup
+// with a CU of its own and with another on it, its start, the scales where
+// they do not come as one flat copy, and the partials.  The times are a fit
+// to 16400 timed (shape, plan) pairs: 844 shapes of 8 to 2048 rows, k 320 to
+// 12288, n 320 to 12288.  The plan chosen is 1.2% slower than the best of them
+// on average (20% at worst); up to 32 rows of 2^27 to 2^28 multiply-adds, and
+// there only, it is up to 7% (2 us) slower than k_sgemm.
+// us a call: k_sgemm / 128-row tiles from 65 rows on, slices of 16 groups and
+// a split priced four times too dear / this:
+//   17 x 5888 x 3456 31 / 34 / 28      192 x 3456 x  5888  55 / 66 / 44
+//   65 x 3072 x 8192 50 / 38 / 34      256 x 3072 x  8192 114 / 52 / 45
+//  129 x 3456 x 5888 51 / 64 / 44      400 x 5888 x  3456  96 / 68 / 59
+//  512 x 3072 x 3072 65 / 54 / 45      129 x 6144 x 10240 156 / 96 / 60
+//  groups of 32: 38 x 4160 x 6144 42 / 48 / 38, 63 x 5504 x 1536 34 / 42 / 32
 struct QxPlan { int bm, nt, splits, kslice; };
+struct QxTile {
+    int bm, nt, lo, hi;          // for calls of lo to hi rows
+    double alone, paired;        // us for 64 k
+    int setup, sgl;              // a workgroup's start in 64-k stages; k_xgemm's SGL
+};
+static const QxTile QX_TILES[] = {
+    {16, 2, 1, 64, 0.29, 0.335, 6, 96},         {32, 2, 17, 128, 0.29, 0.38, 6, 48},
+    {64, 2, 33, 512, 0.53, 0.64, 6, 96},        {128, 2, 65, INT_MAX, 0.64, 0.76, 8, 48},
+    {128, 3, 65, INT_MAX, 0.80, 0.92, 8, 48},   {128, 4, 65, INT_MAX, 0.96, 1.08, 8, 48},
+    {128, 5, 65, INT_MAX, 1.13, 1.24, 8, 48},
+};
 
 static QxPlan qx_plan(int k, int n, int rows, int group)
 {
     QxPlan best = {};
     double cost = 1e300;
-    const int bm = rows > 64 ? 128 : rows > 32 ? 64 : rows > 16 ? 32 : 16;
-    const long rt = (rows + bm - 1) / bm;
-    const int unit = QX_SB * group;                              // a slice is a multiple of this (and of any BK)
-    for (int nt = 2; nt <= (bm == 128 ? 5 : 2); nt++) {
-        const int bn = bm == 128 ? 32 * nt : 128;
-        const long tiles = rt * ((n + bn - 1) / bn);
-        const int units = (k + unit - 1) / unit;
-        for (int sp = 1; sp <= units && (sp == 1 || tiles * sp <= QX_SLOTS); sp++) {
-            const int ks = (units + sp - 1) / sp * unit, real = (k + ks - 1) / ks;
-            if (real != sp) continue;
-            const long rounds = (tiles * sp + QX_SLOTS - 1) / QX_SLOTS;
-            // in MFMA-stage units (64 k of a wave tile column): ~0.06 us
-            const double c = rounds * (((sp == 1 ? k : ks) / 64 + 8) * (nt + 1.0)) +
-                             (sp > 1 ? 30.0 + (double)rows * n * (sp + 1) * 4 / 4e6 / 0.06 : 0.0);
+    const int unit = QX_SLICE * group, units = (k + unit - 1) / unit, groups = k / group;
+    const double mb = (double)rows * n * 4e-6;
+    for (const QxTile &t : QX_TILES) {
+        if (rows < t.lo || rows > t.hi) continue;
+        const bool wide = t.bm == 128, flat = groups <= t.sgl && (long)n * groups % 8 == 0;
+        const int bn = wide ? 32 * t.nt : 128;
+        const long tiles = (long)((rows + t.bm - 1) / t.bm) * ((n + bn - 1) / bn);
+        // groups of 32 have half the k a scale; in stages: a group's scales that
+        // do not come flat, and the stop for each further window of them
+        const double per = group != 32 ? 1.0 : wide ? 1.65 : 1.5;
+        const double scales = flat ? 0.0 : wide ? 0.07 : group == 32 ? 0.33 : 0.2, window = flat ? 0.0 : wide ? 1.0 : 3.0;
+        for (int sp = 1; sp <= units && (sp == 1 || tiles * sp <= 2 * QX_SLOTS); sp++) {
+            const int ks = sp == 1 ? k : (units + sp - 1) / sp * unit, gs = ks / group;
+            if ((k + ks - 1) / ks != sp) continue;
+            const long wgs = tiles * sp, full = wgs / QX_SLOTS, rem = wgs % QX_SLOTS;
+            const double stages = (ks + 63) / 64 + t.setup + scales * gs + window * ((gs - 1) / t.sgl);
+            double c = per * stages * (full * t.paired + (rem > QX_SLOTS / 2 ? t.paired : rem ? t.alone : 0.0));
+            if (sp > 1) c += 1.3 + 0.65 * sp + 0.21 * mb * (sp + 1);
             if (c < cost) {
                 cost = c;
-                best = QxPlan{bm, nt, sp, sp == 1 ? k : ks};
+                best = QxPlan{t.bm, t.nt, sp, ks};
             }
         }
     }
     return best;
+}
+
+// The plan of a call's first rows, for tests: rows a tile (0: k_sgemm),
+// 32-column steps of its width, slices of k, k a slice.
+extern "C" void qwk_qmm_plan(int k, int n, int rows, int group, int out[4])
+{
+    QxPlan p = {};
+    if (qmm_small(k, n, rows)) p.splits = qmm_splits(k, n, rows, &p.kslice);
+    else p = qx_plan(k, n, rows < QX_CHUNK_ROWS ? rows : QX_CHUNK_ROWS, group);
+    out[0] = p.bm;
+    out[1] = p.bm == 128 ? p.nt : p.bm ? 4 : 2;
+    out[2] = p.splits;
+    out[3] = p.kslice;
 }
 
 extern "C" size_t qwk_qmm_work_bytes(int k, int n, int rows, int group)

@@ -78,6 +78,10 @@ size_t qwk_gather_gemm_work_bytes(int k, int pairs, int K, int x_by_pair, int gr
 int qwk_qmm(hipStream_t s, float *y, const float *x, qwk_q4 m, int k, int n, int rows, int group,
             void *work, size_t work_bytes);
 size_t qwk_qmm_work_bytes(int k, int n, int rows, int group);
+/* The plan a call of this shape takes (its first rows): rows a tile (0: the
+ * small products' one-launch kernel), the tile's width in steps of 32
+ * columns, slices of k, k a slice.  For tests. */
+void qwk_qmm_plan(int k, int n, int rows, int group, int out[4]);
 
 /* A second weight bank for grouped tiles of expert `expert` (qwk_moe_group's
  * extra rows): its pairs p >= `pairs` read A row p - pairs when not
