@@ -47,6 +47,7 @@
 #include "qw_kernels.h"
 
 #include <climits>
+#include <cmath>
 
 typedef _Float16 qw_h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 qw_b8 __attribute__((ext_vector_type(8)));
@@ -809,12 +810,34 @@ static int qx_nbw(int k, int nblk, long tiles)
     return w < nblk ? w : nblk;
 }
 
+// The same for a grouped product, whose tiles the host can only estimate (the
+// list's bound is half as many again): the number that ends first, in rounds
+// of QX_SLOTS workgroups, each a start of about 2.5 stages of 256 k and its
+// blocks' stages.  (Filling the places by the bound left 400 rows of 6 picks
+// in 256 experts of 320 x 640 a second round of 30 workgroups, as long as the
+// first: the layer op by op 178 us, now 161, 167 with 64 x 64 tiles.)
+extern "C" int qwk_gather_gemm_blocks(int k, int n, int pairs, int E, int bm)
+{
+    E = E < 1 ? 1 : E;
+    const int nblk = (n + 127) / 128;
+    const double mean = (double)pairs / E, fill = mean / bm + 0.5;
+    const double tiles = E * (1.0 - exp(-mean)) * (fill > 1.0 ? fill : 1.0);
+    const int most = k >= 2048 ? 1 : 2048 / (k < 256 ? 256 : k), stages = (k + 255) / 256;
+    int best = 1;
+    double cost = 1e300;
+    for (int w = 1; w <= most && w <= nblk; w++) {
+        const double c = ceil(tiles * ((nblk + w - 1) / w) / QX_SLOTS) * (2.5 + w * stages);
+        if (c < cost) { cost = c; best = w; }
+    }
+    return best;
+}
+
 // Few rows a tile: four waves side by side over 128 columns.
 template <int G, bool GATHER>
-static void qx_narrow(hipStream_t s, QxArgs &a, int bm, int ntiles, int splits)
+static void qx_narrow(hipStream_t s, QxArgs &a, int bm, int ntiles, int splits, int pairs = 0, int E = 0)
 {
     a.nblk = (a.n + 127) / 128;
-    a.nbw = qx_nbw(a.k, a.nblk, (long)ntiles * splits);
+    a.nbw = GATHER ? qwk_gather_gemm_blocks(a.k, a.n, pairs, E, bm) : qx_nbw(a.k, a.nblk, (long)ntiles * splits);
     const long ngr = (a.nblk + a.nbw - 1) / a.nbw;
     const dim3 grid((unsigned)((ngr * ntiles + 7) / 8 * 8), (unsigned)splits), blk(256);
     if (bm == 16) hipLaunchKernelGGL((k_xgemm<G, 1, 2, 1, 4, 256, 2, 96, GATHER>), grid, blk, 0, s, a);
@@ -845,7 +868,7 @@ extern "C" size_t qwk_gather_gemm_work_bytes(int k, int pairs, int K, int x_by_p
 }
 
 extern "C" int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const int32_t *perm,
-                               const int32_t *tiles, qwk_q4 m, int k, int n, int pairs, int K, int x_by_pair,
+                               const int32_t *tiles, qwk_q4 m, int k, int n, int pairs, int E, int K, int x_by_pair,
                                int group, int bm, int max_tiles, void *work, size_t work_bytes)
 {
     if (!gmm_shape_ok(x, m, k, n, group) || K < 1 || (bm != 16 && bm != 32 && bm != 64)) return (int)hipErrorInvalidValue;
@@ -855,9 +878,9 @@ extern "C" int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const in
     a.y = y; a.perm = perm; a.tiles = tiles; a.w = m.w; a.s = m.s; a.b = m.b;
     a.k = k; a.n = n; a.K = K; a.x_by_pair = x_by_pair; a.kslice = k;
     qx_stage(s, a, x, x_by_pair ? pairs : (pairs + K - 1) / K, group, static_cast<char *>(work));
-    if (group == 32) qx_narrow<32, true>(s, a, bm, max_tiles, 1);
-    else if (group == 64) qx_narrow<64, true>(s, a, bm, max_tiles, 1);
-    else qx_narrow<128, true>(s, a, bm, max_tiles, 1);
+    if (group == 32) qx_narrow<32, true>(s, a, bm, max_tiles, 1, pairs, E);
+    else if (group == 64) qx_narrow<64, true>(s, a, bm, max_tiles, 1, pairs, E);
+    else qx_narrow<128, true>(s, a, bm, max_tiles, 1, pairs, E);
     return (int)hipGetLastError();
 }
 

@@ -68,9 +68,11 @@ int qwk_q4mv_multi(hipStream_t s, const float *x, int k, int group, int count,
  * Tiles were cut at `bm` rows by qwk_moe_group; `max_tiles` bounds the grid.
  * work: qwk_gather_gemm_work_bytes(...) bytes for the staged activations. */
 int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const int32_t *perm,
-                    const int32_t *tiles, qwk_q4 m, int k, int n, int pairs, int K, int x_by_pair,
+                    const int32_t *tiles, qwk_q4 m, int k, int n, int pairs, int E, int K, int x_by_pair,
                     int group, int bm, int max_tiles, void *work, size_t work_bytes);
 size_t qwk_gather_gemm_work_bytes(int k, int pairs, int K, int x_by_pair, int group);
+/* Blocks of 128 columns a workgroup of it runs back to back. */
+int qwk_gather_gemm_blocks(int k, int n, int pairs, int E, int bm);
 
 /* Dense prefill product y[rows, n] = x[rows, k] . W^T (the shared expert). */
 /* work: qwk_qmm_work_bytes(k, n, rows, group) bytes for the staged

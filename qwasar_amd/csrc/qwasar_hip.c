@@ -865,7 +865,7 @@ void qw_op_qmm_q4_gather(qw_cmd c, qw_ref y, qw_ref x, qw_ref perm, qw_ref tiles
     void *work = wb ? scratch(wb) : NULL;
     if (wb && !work) { cmd_fail(c, hipErrorOutOfMemory, "qmm_q4_gather: scratch of %zu bytes", wb); return; }
     launched(c, "qmm_q4_gather", qwk_gather_gemm(G.stream, dp(y), dp(x), dp(perm), dp(tiles),
-                                                 q4(w, scales, biases), k, n, pairs, K, x_by_pair ? 1 : 0,
+                                                 q4(w, scales, biases), k, n, pairs, E, K, x_by_pair ? 1 : 0,
                                                  group, bm, tiles_for(pairs, E, bm), work, wb));
 }
 

@@ -2,6 +2,7 @@
 slices that cover k, and no plan that leaves the chip idle or multiplies
 mostly empty rows where a finer one is at hand."""
 import ctypes as C
+import math
 
 import pytest
 
@@ -48,3 +49,20 @@ def test_middle_sizes_fill_the_chip(rows, k, n, G):
 def test_few_empty_rows(rows, k, n, G):
     """Up to 192 rows no more than 63 rows of padding (129 paid for 256)."""
     assert plan(rows, k, n, G)[0] <= 64
+
+
+@pytest.mark.parametrize("k,n,pairs,E", [(640, 640, 2400, 256), (320, 640, 2400, 256), (640, 640, 360, 256),
+                                         (512, 896, 1432, 256), (256, 1792, 2322, 128)])
+def test_grouped_last_round_is_not_nearly_empty(k, n, pairs, E):
+    """Column blocks are run back to back where k is short, but not so that a
+    few workgroups are left for a round of their own (261 tiles of 5 blocks,
+    three at a time: 522 workgroups, a round of 512 and one of 10)."""
+    rows = gpu.qw_moe_tile_rows(pairs, E)
+    w = C.CDLL(gpu.LIB_PATH).qwk_gather_gemm_blocks(k, n, pairs, E, rows)
+    blocks = cut(n, 128)
+    assert 1 <= w <= min(blocks, 8)
+    p = [math.exp(-pairs / E)]                          # pairs an expert: Poisson
+    for i in range(1, 200):
+        p.append(p[-1] * pairs / E / i)
+    wgs = E * sum(q * cut(i, rows) for i, q in enumerate(p)) * cut(blocks, w)
+    assert wgs <= SLOTS or wgs % SLOTS >= SLOTS // 8 or wgs > 4 * SLOTS, (w, wgs)
