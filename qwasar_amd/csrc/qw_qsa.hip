@@ -939,7 +939,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
 #pragma unroll
     for (int t = 0; t < 16; t++) acc[t] = qa_f4{0.f, 0.f, 0.f, 0.f};
 
-    // list entries of a pass from j0 (past the range: its last, whose weight is then zero)
+    // list entries of a pass from j0 (past the range: its last again, with weight zero)
     auto at = [&](int j) { return min(lr[1 + min(j, j_hi - 1)], (uint32_t)(max_ctx - 1)); };
     uint32_t ki[2], vi[8];
     auto entries = [&](int j0) __attribute__((always_inline)) {
@@ -1018,7 +1018,8 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
         qa_h8 pa[3];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const float p = qa_exp2(sc[i] - m);
+            // (a select: where no score is above -FLT_MAX, neither is m)
+            const float p = j0 + 16 * (i >> 2) + 4 * kg + (i & 3) < j_hi ? qa_exp2(sc[i] - m) : 0.0f;
             l += p;
             _Float16 a, b, c;
             qa_split(p * (float)(1 << QAM_P_EXP), a, b, c);

@@ -652,3 +652,56 @@ def test_qsa_scores_many_rows_match_rowwise(gpu, nq, d, base, rows):
             nb = (base + r + 1) // ratio
             assert same_bits(got[r, :nb], one[0, :nb]), f"row {r}"
             assert np.isnan(got[r, nb:]).all()
+
+
+def listed_attn(gpu, q, kb16, vb16, lst, scale):
+    """attn_masked over the given lists (f16 caches as bits), one call."""
+    B = gpu.Buf
+    rows, qh, D = q.shape
+    kvh, ctx = kb16.shape[:2]
+    cap = lst.shape[1] - 1
+    topk, ratio = cap // 4 - 1, 4
+    assert gpu.qw_qsa_list_cap(topk, ratio) == cap
+    qb, kb, vb, lb, ob = B.of(q), B.of(kb16), B.of(vb16), B.of(lst), B(rows * qh * D * 4)
+    c = gpu.qw_cmd_begin()
+    gpu.qw_op_attn_masked(c, ob.ref(), qb.ref(), kb.ref(), vb.ref(), lb.ref(), rows, qh, kvh, D, ctx, ctx - rows,
+                          scale, topk, ratio)
+    gpu.run(c, "attn masked")
+    got = ob.read(np.float32, (rows, qh, D))
+    for t in (qb, kb, vb, lb, ob):
+        t.free()
+    return got
+
+
+def attn64(q, kb16, vb16, lst, r, h, scale):
+    """Row r, head h of the same in 64 bits."""
+    f64 = lambda b: np.asarray(b).view(np.float16).astype(np.float64)
+    at = lst[r, 1:1 + lst[r, 0]]
+    g = h // (q.shape[1] // kb16.shape[0])
+    with np.errstate(all="ignore"):
+        s = f64(kb16[g][at]) @ q[r, h].astype(np.float64) * float(np.float32(scale))
+        w = np.exp(s - s.max())
+        return (w / w.sum()) @ f64(vb16[g][at])
+
+
+def listed_case(kvh, qh, rows, n, seed):
+    """Random q, caches as f16 bits, and rows that list all of 0 .. n - 1."""
+    D = 256
+    kb16 = sparse.f16_bits(rnd((kvh, n, D), seed)).reshape(kvh, n, D)
+    vb16 = sparse.f16_bits(rnd((kvh, n, D), seed + 1)).reshape(kvh, n, D)
+    lst = np.zeros((rows, 1 + n), np.uint32)
+    lst[:, 0] = n
+    lst[:, 1:] = np.arange(n)
+    return rnd((rows, qh, D), seed + 2), kb16, vb16, lst
+
+
+def test_attn_masked_nothing_counts(gpu):
+    """Every listed score below fp32's range: no weight, so zeros, as a call
+    of one row gives; what a pass reads past the list's end has no weight
+    either."""
+    q, kb16, vb16, lst = listed_case(2, 24, 140, 300, 411)
+    q[:] = -np.abs(q) * np.float32(1e34) - np.float32(1e33)
+    kb16[:] = np.float16(6e4).view(np.uint16)
+    lst[:, 0] = np.arange(140) % 300 + 1
+    assert (listed_attn(gpu, q[7:8], kb16, vb16, lst[7:8], 1.0 / 16.0) == 0).all()
+    assert (listed_attn(gpu, q, kb16, vb16, lst, 1.0 / 16.0) == 0).all()
