@@ -913,11 +913,9 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (g < G) v = reinterpret_cast<const float4 *>(q + ((size_t)row * q_heads + (size_t)kvh * G + g) * QA_D)[lane];
         const float mx = qw_wave_max(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-        int sh = 0;
-        if (mx > 0.0f && mx <= FLT_MAX) {
-            sh = 15 - __builtin_amdgcn_frexp_expf(mx);
-            sh = sh < -100 ? -100 : sh > 100 ? 100 : sh;
-        }
+        // (any finite head: -113 .. 163.  A factor that leaves fp32's range
+        // stands for scores that do.)
+        const int sh = mx > 0.0f && mx <= FLT_MAX ? 15 - __builtin_amdgcn_frexp_expf(mx) : 0;
         const float f[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int i = 0; i < 4; i++) {

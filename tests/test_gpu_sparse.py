@@ -705,3 +705,16 @@ def test_attn_masked_nothing_counts(gpu):
     lst[:, 0] = np.arange(140) % 300 + 1
     assert (listed_attn(gpu, q[7:8], kb16, vb16, lst[7:8], 1.0 / 16.0) == 0).all()
     assert (listed_attn(gpu, q, kb16, vb16, lst, 1.0 / 16.0) == 0).all()
+
+
+@pytest.mark.parametrize("size,scale", [(1e37, 2e-38), (1e-36, 2e35)])
+def test_attn_masked_huge_and_tiny_queries(gpu, size, scale):
+    """Queries near either end of fp32's range against a scale that makes
+    ordinary scores of them.  Bar: scores of up to 8 with errors of a few
+    2^-24 of them, 2e-6 of the weights."""
+    q, kb16, vb16, lst = listed_case(2, 24, 140, 300, 421)
+    q *= np.float32(size)
+    got = listed_attn(gpu, q, kb16, vb16, lst, scale)
+    for r in (0, 77, 139):
+        for h in range(24):
+            assert rel_l2(got[r, h], attn64(q, kb16, vb16, lst, r, h, scale)) < 2e-6, (r, h)
