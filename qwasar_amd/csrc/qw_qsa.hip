@@ -848,11 +848,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
 // query heads a kv head, where k_attn_masked's multiply-adds bind it (G = 12:
 // 26 GFLOP of fp32 vector work for 512 rows of 2052 positions, 850 us).  Both
 // products run on f16 MFMAs with nothing rounded to 16 bits: the caches are
-// f16 as they are, and each fp32 operand is cut into three f16 parts (33
-// bits), a part a MFMA, summed in fp32:
+// f16 as they are, and each fp32 operand is cut into three f16 parts, a part a
+// MFMA, the second and third times 2^12 and summed apart (f16's smallest step
+// would cut the small ones off), all sums in fp32:
 //   q   scaled a head by the power of two that puts its largest magnitude in
-//       [2^14, 2^15); the parts stay in LDS for the row
-//   p   the softmax weights 2^(s - m), at most 2^8 (below), times 2^6
+//       [2^14, 2^15); the parts stay in LDS for the row.  All 24 bits of
+//       elements down to 2^-27 of the largest, 2^-51 of it below
+//   p   the softmax weights 2^(s - m), at most 2^4 (below), times 2^11.  All
+//       24 bits down to 2^-23 of the state's unit; what the parts leave of
+//       smaller ones (a dominant position whose values are near zero makes
+//       them count) is added by further turns where it could come to half a
+//       unit of a sum's last place
 // The scores are computed transposed, S'[position][head] = K q': a lane then
 // holds its head's weights for positions 4 kg .. 4 kg + 3 of two tiles of 16,
 // which is an A operand of the second product as it stands if the MFMA's k
@@ -861,29 +867,32 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
 // its 8 positions and takes column t of that 8 x 8 block, by v_perm, as tile
 // t's operand, so tile t holds dims 8 n + t.  No value passes through LDS.
 // A wave takes 32 positions a pass and keeps its own softmax state; the
-// reference maximum moves only when a score passes it by 8 (a weight is then
-// at most 2^8 of the state's unit), so the sums are seldom rescaled.  The four
+// reference maximum moves only when a score passes it by 4 (a weight is then
+// at most 2^4 of the state's unit), so the sums are seldom rescaled.  The four
 // waves' states meet in LDS at the end, as (w0 + w1) + (w2 + w3).
 // 512 rows of 2052 positions at 16K, 24 / 2 heads: 850 -> 185 us, and closer
 // to 64 bits (2.5e-7 against 4.3e-7).  What bounds it: the gathered rows, 1 KB
 // a position and kv head, 2.1 GB for that call: 11.6 TB/s through the L1s.
 typedef _Float16 qa_h8 __attribute__((ext_vector_type(8)));
 typedef float qa_f4 __attribute__((ext_vector_type(4)));
+typedef unsigned short qa_us2 __attribute__((ext_vector_type(2)));
 #define QAM_HEADS 16                      // a MFMA tile of heads (G of them real)
 #define QAM_QST (QA_D + 8)                // halfs a head's row takes in LDS
 #define QAM_OST (QA_D + 4)                // floats
 #define QAM_STEP 32                       // positions a wave takes a pass
-#define QAM_P_EXP 6
-#define QAM_SLACK 8.0f
+#define QAM_SLACK 4.0f                    // what a weight's exponent may be above its state's unit
+#define QAM_P_UNIT 0x1p11f                // 2^(15 - QAM_SLACK)
 
-// x as three f16 parts, x = a + b + c to 33 bits (fewer near f16's smallest)
-__device__ __forceinline__ void qa_split(float x, _Float16 &a, _Float16 &b, _Float16 &c)
+// x (up to 2^15) as f16 parts, x = a + (b + c + r) 2^-12; r, at most 2^-25, is
+// zero where x has no bit below 2^-36
+__device__ __forceinline__ float qa_split(float x, _Float16 &a, _Float16 &b, _Float16 &c)
 {
     a = (_Float16)x;
-    float r = x - (float)a;
+    float r = (x - (float)a) * 4096.0f;
     b = (_Float16)r;
     r = r - (float)b;
     c = (_Float16)r;
+    return r - (float)c;
 }
 
 template <int G>
@@ -995,12 +1004,12 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int j = j0 + 16 * (i >> 2) + 4 * kg + (i & 3);
-            sc[i] = j < j_hi ? (hi[i >> 2][i & 3] + lo[i >> 2][i & 3]) * fac : -FLT_MAX;
+            sc[i] = j < j_hi ? __builtin_fmaf(lo[i >> 2][i & 3], 0x1p-12f, hi[i >> 2][i & 3]) * fac : -FLT_MAX;
             cm = fmaxf(cm, sc[i]);
         }
         cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
         cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
-        const bool up = cm > m + QAM_SLACK;                    // (at first m + 8 is -FLT_MAX itself)
+        const bool up = cm > m + QAM_SLACK;                    // (at first m + 4 is -FLT_MAX itself)
         if (__ballot(up)) {
             const float mn = up ? cm : m, f = qa_exp2(m - mn);
             m = mn;
@@ -1014,33 +1023,92 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
                 for (int e = 0; e < 4; e++) acc[t][e] *= fr[e];
         }
         qa_h8 pa[3];
+        float rem[8];
+        bool left = false;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             // (a select: where no score is above -FLT_MAX, neither is m)
             const float p = j0 + 16 * (i >> 2) + 4 * kg + (i & 3) < j_hi ? qa_exp2(sc[i] - m) : 0.0f;
             l += p;
             _Float16 a, b, c;
-            qa_split(p * (float)(1 << QAM_P_EXP), a, b, c);
+            rem[i] = qa_split(p * QAM_P_UNIT, a, b, c);
             pa[0][i] = a;
             pa[1][i] = b;
             pa[2][i] = c;
+            left |= fabsf(rem[i]) > 0.0f;
         }
+        const bool deep = __ballot(left) != 0;                 // uniform
+        // column t of the lane's 8 positions x 8 dims
+        auto column = [&](const uint4 (&vv)[8], int t) __attribute__((always_inline)) {
+            uint32_t c[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t x = reinterpret_cast<const uint32_t *>(&vv[2 * i])[t / 2];
+                const uint32_t y = reinterpret_cast<const uint32_t *>(&vv[2 * i + 1])[t / 2];
+                c[i] = __builtin_amdgcn_perm(y, x, t & 1 ? 0x07060302u : 0x05040100u);
+            }
+            return __builtin_bit_cast(qa_h8, make_uint4(c[0], c[1], c[2], c[3]));
+        };
         auto values = [&](const uint4 (&vv)[8], int t0) __attribute__((always_inline)) {
 #pragma unroll
             for (int t = 0; t < 8; t++) {
-                // column t of the lane's 8 positions x 8 dims
-                uint32_t c[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t x = reinterpret_cast<const uint32_t *>(&vv[2 * i])[t / 2];
-                    const uint32_t y = reinterpret_cast<const uint32_t *>(&vv[2 * i + 1])[t / 2];
-                    c[i] = __builtin_amdgcn_perm(y, x, t & 1 ? 0x07060302u : 0x05040100u);
-                }
-                const qa_h8 b = __builtin_bit_cast(qa_h8, make_uint4(c[0], c[1], c[2], c[3]));
+                const qa_h8 b = column(vv, t);
                 qa_f4 &o = acc[t0 + t];
+                qa_f4 u = {0.f, 0.f, 0.f, 0.f};
+                u = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[2], b, u, 0, 0, 0);
+                u = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[1], b, u, 0, 0, 0);
                 o = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[0], b, o, 0, 0, 0);
-                o = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[1], b, o, 0, 0, 0);
-                o = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[2], b, o, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[e] = __builtin_fmaf(u[e], 0x1p-12f, o[e]);
+            }
+            if (!deep) return;
+            // What the parts left of small weights (32 of at most 2^-37) counts
+            // where it may come to 2^-25 of a sum, half a unit of its last place
+            float least = FLT_MAX;
+            qa_us2 big = {0, 0};
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    least = fminf(least, fabsf(acc[t0 + t][e]));
+                    big = __builtin_elementwise_max(
+                        big, __builtin_bit_cast(qa_us2, reinterpret_cast<const uint32_t *>(&vv[t])[e] & 0x7FFF7FFFu));
+                }
+            }
+            float vm = fmaxf(qa_f16(big[0]), qa_f16(big[1]));
+            vm = fmaxf(vm, __shfl_xor(vm, 16, 64));
+            vm = fmaxf(vm, __shfl_xor(vm, 32, 64));
+            if (!__ballot(!(least >= vm * 0x1p-7f))) return;
+            float r[8], dn = 0x1p-12f;
+#pragma unroll
+            for (int i = 0; i < 8; i++) r[i] = rem[i];
+#pragma unroll 1
+            for (int turn = 0; turn < 3; turn++) {             // (50 bits a turn: down to 2^-136)
+                qa_h8 pd[3];
+                bool more = false;
+                dn *= 0x1p-38f;
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    _Float16 a, b, c;
+                    r[i] = qa_split(r[i] * 0x1p38f, a, b, c);
+                    pd[0][i] = a;
+                    pd[1][i] = b;
+                    pd[2][i] = c;
+                    more |= fabsf(r[i]) > 0.0f;
+                }
+#pragma unroll
+                for (int t = 0; t < 8; t++) {
+                    const qa_h8 b = column(vv, t);
+                    qa_f4 h = {0.f, 0.f, 0.f, 0.f}, u = h;
+                    h = __builtin_amdgcn_mfma_f32_16x16x32_f16(pd[0], b, h, 0, 0, 0);
+                    u = __builtin_amdgcn_mfma_f32_16x16x32_f16(pd[2], b, u, 0, 0, 0);
+                    u = __builtin_amdgcn_mfma_f32_16x16x32_f16(pd[1], b, u, 0, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        acc[t0 + t][e] = __builtin_fmaf(__builtin_fmaf(u[e], 0x1p-12f, h[e]), dn, acc[t0 + t][e]);
+                }
+                if (!__ballot(more)) break;
+                dn *= 0x1p-12f;
             }
         };
         values(v0, 0);
@@ -1078,7 +1146,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
                         (wl[2][g] * qa_exp2(wm[2][g] - M) + wl[3][g] * qa_exp2(wm[3][g] - M));
         const float4 a = *reinterpret_cast<const float4 *>(&os[0][g][d]), b = *reinterpret_cast<const float4 *>(&os[1][g][d]);
         const float4 c = *reinterpret_cast<const float4 *>(&os[2][g][d]), e = *reinterpret_cast<const float4 *>(&os[3][g][d]);
-        constexpr float dn = 1.0f / (float)(1 << QAM_P_EXP);
+        constexpr float dn = 1.0f / QAM_P_UNIT;
         float o[4] = {((a.x + b.x) + (c.x + e.x)) * dn, ((a.y + b.y) + (c.y + e.y)) * dn,
                       ((a.z + b.z) + (c.z + e.z)) * dn, ((a.w + b.w) + (c.w + e.w)) * dn};
         if (nsplit == 1) {

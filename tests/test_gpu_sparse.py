@@ -718,3 +718,26 @@ def test_attn_masked_huge_and_tiny_queries(gpu, size, scale):
     for r in (0, 77, 139):
         for h in range(24):
             assert rel_l2(got[r, h], attn64(q, kb16, vb16, lst, r, h, scale)) < 2e-6, (r, h)
+
+
+def test_attn_masked_small_weights_keep_their_bits(gpu):
+    """One listed position takes nearly all weight and has zero values (an
+    attention sink), the others are 2^-14 to 2^-90 of it: the output is what
+    these few bits of weight give.  Bar: a score of s log2 units has an error
+    of 2^-23 |s|, its weight ln 2 of that; the scores reach 4 + lead, and the
+    sums add less than 4 such steps."""
+    leads = (0, 14, 20, 30, 44, 90)
+    q, kb16, vb16, lst = listed_case(2, 24, 132, 2052, 431)
+    kb16[:, :, 0] = 0
+    q *= np.float32(0.25)
+    for sink, g in ((0, 0), (1027, 1)):            # in a wave's first pass, in a later one
+        kb16[g, sink] = 0
+        kb16[g, sink, 0] = np.float16(1.0).view(np.uint16)
+        vb16[g, sink] = 0
+    for r in range(132):
+        q[r, :, 0] = 16.0 * np.log(2.0) * leads[r % len(leads)]
+    got = listed_attn(gpu, q, kb16, vb16, lst, 1.0 / 16.0)
+    for r in range(len(leads)):
+        for h in (0, 5, 11, 12, 23):
+            e = rel_l2(got[r, h], attn64(q, kb16, vb16, lst, r, h, 1.0 / 16.0))
+            assert e < (8 + leads[r]) * 2.0 ** -23, (leads[r], h, e)
