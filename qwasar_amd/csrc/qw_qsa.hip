@@ -870,8 +870,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
 // reference maximum moves only when a score passes it by 4 (a weight is then
 // at most 2^4 of the state's unit), so the sums are seldom rescaled.  The four
 // waves' states meet in LDS at the end, as (w0 + w1) + (w2 + w3).
-// 512 rows of 2052 positions at 16K, 24 / 2 heads: 850 -> 185 us, and closer
-// to 64 bits (2.5e-7 against 4.3e-7).  What bounds it: the gathered rows, 1 KB
+// Scores sum their first parts in four chains met in a tree, and their factor
+// carries what rounding it to fp32 cuts off.  512 rows of 2052 positions at
+// 16K, 24 / 2 heads, k_attn_masked -> this, for scores with a deviation of 1 /
+// 4 / 24: 810 / 821 / 822 -> 180 / 201 / 216 us, error against 64 bits 4.4e-7 /
+// 5.8e-7 / 9.4e-7 -> 2.2e-7 / 4.7e-7 / 9.1e-7 (two serial sums and a plain
+// factor: 3.1e-7 / 7.1e-7 / 12.4e-7).  What bounds it: the gathered rows, 1 KB
 // a position and kv head, 2.1 GB for that call: 11.6 TB/s through the L1s.
 typedef _Float16 qa_h8 __attribute__((ext_vector_type(8)));
 typedef float qa_f4 __attribute__((ext_vector_type(4)));
@@ -904,7 +908,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
 {
     constexpr int QB = 3 * QAM_HEADS * QAM_QST * 2, OB = 4 * QAM_HEADS * QAM_OST * 4;
     __shared__ __align__(16) uint8_t lds[QB > OB ? QB : OB];
-    __shared__ float qf[QAM_HEADS];                   // a head's score factor
+    __shared__ float2 qf[QAM_HEADS];                  // a head's score factor and what it lacks
     __shared__ float wm[4][QAM_HEADS], wl[4][QAM_HEADS];
     _Float16 (*qp)[QAM_HEADS][QAM_QST] = reinterpret_cast<_Float16 (*)[QAM_HEADS][QAM_QST]>(lds);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 15, kg = lane >> 4;
@@ -934,13 +938,18 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
             qp[1][g][4 * lane + i] = b;
             qp[2][g][4 * lane + i] = c;
         }
-        if (lane == 0) qf[g] = __builtin_ldexpf(scale * QA_LOG2E, -sh);
+        if (lane == 0) {
+            // (a score of 100 units times log2 e's own rounding is 1e-6 of its weight)
+            const double f64 = (double)scale * 1.4426950408889634;
+            const float f32 = (float)f64;
+            qf[g] = make_float2(__builtin_ldexpf(f32, -sh), __builtin_ldexpf((float)(f64 - (double)f32), -sh));
+        }
     }
     __syncthreads();
 
     const uint16_t *kbase = kc + (size_t)kvh * max_ctx * QA_D + 8 * kg;      // K: dims 32 s + 8 kg of position ln
     const uint16_t *vbase = vc + (size_t)kvh * max_ctx * QA_D + 8 * ln;      // V: dims 8 ln (and 128 on) of 8 positions
-    const float fac = qf[ln];
+    const float fac = qf[ln].x, fac2 = qf[ln].y;
     float m = -FLT_MAX, l = 0.0f;
     qa_f4 acc[16];
 #pragma unroll
@@ -980,10 +989,10 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
         entries(j0 + 4 * QAM_STEP);                            // the next pass's, ahead of this one's values
 #pragma unroll
         for (int i = 0; i < 8; i++) v0[i] = *reinterpret_cast<const uint4 *>(vp[i]);
-        // scores: the first parts in one sum, the others in another
-        qa_f4 hi[2], lo[2];
+        // scores: the first parts in four sums, the others in another
+        qa_f4 hi[2][4], lo[2];
 #pragma unroll
-        for (int t = 0; t < 2; t++) hi[t] = lo[t] = qa_f4{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < 2; t++) hi[t][0] = hi[t][1] = hi[t][2] = hi[t][3] = lo[t] = qa_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             qa_h8 b[3];
@@ -992,7 +1001,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
 #pragma unroll
             for (int t = 0; t < 2; t++) {
                 const qa_h8 a = __builtin_bit_cast(qa_h8, kv[t][s]);
-                hi[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[0], hi[t], 0, 0, 0);
+                hi[t][s >> 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[0], hi[t][s >> 1], 0, 0, 0);
                 lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[2], lo[t], 0, 0, 0);
                 lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[1], lo[t], 0, 0, 0);
             }
@@ -1004,8 +1013,10 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int j = j0 + 16 * (i >> 2) + 4 * kg + (i & 3);
-            sc[i] = j < j_hi ? __builtin_fmaf(lo[i >> 2][i & 3], 0x1p-12f, hi[i >> 2][i & 3]) * fac : -FLT_MAX;
-            cm = fmaxf(cm, sc[i]);
+            const qa_f4 *h = hi[i >> 2];
+            sc[i] = __builtin_fmaf(lo[i >> 2][i & 3], 0x1p-12f,
+                                   (h[0][i & 3] + h[1][i & 3]) + (h[2][i & 3] + h[3][i & 3]));
+            cm = fmaxf(cm, j < j_hi ? sc[i] * fac : -FLT_MAX);
         }
         cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
         cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
@@ -1028,7 +1039,8 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             // (a select: where no score is above -FLT_MAX, neither is m)
-            const float p = j0 + 16 * (i >> 2) + 4 * kg + (i & 3) < j_hi ? qa_exp2(sc[i] - m) : 0.0f;
+            const bool in = j0 + 16 * (i >> 2) + 4 * kg + (i & 3) < j_hi;
+            const float p = in ? qa_exp2(__builtin_fmaf(sc[i], fac, __builtin_fmaf(sc[i], fac2, -m))) : 0.0f;
             l += p;
             _Float16 a, b, c;
             rem[i] = qa_split(p * QAM_P_UNIT, a, b, c);

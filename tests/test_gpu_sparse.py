@@ -741,3 +741,24 @@ def test_attn_masked_small_weights_keep_their_bits(gpu):
         for h in (0, 5, 11, 12, 23):
             e = rel_l2(got[r, h], attn64(q, kb16, vb16, lst, r, h, 1.0 / 16.0))
             assert e < (8 + leads[r]) * 2.0 ** -23, (leads[r], h, e)
+
+
+def test_attn_masked_error_no_larger_than_one_row(gpu):
+    """Against 64 bits, a call of many rows (matrix cores) is no further off
+    than the same rows one at a time (the fp32 form) where the scores' own
+    rounding decides: tens of log2 units, a few positions with the weight.
+    (With small scores the sums' rounding decides, and one row's 65 splits sum
+    in shorter chains: 2.2e-7 here, 2.0e-7 there, 4.4e-7 for the fp32 form
+    with a workgroup a row.)  Over 144 heads either figure is within 5% of what
+    other inputs give."""
+    q, kb16, vb16, lst = listed_case(2, 24, 132, 2052, 451)
+    q *= np.float32(24.0)
+    got = listed_attn(gpu, q, kb16, vb16, lst, 1.0 / 16.0)
+    many, one = [], []
+    for r in range(0, 132, 23):
+        o = listed_attn(gpu, q[r:r + 1], kb16, vb16, lst[r:r + 1], 1.0 / 16.0)[0]
+        want = np.stack([attn64(q, kb16, vb16, lst, r, h, 1.0 / 16.0) for h in range(24)])
+        many.append((got[r] - want) / np.sqrt((want ** 2).sum()))
+        one.append((o - want) / np.sqrt((want ** 2).sum()))
+    m, o = (float(np.sqrt((np.stack(e) ** 2).sum() / 6)) for e in (many, one))
+    assert m < 1.05 * o, (m, o)
