@@ -612,18 +612,26 @@ __device__ __forceinline__ float qa_f16(uint32_t bits)
 // output; otherwise its softmax state (max, sum, unnormalised output per
 // head) goes to `part` and k_attn_merge combines the splits.
 template <int G>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) k_attn_masked(float *__restrict__ out, const float *__restrict__ gate,
-                                                     const float *__restrict__ q, const uint16_t *__restrict__ kc,
-                                                     const uint16_t *__restrict__ vc, const uint32_t *__restrict__ list,
-                                                     int q_heads, int kv_heads, int max_ctx, float scale, int cap,
-                                                     int nsplit, float *__restrict__ part)
-{
+struct qa_masked_lds {
     // the G heads, pre-scaled; each 32-dim piece padded by 16 bytes so the
     // eight pieces a score reads at once start in different banks
-    __shared__ float4 qs4[G][QA_QROW];
-    __shared__ float ps[G][QA_P];                // a pass's weights (wave w: [8w, 8w + 8))
-    __shared__ float wm[4][G], wl[4][G];         // the waves' softmax states
-    __shared__ float wbuf[G][QA_D];              // the waves' partial outputs meet here
+    float4 qs4[G][QA_QROW];
+    float ps[G][QA_P];                // a pass's weights (wave w: [8w, 8w + 8))
+    float wm[4][G], wl[4][G];         // the waves' softmax states
+    float wbuf[G][QA_D];              // the waves' partial outputs meet here
+};
+
+template <int G>
+__device__ __forceinline__ void qa_masked(qa_masked_lds<G> &sh, float *__restrict__ out, const float *__restrict__ gate,
+                                          const float *__restrict__ q, const uint16_t *__restrict__ kc,
+                                          const uint16_t *__restrict__ vc, const uint32_t *__restrict__ list,
+                                          int q_heads, int kv_heads, int max_ctx, float scale, int cap,
+                                          int nsplit, float *__restrict__ part)
+{
+    auto &qs4 = sh.qs4;
+    auto &ps = sh.ps;
+    auto &wm = sh.wm, &wl = sh.wl;
+    auto &wbuf = sh.wbuf;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int split = blockIdx.x % nsplit, rk = blockIdx.x / nsplit;
     const int row = rk / kv_heads, kvh = rk % kv_heads;
@@ -842,6 +850,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
     }
 }
 
+template <int G>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) k_attn_masked(float *__restrict__ out, const float *__restrict__ gate,
+                                                     const float *__restrict__ q, const uint16_t *__restrict__ kc,
+                                                     const uint16_t *__restrict__ vc, const uint32_t *__restrict__ list,
+                                                     int q_heads, int kv_heads, int max_ctx, float scale, int cap,
+                                                     int nsplit, float *__restrict__ part)
+{
+    __shared__ qa_masked_lds<G> sh;
+    qa_masked<G>(sh, out, gate, q, kc, vc, list, q_heads, kv_heads, max_ctx, scale, cap, nsplit, part);
+}
+
 // ---- masked attention on the matrix cores -------------------------------------------
 //
 // The same split of the work (a workgroup a row, kv head and split) for many
@@ -906,8 +925,9 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
                                                     int q_heads, int kv_heads, int max_ctx, float scale, int cap,
                                                     int nsplit, float *__restrict__ part)
 {
-    constexpr int QB = 3 * QAM_HEADS * QAM_QST * 2, OB = 4 * QAM_HEADS * QAM_OST * 4;
-    __shared__ __align__(16) uint8_t lds[QB > OB ? QB : OB];
+    constexpr int QB = 3 * QAM_HEADS * QAM_QST * 2, OB = 4 * QAM_HEADS * QAM_OST * 4, MB = sizeof(qa_masked_lds<G>);
+    static_assert(MB <= OB && QB <= OB, "one place for all three");
+    __shared__ __align__(16) uint8_t lds[OB];
     __shared__ float2 qf[QAM_HEADS];                  // a head's score factor and what it lacks
     __shared__ float wm[4][QAM_HEADS], wl[4][QAM_HEADS];
     _Float16 (*qp)[QAM_HEADS][QAM_QST] = reinterpret_cast<_Float16 (*)[QAM_HEADS][QAM_QST]>(lds);
@@ -1128,6 +1148,23 @@ __global__ void __launch_bounds__(256, 2) k_attn_mx(float *__restrict__ out, con
         load_k();
         __builtin_amdgcn_sched_barrier(0);
         values(v1, 8);
+    }
+    // A key, value or query that is no finite number meets zeros and parts of
+    // either sign above, where plain arithmetic has one product: the
+    // workgroup does its share over as k_attn_masked does.  (Any of them
+    // leaves an infinity or NaN in a sum.  A dead head's sums count too: the
+    // same answer, later.)
+    {
+        float z = l * 0.0f;
+#pragma unroll
+        for (int t = 0; t < 16; t++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) z = __builtin_fmaf(acc[t][e], 0.0f, z);
+        if (__syncthreads_or(z != 0.0f)) {                     // (q is no longer read)
+            qa_masked<G>(*reinterpret_cast<qa_masked_lds<G> *>(lds), out, gate, q, kc, vc, list, q_heads, kv_heads,
+                         max_ctx, scale, cap, nsplit, part);
+            return;
+        }
     }
     // the waves' states meet
     l += __shfl_xor(l, 16, 64);

@@ -762,3 +762,39 @@ def test_attn_masked_error_no_larger_than_one_row(gpu):
         one.append((o - want) / np.sqrt((want ** 2).sum()))
     m, o = (float(np.sqrt((np.stack(e) ** 2).sum() / 6)) for e in (many, one))
     assert m < 1.05 * o, (m, o)
+
+
+@pytest.mark.parametrize("where,value", [("k", -np.inf), ("k", np.nan), ("v", np.inf), ("v", -np.inf), ("v", np.nan),
+                                         ("q", np.inf)])
+def test_attn_masked_not_finite(gpu, where, value):
+    """An infinity or NaN in a cache or a query reaches what it reaches in
+    a call of one row and no more: a key of -inf has weight 0 where q's element
+    is positive, a value's infinity stays in its dim; rows that don't list the
+    position and other kv heads are the bits they are without it.  Bar as
+    above, on O(1) values."""
+    q, kb16, vb16, lst = listed_case(2, 24, 140, 300, 441)
+    lst[:, 0] = 100 + np.arange(140)               # the position is listed from row 51 on
+    at, g, bits = 150, 1, np.float16(value).view(np.uint16)
+    clean = listed_attn(gpu, q, kb16, vb16, lst, 1.0 / 16.0)
+    if where == "k":
+        kb16[g, at, 9] = bits
+        q[:, 12:18, 9] = np.abs(q[:, 12:18, 9]) + np.float32(0.1)
+    elif where == "v":
+        vb16[g, at, 9] = bits
+    else:
+        q[100, 14, 9] = value
+    got = listed_attn(gpu, q, kb16, vb16, lst, 1.0 / 16.0)
+    if where == "v":
+        assert same_bits(got[:, :12], clean[:, :12]) and same_bits(got[:51], clean[:51])
+    for r in (0, 50, 51, 100, 139):
+        one = listed_attn(gpu, q[r:r + 1], kb16, vb16, lst[r:r + 1], 1.0 / 16.0)[0]
+        assert np.array_equal(np.isfinite(one), np.isfinite(got[r])), r
+        assert np.array_equal(one[~np.isfinite(one)], got[r][~np.isfinite(one)], equal_nan=True), r
+        for h in (0, 11, 12, 14, 17, 23):
+            want = attn64(q, kb16, vb16, lst, r, h, 1.0 / 16.0)
+            ok = np.isfinite(want)
+            if where == "v" or ok.all():
+                assert np.array_equal(got[r, h][~ok], want[~ok].astype(np.float32), equal_nan=True), (r, h)
+                assert np.abs(got[r, h][ok] - want[ok]).max() < 2e-6, (r, h)
+            else:                                  # a weight that is no number: both kernels give zeros
+                assert (got[r, h] == 0).all(), (r, h)
