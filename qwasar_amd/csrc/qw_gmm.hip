@@ -605,6 +605,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_xgemm(QxArgs a)
 // (exact); the group's map is applied to the fp32 partial:
 //   sum_i (s q_i + b) x_i = s C_g + (b - 1024 s) X_g,
 //   C_g = sum_i (1024 + q_i) x_i,   X_g = sum_i x_i.
+// It needs no scratch, so it also takes the calls, dense or grouped, that
+// would be staged but for scratch that cannot be had.
 #define QW_GMM_BN 64
 #define QW_GMM_BK 128
 #define QW_GMM_THREADS 256
@@ -618,11 +620,13 @@ struct QwGmmArgs {
     int k, n, rows, nblk;
     int kslice;      // k range of a blockIdx.y slice (k: no split)
     float *part;     // split-K: slice s writes part[s][rows][n]
+    const int32_t *perm, *tiles;
+    int K, x_by_pair;        // grouped: as in QxArgs
 };
 
 union qw_h8u { qw_h8 h; uint32_t u[4]; uint4 v; };
 
-template <int G, int BM>
+template <int G, int BM, bool GATHER>
 __global__ __launch_bounds__(QW_GMM_THREADS) void k_sgemm(QwGmmArgs a)
 {
     constexpr int MT = BM / 16;
@@ -638,13 +642,16 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_sgemm(QwGmmArgs a)
     const unsigned v = (total % 8u == 0u) ? (b % 8u) * (total / 8u) + b / 8u : b;
     const int tile = (int)(v / (unsigned)a.nblk), nb = (int)(v % (unsigned)a.nblk);
 
-    const int first = tile * BM, len = min(BM, a.rows - first);
+    if (GATHER && tile >= a.tiles[0]) return;
+    const int first = GATHER ? a.tiles[2 + 3 * tile] : tile * BM;
+    const int len = GATHER ? a.tiles[3 + 3 * tile] : min(BM, a.rows - first);
     if (len <= 0) return;
     const int k = a.k, n = a.n, words = k / 8, groups = k / G;
     const int n0 = nb * QW_GMM_BN;
     const int kb = (int)blockIdx.y * a.kslice, ke = min(k, kb + a.kslice);
-    const uint32_t *wb = a.m.w;
-    const uint16_t *sb = a.m.s, *bb = a.m.b;
+    const size_t bank = GATHER ? (size_t)a.tiles[1 + 3 * tile] * n : 0;      // the expert's first weight row
+    const uint32_t *wb = a.m.w + bank * words;
+    const uint16_t *sb = a.m.s + bank * groups, *bb = a.m.b + bank * groups;
 
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
     const int ln = lane & 15, lg = lane >> 4;
@@ -665,7 +672,8 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_sgemm(QwGmmArgs a)
             qw_h8u h;
             float bsum = 0.0f;
             if (m < len && bk * 8 < klen) {
-                const float4 *xv = reinterpret_cast<const float4 *>(a.x + (size_t)(first + m) * k + k0 + bk * 8);
+                const int p = GATHER ? a.perm[first + m] : first + m, r = GATHER && !a.x_by_pair ? p / a.K : p;
+                const float4 *xv = reinterpret_cast<const float4 *>(a.x + (size_t)r * k + k0 + bk * 8);
                 const float4 lo = xv[0], hi = xv[1];
                 const float f[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
                 _Float16 q[8];
@@ -744,7 +752,7 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_sgemm(QwGmmArgs a)
             for (int i = 0; i < 4; i++) {
                 const int m = mt * 16 + 4 * lg + i;
                 if (m < len) {
-                    yo[(size_t)(first + m) * n + col] = acc[mt][i];
+                    yo[(size_t)(GATHER ? a.perm[first + m] : first + m) * n + col] = acc[mt][i];
                 }
             }
         }
@@ -861,6 +869,23 @@ static void qx_wide(hipStream_t s, QxArgs &a, int nt, int splits)
     }
 }
 
+template <int G, bool GATHER>
+static void qs_launch_g(hipStream_t s, const QwGmmArgs &a, int bm, int ntiles, int splits)
+{
+    const dim3 grid((unsigned)(a.nblk * ntiles), (unsigned)splits), blk(QW_GMM_THREADS);
+    if (bm == 16) hipLaunchKernelGGL((k_sgemm<G, 16, GATHER>), grid, blk, 0, s, a);
+    else if (bm == 32) hipLaunchKernelGGL((k_sgemm<G, 32, GATHER>), grid, blk, 0, s, a);
+    else hipLaunchKernelGGL((k_sgemm<G, 64, GATHER>), grid, blk, 0, s, a);
+}
+
+template <bool GATHER>
+static void qs_launch(hipStream_t s, const QwGmmArgs &a, int group, int bm, int ntiles, int splits)
+{
+    if (group == 32) qs_launch_g<32, GATHER>(s, a, bm, ntiles, splits);
+    else if (group == 64) qs_launch_g<64, GATHER>(s, a, bm, ntiles, splits);
+    else qs_launch_g<128, GATHER>(s, a, bm, ntiles, splits);
+}
+
 extern "C" size_t qwk_gather_gemm_work_bytes(int k, int pairs, int K, int x_by_pair, int group)
 {
     if (k < 1 || pairs < 1 || K < 1 || group < 1) return 0;
@@ -873,7 +898,11 @@ extern "C" int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const in
 {
     if (!gmm_shape_ok(x, m, k, n, group) || K < 1 || (bm != 16 && bm != 32 && bm != 64)) return (int)hipErrorInvalidValue;
     if (max_tiles <= 0 || pairs <= 0) return 0;
-    if (!work || work_bytes < qwk_gather_gemm_work_bytes(k, pairs, K, x_by_pair, group)) return (int)hipErrorInvalidValue;
+    if (!work || ((uintptr_t)work & 15u) || work_bytes < qwk_gather_gemm_work_bytes(k, pairs, K, x_by_pair, group)) {
+        const QwGmmArgs a = {y, x, m, k, n, 0, (n + QW_GMM_BN - 1) / QW_GMM_BN, k, nullptr, perm, tiles, K, x_by_pair};
+        qs_launch<true>(s, a, group, bm, max_tiles, 1);
+        return (int)hipGetLastError();
+    }
     QxArgs a = {};
     a.y = y; a.perm = perm; a.tiles = tiles; a.w = m.w; a.s = m.s; a.b = m.b;
     a.k = k; a.n = n; a.K = K; a.x_by_pair = x_by_pair; a.kslice = k;
@@ -918,16 +947,6 @@ static int qmm_splits(int k, int n, int rows, int *kslice)
     const int ks = (int)(((k + sp - 1) / sp + QW_GMM_BK - 1) / QW_GMM_BK * QW_GMM_BK);
     *kslice = ks;
     return (k + ks - 1) / ks;
-}
-
-template <int G>
-static void qmm_small_launch(hipStream_t s, const QwGmmArgs &a, int splits)
-{
-    const int bm = qmm_bm(a.rows);
-    const dim3 grid((unsigned)(a.nblk * ((a.rows + bm - 1) / bm)), (unsigned)splits), blk(QW_GMM_THREADS);
-    if (bm == 16) hipLaunchKernelGGL((k_sgemm<G, 16>), grid, blk, 0, s, a);
-    else if (bm == 32) hipLaunchKernelGGL((k_sgemm<G, 32>), grid, blk, 0, s, a);
-    else hipLaunchKernelGGL((k_sgemm<G, 64>), grid, blk, 0, s, a);
 }
 
 static void qmm_reduce(hipStream_t s, float *y, const float *part, long total, int splits)
@@ -1034,15 +1053,13 @@ extern "C" int qwk_qmm(hipStream_t s, float *y, const float *x, qwk_q4 m, int k,
 {
     if (!gmm_shape_ok(x, m, k, n, group) || rows < 1) return (int)hipErrorInvalidValue;
     const size_t need = qwk_qmm_work_bytes(k, n, rows, group);
-    if (need > 0 && (!work || ((uintptr_t)work & 15u) || work_bytes < need)) return (int)hipErrorInvalidValue;
-    if (qmm_small(k, n, rows)) {
-        int ks;
-        const int sp = qmm_splits(k, n, rows, &ks);
+    const bool lacks = need > 0 && (!work || ((uintptr_t)work & 15u) || work_bytes < need);
+    if (lacks || qmm_small(k, n, rows)) {
+        int ks = k;
+        const int sp = lacks ? 1 : qmm_splits(k, n, rows, &ks), bm = qmm_bm(rows);
         const QwGmmArgs a = {y, x, m, k, n, rows, (n + QW_GMM_BN - 1) / QW_GMM_BN, ks,
-                             sp > 1 ? static_cast<float *>(work) : nullptr};
-        if (group == 32) qmm_small_launch<32>(s, a, sp);
-        else if (group == 64) qmm_small_launch<64>(s, a, sp);
-        else qmm_small_launch<128>(s, a, sp);
+                             sp > 1 ? static_cast<float *>(work) : nullptr, nullptr, nullptr, 1, 1};
+        qs_launch<false>(s, a, group, bm, (rows + bm - 1) / bm, sp);
         if (sp > 1) qmm_reduce(s, y, a.part, (long)rows * n, sp);
         return (int)hipGetLastError();
     }

@@ -66,7 +66,8 @@ int qwk_q4mv_multi(hipStream_t s, const float *x, int k, int group, int count,
 /* The grouped (prefill) product: per tile of pairs routed to one expert,
  * y[perm[j], :] = W_e . in(perm[j]), in(p) = x row (x_by_pair ? p : p/K).
  * Tiles were cut at `bm` rows by qwk_moe_group; `max_tiles` bounds the grid.
- * work: qwk_gather_gemm_work_bytes(...) bytes for the staged activations. */
+ * work: qwk_gather_gemm_work_bytes(...) bytes for the staged activations;
+ * with less the product runs without them, slower. */
 int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const int32_t *perm,
                     const int32_t *tiles, qwk_q4 m, int k, int n, int pairs, int E, int K, int x_by_pair,
                     int group, int bm, int max_tiles, void *work, size_t work_bytes);
@@ -76,7 +77,8 @@ int qwk_gather_gemm_blocks(int k, int n, int pairs, int E, int bm);
 
 /* Dense prefill product y[rows, n] = x[rows, k] . W^T (the shared expert). */
 /* work: qwk_qmm_work_bytes(k, n, rows, group) bytes for the staged
- * activations and the split-K partials. */
+ * activations and the split-K partials; with less the product runs unstaged
+ * and unsplit, slower. */
 int qwk_qmm(hipStream_t s, float *y, const float *x, qwk_q4 m, int k, int n, int rows, int group,
             void *work, size_t work_bytes);
 size_t qwk_qmm_work_bytes(int k, int n, int rows, int group);
@@ -277,7 +279,8 @@ int qwk_conv1d_causal_silu(hipStream_t s, float *y, const float *x, float *state
 int qwk_gdn_gates(hipStream_t s, float *g, float *beta, const float *a, const float *b,
                   const uint16_t *A_log, const uint16_t *dt_bias, int hv, int rows);
 /* prep NULL: q, k normed and g, beta given; else g and beta are unused.
- * work: qwk_gated_delta_work() bytes of device memory (NULL when that is 0):
+ * work: qwk_gated_delta_work() bytes of device memory, or NULL (when that is
+ * 0, or they cannot be had: the steps one by one, everything in the kernel):
  * a prepared call of 64 steps on computes its norms and gates there first, in
  * parallel, instead of a chunk at a time inside the recurrence; a call of 256
  * on without snapshots works in chunks of 32 steps (qw_gdn.hip) and keeps

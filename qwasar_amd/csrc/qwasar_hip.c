@@ -536,7 +536,6 @@ void qw_op_qmm_q4(qw_cmd c, qw_ref y, qw_ref x, qw_ref w, qw_ref scales, qw_ref 
     touch(c, x, 0); touch(c, w, 0); touch(c, scales, 0); touch(c, biases, 0); touch(c, y, 1);
     const size_t wb = qwk_qmm_work_bytes(k, n, rows, group);
     void *work = wb ? scratch(wb) : NULL;
-    if (wb && !work) { cmd_fail(c, hipErrorOutOfMemory, "qmm_q4: scratch of %zu bytes", wb); return; }
     launched(c, "qmm_q4", qwk_qmm(G.stream, dp(y), dp(x), q4(w, scales, biases), k, n, rows, group, work,
                                   work ? wb : 0));
 }
@@ -863,10 +862,9 @@ void qw_op_qmm_q4_gather(qw_cmd c, qw_ref y, qw_ref x, qw_ref perm, qw_ref tiles
     const int32_t bm = qw_moe_tile_rows(pairs, E);
     const size_t wb = qwk_gather_gemm_work_bytes(k, pairs, K, x_by_pair ? 1 : 0, group);
     void *work = wb ? scratch(wb) : NULL;
-    if (wb && !work) { cmd_fail(c, hipErrorOutOfMemory, "qmm_q4_gather: scratch of %zu bytes", wb); return; }
     launched(c, "qmm_q4_gather", qwk_gather_gemm(G.stream, dp(y), dp(x), dp(perm), dp(tiles),
                                                  q4(w, scales, biases), k, n, pairs, E, K, x_by_pair ? 1 : 0,
-                                                 group, bm, tiles_for(pairs, E, bm), work, wb));
+                                                 group, bm, tiles_for(pairs, E, bm), work, work ? wb : 0));
 }
 
 /* ---- the whole MoE layer ------------------------------------------------------ */
@@ -877,7 +875,11 @@ static void *scratch(size_t bytes) {
     if (G.scratch) hipFree(G.scratch);
     G.scratch = NULL;
     G.scratch_len = 0;
-    if (hipMalloc(&G.scratch, bytes) != hipSuccess) return NULL;
+    if (hipMalloc(&G.scratch, bytes) != hipSuccess) {
+        (void)hipGetLastError();   /* the caller may do without: no error of its launches */
+        G.scratch = NULL;
+        return NULL;
+    }
     G.scratch_len = bytes;
     return G.scratch;
 }
@@ -1212,7 +1214,6 @@ static void gated_delta(qw_cmd c, qw_ref y, qw_ref q, qw_ref k, qw_ref v, qw_ref
     }
     const size_t wb = qwk_gated_delta_work(hk, hv, rows, prep != NULL, n_snap > 0 ? n_snap : 0);
     void *work = wb ? scratch(wb) : NULL;
-    if (wb && !work) { cmd_fail(c, hipErrorOutOfMemory, "gated_delta: scratch of %zu bytes", wb); return; }
     launched(c, prep ? "gated_delta_prep" : "gated_delta",
              qwk_gated_delta(G.stream, dp(y), dp(q), dp(k), dp(v), dp(g), dp(beta), dp(state), hk, hv, dk, dv, rows,
                              n_snap > 0 ? dp(snap) : NULL, n_snap, snap_stride, prep ? &pp : NULL, work));
