@@ -169,10 +169,11 @@ struct QxArgs {
 // 16 bytes a lane from its own address straight into LDS at lds + 16 lane.
 // Written as asm because the compiler, which cannot tell the ring's stages
 // apart, waits for every such load before any LDS read; the waits on the
-// vector memory counter in k_xgemm are this kernel's own.
+// vector memory counter in k_xgemm are this kernel's own.  (m0 is an operand, so
+// the compiler knows of it; the instruction may not follow its write at once.)
 __device__ __forceinline__ void qx_dma(uint32_t lds, const void *src)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(src) : "memory");
 }
 
 template <int N>

@@ -209,8 +209,8 @@ typedef float qr_f16v __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ void qd_dma(uint32_t lds, const void *src)
 {
     // (asm: the compiler would wait for every such load before any LDS read;
-    // the kernel's own waits follow)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+    // the kernel's own waits follow.  m0 is an operand, so that it knows of it)
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(src) : "memory");
 }
 template <int RT>
 __global__ __launch_bounds__(256, 1) void k_dmat_mfma(float *__restrict__ y, const float *__restrict__ x,
