@@ -576,6 +576,20 @@ def test_gated_delta_prep_chunks(gpu, hk, hv, rows):
     wy, ws, _ = sparse.gated_delta_prep(q, k, v, a, b, Al, dt, eps, qs, ks, s0, hk, hv, dk, dv, rows)
     for yb, sb in ((y1, s1), (y2, s2)):
         assert rel_l2(yb.read(np.float32, v.shape), wy) < 5e-6 and rel_l2(sb.read(np.float32, s0.shape), ws) < 5e-6
+    # the call with a snapshot: the bits of a first step and two calls under 256 steps
+    s3, y3, t0 = B.of(s0), B(v.nbytes), 0
+    for n in (1, rows // 2, rows - 1 - rows // 2):
+        off = lambda a: a[t0].nbytes * t0
+        p3 = gpu.qw_gdn_prep(ab.ref(off(a)), bb.ref(off(b)), Ab.ref(), db.ref(), eps, qs, ks)
+        c = gpu.qw_cmd_begin()
+        gpu.qw_op_gated_delta_prep(c, y3.ref(off(v)), qb.ref(off(q)), kb.ref(off(k)), vb.ref(off(v)), p3, s3.ref(), hk,
+                                   hv, dk, dv, n, gpu.NULL_REF, 0, 0)
+        gpu.run(c, "gated delta prep, short calls")
+        if t0 == 0:
+            assert same_bits(snap.read(np.float32, s0.shape), s3.read(np.float32, s0.shape)), "the snapshot"
+        t0 += n
+    assert same_bits(y2.read(np.float32, v.shape), y3.read(np.float32, v.shape))
+    assert same_bits(s2.read(np.float32, s0.shape), s3.read(np.float32, s0.shape))
 
 
 # ---- masked attention on the matrix cores (8 query heads a kv head on) ---------------------
