@@ -615,41 +615,38 @@ __device__ __forceinline__ void qg_sync()
 // Wave w of four: rows (w & 1) 16 .. of the chunk, of K for waves 0 and 1
 // (which make U) and of Q for 2 and 3 (which make Y); and columns 32 w .. of
 // the state, as D tiles of S' (k rows, v columns), so that a lane's four are
-// a 16-byte piece of S[v][k].  QG_VT tiles of 16 value rows a workgroup: with
-// one, two workgroups share a CU and cover each other's barriers (2048 steps:
-// 243 us; with two, 316).
-#define QG_VT 1
+// a 16-byte piece of S[v][k].  16 value rows a workgroup, so that two share a
+// CU and cover each other's barriers.  (32 rows, one a CU, before infinities
+// were kept apart: 2048 steps 316 us against 243.)
 __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restrict__ y, const float *__restrict__ v,
                                                       float *state, int hk, int hv, int rows)
 {
-    __shared__ __align__(16) float Ss[16 * QG_VT][QG_CS], Ks[QG_C][QG_CS];
-    __shared__ __align__(16) float Rt[16 * QG_VT][QG_TS], Ut[16 * QG_VT][QG_TS], Up[16 * QG_VT][QG_TS];
-    __shared__ int bad[2][16 * QG_VT];       // by the chunk's parity
+    __shared__ __align__(16) float Ss[16][QG_CS], Ks[QG_C][QG_CS];
+    __shared__ __align__(16) float Rt[16][QG_TS], Ut[16][QG_TS], Up[16][QG_TS];
+    __shared__ int bad[2][16];       // by the chunk's parity
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 15, kg = lane >> 4;
     // the workgroups of a key head (which read its q and k) on one XCD
-    constexpr unsigned per = QG_DV / (16 * QG_VT);
+    constexpr unsigned per = QG_DV / 16;
     const unsigned total = gridDim.x, b = blockIdx.x;
     const unsigned id = total % 8u == 0u ? (b % 8u) * (total / 8u) + b / 8u : b;
-    const int h = (int)(id / per), v0 = 16 * QG_VT * (int)(id % per), hx = h / (hv / hk);
+    const int h = (int)(id / per), v0 = 16 * (int)(id % per), hx = h / (hv / hk);
     const int nch = (rows + QG_C - 1) / QG_C, t0 = 16 * (wave & 1);
     const bool isq = wave >= 2;
 
     float *sp = state + ((size_t)h * QG_DV + v0 + ln) * QG_DK + 32 * wave + 4 * kg;
-    qg_f4 S[QG_VT][2];
+    qg_f4 S[2];
 #pragma unroll
-    for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            S[z][u] = *reinterpret_cast<const qg_f4 *>(sp + z * 16 * QG_DK + 16 * u);
-            *reinterpret_cast<qg_f4 *>(&Ss[16 * z + ln][32 * wave + 16 * u + 4 * kg]) = S[z][u];
-        }
+    for (int u = 0; u < 2; u++) {
+        S[u] = *reinterpret_cast<const qg_f4 *>(sp + 16 * u);
+        *reinterpret_cast<qg_f4 *>(&Ss[ln][32 * wave + 16 * u + 4 * kg]) = S[u];
+    }
     // a chunk's operands, fetched a chunk ahead: 16 rows of K or Q, the rows'
     // scalars, T or the masked Q K' and (waves 0 and 1) V
     const float4 *kq = reinterpret_cast<const float4 *>(isq ? w.qn : w.kn) + ((size_t)hx * nch * 16 + t0 / 2) * 64 + lane;
     const float4 *tq = reinterpret_cast<const float4 *>(isq ? w.QK : w.T) + ((size_t)h * nch * 4 + t0 / 8) * 64 + lane;
     const float4 *sc = w.sc + (size_t)h * nch * QG_C + t0 + 4 * kg;
     float4 fa[8], ft[2], fs[4];
-    float fv[QG_VT][4] = {}, fg;
+    float fv[4] = {}, fg;
     auto fetch = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 8; j++) fa[j] = kq[((size_t)c * 16 + j) * 64];
@@ -660,19 +657,17 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
         if (!isq) {
 #pragma unroll
             for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int z = 0; z < QG_VT; z++)
-                    fv[z][e] = v[((size_t)min(c * QG_C + t0 + 4 * kg + e, rows - 1) * hv + h) * QG_DV + v0 + 16 * z + ln];
+                fv[e] = v[((size_t)min(c * QG_C + t0 + 4 * kg + e, rows - 1) * hv + h) * QG_DV + v0 + ln];
         }
         fg = w.sc[((size_t)h * nch + c) * QG_C + QG_C - 1].z;     // G[C - 1]
     };
-    if (tid < 32 * QG_VT) (&bad[0][0])[tid] = QG_C;
+    if (tid < 32) (&bad[0][0])[tid] = QG_C;
     auto finite = [](float x) { return (__float_as_uint(x) & 0x7F800000u) != 0x7F800000u; };
     fetch(0);
     qg_sync();
     for (int c = 0; c < nch; c++) {
         float4 a[8], tm[2], s4[4];
-        float vv[QG_VT][4];
+        float vv[4];
 #pragma unroll
         for (int j = 0; j < 8; j++) a[j] = fa[j];
 #pragma unroll
@@ -680,8 +675,7 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             s4[e] = fs[e];
-#pragma unroll
-            for (int z = 0; z < QG_VT; z++) vv[z][e] = fv[z][e];
+            vv[e] = fv[e];
         }
         const float gc = fg;
         if (c + 1 < nch) fetch(c + 1);
@@ -691,115 +685,86 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
         }
         // K S0' or Q S0': eight chains a tile, met in a tree (here and below a
         // long chain, or one that starts on a large value, rounds more than the serial form)
-        qg_f4 d[QG_VT];
+        qg_f4 d;
         {
-            qg_f4 dd[QG_VT][8];
-            float4 sb[QG_VT][8];
+            qg_f4 dd[8];
+            float4 sb[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++)
-#pragma unroll
-                for (int z = 0; z < QG_VT; z++)
-                    sb[z][j] = *reinterpret_cast<const float4 *>(&Ss[16 * z + ln][16 * j + 4 * kg]);
+            for (int j = 0; j < 8; j++) sb[j] = *reinterpret_cast<const float4 *>(&Ss[ln][16 * j + 4 * kg]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-                for (int j = 0; j < 8; j++) dd[z][j] = qg_f4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < 8; j++) dd[j] = qg_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int j = 0; j < 8; j++)
 #pragma unroll
                 for (int e = 0; e < 4; e++)
+                    dd[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&a[j])[e],
+                                                                 reinterpret_cast<const float *>(&sb[j])[e], dd[j], 0, 0, 0);
 #pragma unroll
-                    for (int z = 0; z < QG_VT; z++)
-                        dd[z][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&a[j])[e],
-                                                                       reinterpret_cast<const float *>(&sb[z][j])[e],
-                                                                       dd[z][j], 0, 0, 0);
-#pragma unroll
-            for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    d[z][e] = ((dd[z][0][e] + dd[z][1][e]) + (dd[z][2][e] + dd[z][3][e])) +
-                              ((dd[z][4][e] + dd[z][5][e]) + (dd[z][6][e] + dd[z][7][e]));
+            for (int e = 0; e < 4; e++)
+                d[e] = ((dd[0][e] + dd[1][e]) + (dd[2][e] + dd[3][e])) +
+                       ((dd[4][e] + dd[5][e]) + (dd[6][e] + dd[7][e]));
         }
         if (!isq) {
+            qg_f4 r;
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++) {
-                qg_f4 r;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const bool in = c * QG_C + t0 + 4 * kg + e < rows;
-                    r[e] = in ? __builtin_fmaf(s4[e].x, vv[z][e], -(s4[e].y * d[z][e])) : 0.0f;
-                }
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    if (!finite(r[e])) {
-                        atomicMin(&bad[c & 1][16 * z + ln], t0 + 4 * kg + e);
-                        r[e] = 0.0f;
-                    }
-                *reinterpret_cast<qg_f4 *>(&Rt[16 * z + ln][t0 + 4 * kg]) = r;
+            for (int e = 0; e < 4; e++) {
+                const bool in = c * QG_C + t0 + 4 * kg + e < rows;
+                r[e] = in ? __builtin_fmaf(s4[e].x, vv[e], -(s4[e].y * d[e])) : 0.0f;
             }
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (!finite(r[e])) {
+                    atomicMin(&bad[c & 1][ln], t0 + 4 * kg + e);
+                    r[e] = 0.0f;
+                }
+            *reinterpret_cast<qg_f4 *>(&Rt[ln][t0 + 4 * kg]) = r;
         }
         qg_sync();
         // X over the chunk's 32 steps against T's or the masked Q K's 16 rows (upper right tile zero)
-        auto over = [&](const float (*X)[QG_TS], qg_f4 (&o)[QG_VT]) __attribute__((always_inline)) {
-            float4 x0[QG_VT], x1[QG_VT];
+        auto over = [&](const float (*X)[QG_TS], qg_f4 &o) __attribute__((always_inline)) {
+            const float4 x0 = *reinterpret_cast<const float4 *>(&X[ln][4 * kg]);
+            const float4 x1 = *reinterpret_cast<const float4 *>(&X[ln][16 + 4 * kg]);
+            qg_f4 p[4];
+            p[0] = p[1] = p[2] = p[3] = qg_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++) {
-                x0[z] = *reinterpret_cast<const float4 *>(&X[16 * z + ln][4 * kg]);
-                x1[z] = *reinterpret_cast<const float4 *>(&X[16 * z + ln][16 + 4 * kg]);
+            for (int e = 0; e < 4; e++) {
+                p[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&tm[0])[e],
+                                                                reinterpret_cast<const float *>(&x0)[e], p[e & 1], 0, 0, 0);
+                if (t0)
+                    p[2 + (e & 1)] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&tm[1])[e],
+                                                                          reinterpret_cast<const float *>(&x1)[e],
+                                                                          p[2 + (e & 1)], 0, 0, 0);
             }
-            qg_f4 p[QG_VT][4];
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++) p[z][0] = p[z][1] = p[z][2] = p[z][3] = qg_f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int z = 0; z < QG_VT; z++) {
-                    p[z][e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&tm[0])[e],
-                                                                       reinterpret_cast<const float *>(&x0[z])[e], p[z][e & 1], 0, 0, 0);
-                    if (t0)
-                        p[z][2 + (e & 1)] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&tm[1])[e],
-                                                                                 reinterpret_cast<const float *>(&x1[z])[e],
-                                                                                 p[z][2 + (e & 1)], 0, 0, 0);
-                }
-#pragma unroll
-            for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) o[z][e] += (p[z][0][e] + p[z][1][e]) + (p[z][2][e] + p[z][3][e]);
+            for (int e = 0; e < 4; e++) o[e] += (p[0][e] + p[1][e]) + (p[2][e] + p[3][e]);
         };
-        if (tid >= 256 - 16 * QG_VT) bad[(c + 1) & 1][tid - (256 - 16 * QG_VT)] = QG_C;   // the next chunk's
+        if (tid >= 240) bad[(c + 1) & 1][tid - 240] = QG_C;   // the next chunk's
         if (!isq) {
             // U = T R
-            qg_f4 u[QG_VT];
-#pragma unroll
-            for (int z = 0; z < QG_VT; z++) u[z] = qg_f4{0.f, 0.f, 0.f, 0.f};
+            qg_f4 u = {0.f, 0.f, 0.f, 0.f};
             over(Rt, u);
+            qg_f4 up;
+            const int fb = bad[c & 1][ln];
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++) {
-                qg_f4 up;
-                const int fb = bad[c & 1][16 * z + ln];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int t = t0 + 4 * kg + e;
-                    if (t >= fb) u[z][e] = __builtin_nanf("");
-                    up[e] = u[z][e] * s4[e].w;
-                    if (!finite(u[z][e])) {
-                        atomicMin(&bad[c & 1][16 * z + ln], t);
-                        u[z][e] = 0.0f;
-                    }
+            for (int e = 0; e < 4; e++) {
+                const int t = t0 + 4 * kg + e;
+                if (t >= fb) u[e] = __builtin_nanf("");
+                up[e] = u[e] * s4[e].w;
+                if (!finite(u[e])) {
+                    atomicMin(&bad[c & 1][ln], t);
+                    u[e] = 0.0f;
                 }
-                *reinterpret_cast<qg_f4 *>(&Ut[16 * z + ln][t0 + 4 * kg]) = u[z];
-                *reinterpret_cast<qg_f4 *>(&Up[16 * z + ln][t0 + 4 * kg]) = up;
             }
+            *reinterpret_cast<qg_f4 *>(&Ut[ln][t0 + 4 * kg]) = u;
+            *reinterpret_cast<qg_f4 *>(&Up[ln][t0 + 4 * kg]) = up;
         }
         qg_sync();
         // S' = G[C-1] S0' + K' (P U)
         {
-            float4 bu[QG_VT][2], ka[2][2];
+            float4 bu[2], ka[2][2];
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-                for (int i = 0; i < 2; i++) bu[z][i] = *reinterpret_cast<const float4 *>(&Up[16 * z + ln][16 * i + 4 * kg]);
+            for (int i = 0; i < 2; i++) bu[i] = *reinterpret_cast<const float4 *>(&Up[ln][16 * i + 4 * kg]);
 #pragma unroll
             for (int u = 0; u < 2; u++)
 #pragma unroll
@@ -807,9 +772,8 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
                     const int kc = 32 * wave + 16 * u + ln, r = 16 * i + 4 * kg;
                     ka[u][i] = make_float4(Ks[r][kc], Ks[r + 1][kc], Ks[r + 2][kc], Ks[r + 3][kc]);
                 }
-            qg_f4 ds[QG_VT][2];
-#pragma unroll
-            for (int z = 0; z < QG_VT; z++) ds[z][0] = ds[z][1] = qg_f4{0.f, 0.f, 0.f, 0.f};
+            qg_f4 ds[2];
+            ds[0] = ds[1] = qg_f4{0.f, 0.f, 0.f, 0.f};
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < 2; i++)
@@ -817,45 +781,33 @@ __global__ void __launch_bounds__(256, 2) k_gdn_chunk(qg_long w, float *__restri
                 for (int e = 0; e < 4; e++)
 #pragma unroll
                     for (int u = 0; u < 2; u++)
+                        ds[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&ka[u][i])[e],
+                                                                     reinterpret_cast<const float *>(&bu[i])[e],
+                                                                     ds[u], 0, 0, 0);
 #pragma unroll
-                        for (int z = 0; z < QG_VT; z++)
-                            ds[z][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float *>(&ka[u][i])[e],
-                                                                           reinterpret_cast<const float *>(&bu[z][i])[e],
-                                                                           ds[z][u], 0, 0, 0);
+            for (int u = 0; u < 2; u++)
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-                for (int u = 0; u < 2; u++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) S[z][u][e] = __builtin_fmaf(S[z][u][e], gc, ds[z][u][e]);
+                for (int e = 0; e < 4; e++) S[u][e] = __builtin_fmaf(S[u][e], gc, ds[u][e]);
         }
         if (isq) {
             // Y = G Q S0' + (P o Q K') U
-            qg_f4 o[QG_VT];
+            qg_f4 o;
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) o[z][e] = s4[e].z * d[z][e];
+            for (int e = 0; e < 4; e++) o[e] = s4[e].z * d[e];
             over(Ut, o);
 #pragma unroll
-            for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int t = c * QG_C + t0 + 4 * kg + e;
-                    const float yv = t0 + 4 * kg + e >= bad[c & 1][16 * z + ln] ? __builtin_nanf("") : o[z][e];
-                    if (t < rows) y[((size_t)t * hv + h) * QG_DV + v0 + 16 * z + ln] = yv;
-                }
+            for (int e = 0; e < 4; e++) {
+                const int t = c * QG_C + t0 + 4 * kg + e;
+                const float yv = t0 + 4 * kg + e >= bad[c & 1][ln] ? __builtin_nanf("") : o[e];
+                if (t < rows) y[((size_t)t * hv + h) * QG_DV + v0 + ln] = yv;
+            }
         }
 #pragma unroll
-        for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-            for (int u = 0; u < 2; u++) *reinterpret_cast<qg_f4 *>(&Ss[16 * z + ln][32 * wave + 16 * u + 4 * kg]) = S[z][u];
+        for (int u = 0; u < 2; u++) *reinterpret_cast<qg_f4 *>(&Ss[ln][32 * wave + 16 * u + 4 * kg]) = S[u];
         qg_sync();
     }
 #pragma unroll
-    for (int z = 0; z < QG_VT; z++)
-#pragma unroll
-        for (int u = 0; u < 2; u++) *reinterpret_cast<qg_f4 *>(sp + z * 16 * QG_DK + 16 * u) = S[z][u];
+    for (int u = 0; u < 2; u++) *reinterpret_cast<qg_f4 *>(sp + 16 * u) = S[u];
 }
 
 // ---- launchers ----------------------------------------------------------------
@@ -938,7 +890,7 @@ extern "C" int qwk_gated_delta(hipStream_t s, float *y, const float *q, const fl
                 hipLaunchKernelGGL(k_gdn_chunk_pre<false>, pre, dim3(256), 0, s, w, q + oq, k + oq, g + og, beta + og,
                                    hk, hv, r, pp);
             }
-            hipLaunchKernelGGL(k_gdn_chunk, dim3(hv * (QG_DV / (16 * QG_VT))), dim3(256), 0, s, w, y + ov, v + ov, state, hk, hv, r);
+            hipLaunchKernelGGL(k_gdn_chunk, dim3(hv * (QG_DV / 16)), dim3(256), 0, s, w, y + ov, v + ov, state, hk, hv, r);
         }
         return (int)hipGetLastError();
     }
