@@ -395,8 +395,8 @@ __global__ void __launch_bounds__(QG_THREADS) k_gated_delta(float *__restrict__ 
 // a workgroup 16 value rows of a head, every product on the fp32 matrix cores
 // (v_mfma_f32_16x16x4_f32: fp32 inputs and sums, as the serial form).
 // 2048 steps of 16 key and 48 value heads: 10 + 590 us serial (70 vector
-// operations a step on the CUs that hold two workgroups), 39 + 268 here; the
-// call with conv and output gate 690 -> 370.  Error against 64 bits over calls
+// operations a step on the CUs that hold two workgroups), 39 + 264 here; the
+// call with conv and output gate 690 -> 363.  Error against 64 bits over calls
 // of 600 and 2048 steps: y 1.50 to 1.51e-7 serial, 1.48 to 1.51e-7 here, the
 // state 1.19 to 1.33e-7 and 1.09 to 1.22e-7.  That takes short chains from zero
 // met in trees, and the norms' factors and the gates' products in 64 bits
@@ -409,7 +409,7 @@ __global__ void __launch_bounds__(QG_THREADS) k_gated_delta(float *__restrict__ 
 // of T and Q K' above the diagonal, so a value row's first step with one is
 // kept (`bad`): R and U are zero from there on as operands of those products,
 // and the row's outputs from there on are NaN, its state what it comes to
-// (34 us of the 268).
+// (34 us of the 264).
 #define QG_C 32
 #define QG_LONG_MIN_ROWS 256     // below, the serial kernel (and its bits) stay
 #define QG_LONG_ROWS 4096        // steps a pair of launches takes: bounds the scratch

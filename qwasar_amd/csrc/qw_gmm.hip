@@ -20,8 +20,12 @@
 // and the second sum is a product of its own: the biases (bf16, as stored)
 // against X_g cut into three bf16 parts (24 bits: exactly), 16 groups' parts
 // in two bf16 MFMAs.  So the weights enter with no rounding at all;
-// activations are rounded to f16 (relative error <= 2^-11 an element), the
-// only approximation.
+// activations are rounded to f16, the only approximation: a relative error of
+// 2^-11 for elements down to 2^-29 of their row's largest (even positions) or
+// 2^-25 (odd ones), and 2^-39 (2^-35) of that largest below.  (Unscaled f16,
+// which small products still take, has 2^-11 from 2^-14 on, whatever the row:
+// finer for odd elements of rows whose largest is above 2^11, and nothing
+// above 65504.)
 //
 // k order within an MFMA.  The masks leave a word's nibbles in register order
 // 0,4,1,5,2,6,3,7; the stage stores every 8-element block in that order.
