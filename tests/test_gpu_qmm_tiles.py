@@ -3,7 +3,8 @@ column remainders of every tile height, k that is no whole number of stages
 (of 64, 128 or 256) or of 16-group blocks, split k, scale rows that come as
 one flat copy, 8 groups a load or one by one (group counts past what LDS
 holds, banks off a 16-byte boundary, odd group counts), and inputs whose
-magnitude or layout the staging has to survive.
+magnitude or layout the staging has to survive.  (Each form of the plan by
+name, unsplit and reloaded ones too: test_gpu_qmm_plans.py.)
 
 Bar: the weights enter exactly and the activations carry one f16 rounding
 (relative 2^-11 at most, 2^-13 rms), so rel-L2 against the fp32 oracle is
@@ -35,15 +36,15 @@ def put(gpu, a, off):
 
 @pytest.mark.parametrize("rows,k,n,G,off", [
     (129, 1088, 1090, 64, 0),     # one row past a tile, 17 groups (odd: one by one), ragged columns
-    (65, 3136, 1000, 64, 0),      # 49 groups: more than a wide tile's LDS holds, no whole stage
-    (300, 3328, 640, 64, 0),      # 52 groups, a multiple of 4
-    (257, 4096, 512, 64, 0),      # 64 groups: 8 a load, reloaded
+    (65, 3136, 1000, 64, 0),      # 49 groups in slices of 8: one by one, the last slice one group
+    (300, 3328, 640, 64, 0),      # 52 groups, a multiple of 4, in slices of 8
+    (257, 4096, 512, 64, 0),      # 64 groups in eight slices, flat; one row past a tile
     (200, 4096, 900, 128, 0),     # groups of 128
-    (140, 2080, 1030, 32, 0),     # groups of 32, 65 of them, k % 64 = 32
+    (140, 2080, 1030, 32, 0),     # groups of 32, 65 of them, k % 64 = 32, one by one
     (16, 6144, 3000, 64, 0),      # one 16-row tile, flat scales
-    (9, 8192, 4096, 32, 0),       # 256 groups of 32
-    (17, 6144, 3072, 64, 0),      # 32-row tile
-    (40, 6176, 1500, 32, 0),      # 64-row tile, k % 128 = 32
+    (9, 8192, 4096, 32, 0),       # 256 groups of 32, 8 a load, slices of 32
+    (17, 6144, 3072, 64, 0),      # 32-row tile, 8 a load
+    (40, 6176, 1500, 32, 0),      # two 32-row tiles, k % 128 = 32
     (130, 3072, 700, 64, 2),      # scales and biases 2 bytes off: one by one
     (48, 3072, 2000, 64, 8),      # and 8 bytes off
     (300, 12288, 320, 64, 0),     # split k
