@@ -209,13 +209,13 @@ __global__ void __launch_bounds__(QS_THREADS) __attribute__((amdgpu_waves_per_eu
 // 4.1 here.  What bounds it: many rows, the fp32 MFMA's issue (35 cycles each,
 // 60 of the 102) and the staging between groups of rows; one row, the trip to
 // memory.
-#define QM_ROWS 32
+#define QM_ROWS 32                                 // the most rows a workgroup walks
 #define QM_GROUP 8                                 // rows staged at once
 template <int D, bool POOLED, int TB, int NW, bool ONE>
 __global__ void __launch_bounds__(64 * NW, ONE ? 1 : 2) k_qsa_scores_mx(
     float *__restrict__ scores, const float *__restrict__ qn, const float *__restrict__ src,
     const uint16_t *__restrict__ kw, const float *__restrict__ inv_freq, int rows, int nq, int d, int ratio,
-    int base_pos, int max_blocks, float eps)
+    int base_pos, int max_blocks, float eps, int wg_rows)
 {
     typedef float f4v __attribute__((ext_vector_type(4)));
     static_assert(POOLED || (16 * TB * NW == QS_BLK && 64 * NW == QS_THREADS), "direct keys: qs_keys_to_lds's workgroup");
@@ -224,8 +224,8 @@ __global__ void __launch_bounds__(64 * NW, ONE ? 1 : 2) k_qsa_scores_mx(
     __shared__ float4 lds4[LN / 4 + 1];
     float *lds = reinterpret_cast<float *>(lds4);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 15, kg = lane >> 4;
-    const int b0 = blockIdx.x * (16 * TB * NW), r0 = blockIdx.y * QM_ROWS;
-    const int rend = min(r0 + QM_ROWS, rows), wb = b0 + wave * 16 * TB;
+    const int b0 = blockIdx.x * (16 * TB * NW), r0 = blockIdx.y * wg_rows;
+    const int rend = min(r0 + wg_rows, rows), wb = b0 + wave * 16 * TB;
     const int nb_hi = (base_pos + rend) / ratio;
     if (nb_hi <= b0) return;                                   // uniform
     const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1301,16 +1301,29 @@ static int qs_launch_scores(hipStream_t s, float *scores, const float *qn, const
     const int D = d <= 64 ? 64 : d <= 128 ? 128 : d <= 192 ? 192 : 256;
     if (nq <= 16 && D <= 128) {
         // one row of stored keys: a wave a workgroup, so that 8192 blocks are
-        // 512 workgroups; from 64 rows on two tiles a wave share a row's heads
-        const unsigned gy = (unsigned)((rows + QM_ROWS - 1) / QM_ROWS);
+        // 512 workgroups.  More rows, stored keys: two tiles a wave share a
+        // row's heads where workgroups of 32 rows fill the chip's 512 places,
+        // else one, over the most rows that fill them.  Keys made here (half
+        // of a short workgroup's time): the fewest rows that go in one round.
+        // us, the K = 1 form / 32 rows and two tiles from 64 rows on / this:
+        //   stored  64 rows,  512 blocks 35 / 54 / 12    made here 53 / 56 / 31
+        //          256       2048        37 / 55 / 30              54 / 57 / 47
+        //          512       4096       114 / 91 / 91             165 / 167 / 167
+        const int gx1 = (blocks + 63) / 64, gx2 = (blocks + 127) / 128;
+        auto fill = [&](int gx, int r) { return (long)gx * rows >= 512L * r; };
+        auto fits = [&](int r) { return (long)gx1 * ((rows + r - 1) / r) <= 512; };
+        const bool two = POOLED && (long)gx2 * ((rows + 31) / 32) >= 512;
+        const int wr = POOLED ? two || fill(gx1, 32) ? QM_ROWS : fill(gx1, 16) ? 16 : QM_GROUP
+                              : fits(8) ? QM_GROUP : fits(16) ? 16 : QM_ROWS;
+        const unsigned gy = (unsigned)((rows + wr - 1) / wr);
 #define QS_MX(DD, TB, NW, ONE)                                                                                         \
     hipLaunchKernelGGL((k_qsa_scores_mx<DD, POOLED, TB, NW, ONE>), dim3((blocks + 16 * TB * NW - 1) / (16 * TB * NW), gy), \
-                       dim3(64 * NW), 0, s, scores, qn, src, kw, inv_freq, rows, nq, d, ratio, base_pos, max_blocks, eps)
+                       dim3(64 * NW), 0, s, scores, qn, src, kw, inv_freq, rows, nq, d, ratio, base_pos, max_blocks, eps, wr)
 #define QS_MXD(DD)                                                                                                     \
     if constexpr (POOLED) {                                                                                            \
         if (rows == 1) QS_MX(DD, 1, 1, true);                                                                          \
-        else if (rows < 64) QS_MX(DD, 1, 4, false);                                                                    \
-        else QS_MX(DD, 2, 4, false);                                                                                   \
+        else if (two) QS_MX(DD, 2, 4, false);                                                                          \
+        else QS_MX(DD, 1, 4, false);                                                                                   \
     } else {                                                                                                           \
         if (rows == 1) QS_MX(DD, 1, 4, true);                                                                          \
         else QS_MX(DD, 1, 4, false);                                                                                   \

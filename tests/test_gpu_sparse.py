@@ -652,9 +652,9 @@ def test_attn_masked_matrix_cores_ranges(gpu):
 
 @pytest.mark.parametrize("nq,d,base,rows", [(16, 128, 900, 75), (7, 96, 3, 130)])
 def test_qsa_scores_many_rows_match_rowwise(gpu, nq, d, base, rows):
-    """From 64 rows on a wave scores two tiles of 16 blocks: the bits of one
-    row at a time (a wave a tile), at the first, a middle and the last rows;
-    blocks that end inside a tile, fewer heads than a tile's rows."""
+    """Many rows over few blocks: the bits of one row at a time, at the first,
+    a middle and the last rows; blocks that end inside a tile, fewer heads than
+    a tile's rows."""
     ratio = 4
     mb = (base + rows) // ratio + 3
     kw = FX["k_norm"] if d == 128 else synth.to_bf16(1.0 + 0.1 * rnd(d, d + nq))
@@ -666,6 +666,29 @@ def test_qsa_scores_many_rows_match_rowwise(gpu, nq, d, base, rows):
             nb = (base + r + 1) // ratio
             assert same_bits(got[r, :nb], one[0, :nb]), f"row {r}"
             assert np.isnan(got[r, nb:]).all()
+
+
+@pytest.mark.parametrize("rows,blocks,nq,pooled", [
+    (35, 700, 16, True),       # 8 rows a workgroup
+    (130, 5003, 16, True),     # 16
+    (100, 11001, 12, True),    # 32
+    (521, 4030, 16, True),     # 32, two tiles a wave
+    (35, 700, 16, False),      # 8, keys made in the kernel
+    (41, 8099, 12, False),     # 16
+    (100, 8099, 16, False),    # 32
+])
+def test_qsa_scores_workgroup_rows_match_rowwise(gpu, rows, blocks, nq, pooled):
+    """Every number of rows a workgroup walks, on both sides of its edges: the
+    bits of one row at a time, the last blocks' causal edge among them."""
+    d, ratio = 128, 4
+    base = blocks * ratio - rows
+    qn, ik, inv = rnd((rows, nq, d), 81), rnd((blocks * ratio, d), 82), rope_inv()
+    got, _ = gpu_scores(gpu, qn, ik, FX["k_norm"], inv, rows, nq, d, ratio, base, blocks, pooled=pooled)
+    for r in sorted({0, 7, 8, 15, 16, 31, 32, 33, rows - 1}):
+        one, _ = gpu_scores(gpu, qn[r:r + 1], ik, FX["k_norm"], inv, 1, nq, d, ratio, base + r, blocks, pooled=pooled)
+        nb = (base + r + 1) // ratio
+        assert same_bits(got[r, :nb], one[0, :nb]), f"row {r}"
+        assert np.isnan(got[r, nb:]).all()
 
 
 def listed_attn(gpu, q, kb16, vb16, lst, scale):
