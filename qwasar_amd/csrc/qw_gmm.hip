@@ -50,8 +50,10 @@
 #include "qw_device.h"
 #include "qw_kernels.h"
 
+#include <cfloat>
 #include <climits>
 #include <cmath>
+#include <type_traits>
 
 typedef _Float16 qw_h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 qw_b8 __attribute__((ext_vector_type(8)));
@@ -65,6 +67,14 @@ typedef float qw_f4 __attribute__((ext_vector_type(4)));
 #define QX_CHUNK_ROWS 8192       // rows a dense call stages at a time (bounds its scratch)
 
 // ---- staging -------------------------------------------------------------------
+
+// The power of two that puts a row's largest magnitude m in [2^14, 2^15).
+__device__ __forceinline__ int qx_shift(float m)
+{
+    if (!(m > 0.0f && m <= FLT_MAX)) return 0;
+    const int sh = 15 - __builtin_amdgcn_frexp_expf(m);
+    return sh < -126 ? -126 : sh > 126 ? 126 : sh;
+}
 
 // W waves a row (one under QX_WIDE_K elements, else the workgroup's four: a
 // lane's blocks of 8 stay in registers up to NI of them, so the row is read
@@ -111,11 +121,7 @@ __global__ __launch_bounds__(256) void k_xstage(_Float16 *__restrict__ ah, uint1
         __syncthreads();
         m = fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3]));
     }
-    int sh = 0;
-    if (m > 0.0f && m <= 3.40282346638528859812e+38f) {
-        sh = 15 - __builtin_amdgcn_frexp_expf(m);
-        sh = sh < -126 ? -126 : sh > 126 ? 126 : sh;
-    }
+    const int sh = qx_shift(m);
     if (lane == 0) ex[row] = 24 - sh;
     const float up = __builtin_ldexpf(1.0f, sh), up4 = __builtin_ldexpf(1.0f, sh - 4);
     qw_h8 *hr = reinterpret_cast<qw_h8 *>(ah + (size_t)row * kp);
@@ -601,7 +607,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_xgemm(QxArgs a)
     }
 }
 
-// ---- small dense products ------------------------------------------------------------
+// ---- small products ------------------------------------------------------------
 //
 // Where the whole product is a few microseconds, the stage's launch costs more
 // than it saves (8 rows, 3072 x 512: 23.2 us a call against 25.7): one launch
@@ -610,8 +616,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void k_xgemm(QxArgs a)
 // (exact); the group's map is applied to the fp32 partial:
 //   sum_i (s q_i + b) x_i = s C_g + (b - 1024 s) X_g,
 //   C_g = sum_i (1024 + q_i) x_i,   X_g = sum_i x_i.
-// It needs no scratch, so it also takes the calls, dense or grouped, that
-// would be staged but for scratch that cannot be had.
+// Grouped, it takes short k (qwk_gather_gemm_small); and as it needs no
+// scratch, the calls of either kind that would be staged but for scratch that
+// cannot be had.
 #define QW_GMM_BN 64
 #define QW_GMM_BK 128
 #define QW_GMM_THREADS 256
@@ -640,6 +647,7 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_sgemm(QwGmmArgs a)
     __shared__ __align__(16) uint32_t Bw[QW_GMM_BN][QW_GMM_BSTRIDE];
     __shared__ float Xb[BM][QW_GMM_BK / 8];
     __shared__ float Xs[BM][GPS];
+    __shared__ int sh_s[GATHER ? BM : 1], out_s[4];
 
     // XCD-aware order: consecutive virtual blocks (the n-blocks of one tile,
     // which share its activation rows) land on the same XCD and its L2.
@@ -662,7 +670,21 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_sgemm(QwGmmArgs a)
     const int ln = lane & 15, lg = lane >> 4;
     const int col = n0 + wave * 16 + ln;                 // this lane's weight row
 
+    auto x_row = [&](int m) {
+        const int p = GATHER ? a.perm[first + m] : first + m;
+        return reinterpret_cast<const float4 *>(a.x + (size_t)(GATHER && !a.x_by_pair ? p / a.K : p) * k);
+    };
+    // Grouped rows as they are, which f16 holds well enough where their largest
+    // is 2^-8 to 65504; a tile with one outside is done over with that row
+    // scaled as k_xstage scales it, the others to the same bits.  (The maxima
+    // first would be a trip to memory: 4 us of 20.)
     qw_f4 acc[MT], C[MT];
+    float top[MT];                                       // of rows 16 i + t / 16, this thread's share
+#pragma unroll
+    for (int i = 0; i < MT; i++) top[i] = 0.0f;
+    bool again = false;
+    auto run = [&](auto scaled) __attribute__((always_inline)) {
+    constexpr bool SCALED = decltype(scaled)::value, LOOK = GATHER && !SCALED;
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
         acc[mt] = qw_f4{0.f, 0.f, 0.f, 0.f};
@@ -672,24 +694,40 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_sgemm(QwGmmArgs a)
     for (int k0 = kb; k0 < ke; k0 += QW_GMM_BK) {
         const int klen = min(QW_GMM_BK, ke - k0);
         // Activations: 8-element blocks, f16, written in nibble register order.
-        for (int blk = t; blk < BM * (QW_GMM_BK / 8); blk += QW_GMM_THREADS) {
-            const int m = blk / (QW_GMM_BK / 8), bk = blk % (QW_GMM_BK / 8);
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            const int m = 16 * i + t / 16, bk = t % 16;
             qw_h8u h;
             float bsum = 0.0f;
             if (m < len && bk * 8 < klen) {
-                const int p = GATHER ? a.perm[first + m] : first + m, r = GATHER && !a.x_by_pair ? p / a.K : p;
-                const float4 *xv = reinterpret_cast<const float4 *>(a.x + (size_t)r * k + k0 + bk * 8);
+                const float4 *xv = x_row(m) + (k0 + bk * 8) / 4;
                 const float4 lo = xv[0], hi = xv[1];
                 const float f[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                const float up = SCALED ? __builtin_ldexpf(1.0f, sh_s[m]) : 1.0f;
                 _Float16 q[8];
 #pragma unroll
-                for (int i = 0; i < 8; i++) { q[i] = (_Float16)f[i]; bsum += (float)q[i]; }
+                for (int j = 0; j < 8; j++) {
+                    if (LOOK) top[i] = fmaxf(top[i], fabsf(f[j]));
+                    q[j] = (_Float16)(SCALED ? f[j] * up : f[j]);
+                    bsum += (float)q[j];
+                }
                 h.h = qw_h8{q[0], q[4], q[1], q[5], q[2], q[6], q[3], q[7]};
             } else {
                 h.v = make_uint4(0, 0, 0, 0);
             }
             *reinterpret_cast<uint4 *>(&As[m][bk * 8]) = h.v;
             Xb[m][bk] = bsum;
+        }
+        if (LOOK && k0 + QW_GMM_BK >= ke) {            // (the barriers below hand it on)
+            bool out = false;
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                uint64_t some = __ballot(top[i] > 0.0f), large = __ballot(top[i] >= 0x1p-8f);
+                out |= __ballot(top[i] > 65504.0f && top[i] <= FLT_MAX) != 0;
+#pragma unroll
+                for (int r = 0; r < 4; r++) out |= (large >> 16 * r & 0xFFFF) == 0 && (some >> 16 * r & 0xFFFF) != 0;
+            }
+            if (lane == 0) out_s[wave] = out;
         }
         // Weights: 64 rows x 16 words, one 16-byte load per thread.
         {
@@ -749,6 +787,23 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_sgemm(QwGmmArgs a)
         __syncthreads();
     }
 
+    };
+    run(std::false_type{});
+    if constexpr (GATHER) {
+        again = (out_s[0] | out_s[1] | out_s[2] | out_s[3]) != 0;
+        if (again) {
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+#pragma unroll
+                for (int o = 1; o < 16; o <<= 1) top[i] = fmaxf(top[i], __shfl_xor(top[i], o, 64));
+                const bool in = top[i] >= 0x1p-8f && top[i] <= 65504.0f;
+                if ((t & 15) == 0) sh_s[16 * i + t / 16] = in ? 0 : qx_shift(top[i]);
+            }
+            __syncthreads();
+            run(std::true_type{});
+        }
+    }
+
     float *yo = a.part ? a.part + (size_t)blockIdx.y * a.rows * n : a.y;
     if (col < n) {
 #pragma unroll
@@ -757,7 +812,8 @@ __global__ __launch_bounds__(QW_GMM_THREADS) void k_sgemm(QwGmmArgs a)
             for (int i = 0; i < 4; i++) {
                 const int m = mt * 16 + 4 * lg + i;
                 if (m < len) {
-                    yo[(size_t)(GATHER ? a.perm[first + m] : first + m) * n + col] = acc[mt][i];
+                    yo[(size_t)(GATHER ? a.perm[first + m] : first + m) * n + col] =
+                        again ? __builtin_ldexpf(acc[mt][i], -sh_s[m]) : acc[mt][i];
                 }
             }
         }
@@ -845,6 +901,21 @@ extern "C" int qwk_gather_gemm_blocks(int k, int n, int pairs, int E, int bm)
     return best;
 }
 
+// Whether a grouped product goes unstaged, to k_sgemm: where k is short and the
+// touched experts' weights are few, the stage's launch and the blocks' starts
+// cost more than they save.  us a call over cold banks, 64 x 64 tiles before /
+// staged / this:
+//   256 experts 320 x  640, 33 / 100 / 400 rows of 6  10 / 15 / 11, 19 / 21 / 20, 23 / 32 / 23
+//   128         256 x 1664, 33 / 200 rows of 6        15 / 18 / 16, 19 / 26 / 20
+//   512         256 x 1024,  9 rows of 10              8 / 12 /  9
+// but 33 rows of the last (64 M weights) 23 / 19 / 24, and 640 x 320 of the
+// first, 33 / 100 rows, 16 / 12, 19 / 19 staged.
+extern "C" int qwk_gather_gemm_small(int k, int n, int pairs, int E, int bm)
+{
+    E = E < 1 ? 1 : E;
+    return k <= 320 && bm == 16 && E * (1.0 - exp(-(double)pairs / E)) * n * k <= 58720256.0;
+}
+
 // Few rows a tile: four waves side by side over 128 columns.
 template <int G, bool GATHER>
 static void qx_narrow(hipStream_t s, QxArgs &a, int bm, int ntiles, int splits, int pairs = 0, int E = 0)
@@ -903,7 +974,8 @@ extern "C" int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const in
 {
     if (!gmm_shape_ok(x, m, k, n, group) || K < 1 || (bm != 16 && bm != 32 && bm != 64)) return (int)hipErrorInvalidValue;
     if (max_tiles <= 0 || pairs <= 0) return 0;
-    if (!work || ((uintptr_t)work & 15u) || work_bytes < qwk_gather_gemm_work_bytes(k, pairs, K, x_by_pair, group)) {
+    if (qwk_gather_gemm_small(k, n, pairs, E, bm) || !work || ((uintptr_t)work & 15u) ||
+        work_bytes < qwk_gather_gemm_work_bytes(k, pairs, K, x_by_pair, group)) {
         const QwGmmArgs a = {y, x, m, k, n, 0, (n + QW_GMM_BN - 1) / QW_GMM_BN, k, nullptr, perm, tiles, K, x_by_pair};
         qs_launch<true>(s, a, group, bm, max_tiles, 1);
         return (int)hipGetLastError();

@@ -72,6 +72,8 @@ int qwk_gather_gemm(hipStream_t s, float *y, const float *x, const int32_t *perm
                     const int32_t *tiles, qwk_q4 m, int k, int n, int pairs, int E, int K, int x_by_pair,
                     int group, int bm, int max_tiles, void *work, size_t work_bytes);
 size_t qwk_gather_gemm_work_bytes(int k, int pairs, int K, int x_by_pair, int group);
+/* Whether it goes unstaged (its work is then unused), in one launch. */
+int qwk_gather_gemm_small(int k, int n, int pairs, int E, int bm);
 /* Blocks of 128 columns a workgroup of it runs back to back. */
 int qwk_gather_gemm_blocks(int k, int n, int pairs, int E, int bm);
 

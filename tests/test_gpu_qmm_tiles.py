@@ -9,6 +9,8 @@ name, unsplit and reloaded ones too: test_gpu_qmm_plans.py.)
 Bar: the weights enter exactly and the activations carry one f16 rounding
 (relative 2^-11 at most, 2^-13 rms), so rel-L2 against the fp32 oracle is
 about 2.1e-4; 4e-4 is bounded by twice that."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -145,3 +147,55 @@ def test_staged_product_scale_windows(gpu, rows, k, n, G):
     y, w = yb.read(np.float32, (rows, n)), want(q, x)
     for c0 in range(0, n, 128):
         assert rel_l2(y[:, c0:c0 + 128], w[:, c0:c0 + 128]) < 4e-4, f"columns from {c0}"
+
+
+@pytest.mark.parametrize("E,K,rows,k,n,G,by_pair", [
+    (64, 4, 33, 288, 200, 32, False),     # 9 groups, k % 128 = 32, ragged columns
+    (256, 6, 100, 320, 640, 64, True),
+    (37, 2, 9, 256, 70, 128, True),       # tiles of one pair
+    (16, 4, 40, 64, 64, 64, False),       # one stage of half a block; 10 pairs an expert
+])
+def test_grouped_short_k(gpu, E, K, rows, k, n, G, by_pair):
+    """The unstaged form: rows as f16 holds them, and tiles with a row outside
+    2^-8 .. 65504 done over with that row scaled: rows of 1e6, 1e-6, 1e-30, just
+    either side of both limits, zeros, and one not finite that stays its own.
+    Bar: one row's rounding error is under 6e-4 (above); f16's step of 2^-24 in
+    a row whose largest is 2^-8 adds under 2^-25 / 2^-9.2, its rms, 2e-5."""
+    pairs = rows * K
+    assert C.CDLL(gpu.LIB_PATH).qwk_gather_gemm_small(k, n, pairs, E, gpu.qw_moe_tile_rows(pairs, E))
+    q = synth.make_q4(E + k, "gshort", E * n, k, G)
+    g = np.random.default_rng(pairs)
+    src = pairs if by_pair else rows
+    x = g.uniform(-1, 1, (src, k)).astype(np.float32)
+    x[:, 0] = 1.0
+    for r, m in enumerate((1e6, 1e-6, 1e-30, 65504.0, 65520.0, 2.0 ** -8, 2.0 ** -8.01, 0.0)):
+        x[r] *= np.float32(m)
+    idx = np.stack([g.choice(E, K, replace=False) for _ in range(rows)]).astype(np.int32)
+    B = gpu.Buf
+    wb, sb, bb, ib = B.of(q.w), B.of(q.s), B.of(q.b), B.of(idx)
+    perm, cur, tiles = B(pairs * 4), B(E * 4), B((1 + 3 * gpu.qw_moe_max_tiles(pairs, E)) * 4)
+
+    def product(x):
+        xb, yb = B.of(x), B(pairs * n * 4)
+        c = gpu.qw_cmd_begin()
+        gpu.qw_op_moe_group(c, perm.ref(), tiles.ref(), cur.ref(), ib.ref(), pairs, E)
+        gpu.qw_op_qmm_q4_gather(c, yb.ref(), xb.ref(), perm.ref(), tiles.ref(), wb.ref(), sb.ref(), bb.ref(), k, n,
+                                pairs, E, K, by_pair, G)
+        gpu.run(c, "gather")
+        return yb.read(np.float32, (pairs, n))
+
+    y = product(x)
+    flat, of = idx.ravel(), np.arange(pairs) if by_pair else np.arange(pairs) // K
+    for p in range(pairs):
+        if p < 12 * K or p % 7 == 0:
+            w = q.dequant(flat[p] * n, n).astype(np.float64) @ x[of[p]].astype(np.float64)
+            assert rel_l2(y[p], w) < 7e-4, (p, of[p])
+    x[8, 3] = np.inf
+    y2 = product(x)
+    assert not np.isfinite(y2[of == 8]).any()
+    assert np.isfinite(y2[of != 8]).all()
+    # a row's bits are its own, whatever else is in its tile
+    x[:8] = x[9:17] if src > 17 else 1.0
+    y3 = product(x)
+    assert np.array_equal(y2[of > 8].view(np.uint32), y[of > 8].view(np.uint32))
+    assert np.array_equal(y3[of > 8].view(np.uint32), y[of > 8].view(np.uint32))
