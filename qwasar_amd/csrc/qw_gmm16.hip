@@ -212,12 +212,16 @@ __global__ __launch_bounds__(G16_THREADS, BM == 64 ? 1 : 2) void k_gmm16(Gmm16Ar
     }
     const int tile = xcd * tpx + tl;
     // NT weight tiles of 16 a wave: the item's BNT weight rows; MT row tiles
-    // of 16: those that hold rows of the tile.  An expert of a 2048-token
-    // chunk has about 40 rows, of a 512-token one about 10, and the empty row
-    // tiles' MFMAs and LDS reads stood beside the conversions on the same
-    // SIMDs (of the gate / up launch's cycles at 2048 tokens the matrix unit
-    // now runs 23%, the vector unit 45%): a layer of 512 tokens with skewed
-    // experts 288 -> 279 us, of 2048 1% at most (runs differ by as much).
+    // of 16: one, two or all four of the tile's, by its length.  An expert of a
+    // 2048-token chunk has about 40 rows, of a 512-token one about 10, and the
+    // empty row tiles' MFMAs and LDS reads stood beside the conversions on the
+    // same SIMDs (of the gate / up launch's cycles at 2048 tokens the matrix
+    // unit now runs 23%, the vector unit 45%): a layer of 512 tokens with
+    // skewed experts 288 -> 275 us, of 2048 1% at most (runs differ by as
+    // much).  A body is 10 to 20 KB of code, and two CUs share 64 KB of it: with
+    // one for three row tiles too, and all four for half items, short launches
+    // waited for code (32 experts of 512 x 1024, 300 rows: 18 + 12 us the two
+    // products as one body, 21 + 14 with eight; the layer 103, 106, now 103).
     auto body = [&](auto ntc, auto mtc) {
     constexpr int NT = decltype(ntc)::value, NH = NT / 2, BNT = NT * 16 * (G16_THREADS / 64), MT = decltype(mtc)::value;
     int expert, first, len;
@@ -529,18 +533,16 @@ __global__ __launch_bounds__(G16_THREADS, BM == 64 ? 1 : 2) void k_gmm16(Gmm16Ar
         }
     }
     };
-    auto rows_of = [&](auto mtc) {
-        if (half) body(std::integral_constant<int, 2>{}, mtc);
-        else body(std::integral_constant<int, 4>{}, mtc);
-    };
+    using std::integral_constant;
     if constexpr (BM == 64 && !DENSE && KC == 256) {
-        const int len = a.tiles[3 + 3 * tile], mt = rh == 0 ? min(len, 32) : len;
-        if (mt <= 16) rows_of(std::integral_constant<int, 1>{});
-        else if (mt <= 32) rows_of(std::integral_constant<int, 2>{});
-        else if (mt <= 48) rows_of(std::integral_constant<int, 3>{});
-        else rows_of(std::integral_constant<int, 4>{});
+        const int len = a.tiles[3 + 3 * tile];
+        if (half) body(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+        else if (len <= 16) body(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+        else if (len <= 32) body(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+        else body(integral_constant<int, 4>{}, integral_constant<int, 4>{});
     } else {
-        rows_of(std::integral_constant<int, BM / 16>{});
+        if (half) body(integral_constant<int, 2>{}, integral_constant<int, BM / 16>{});
+        else body(integral_constant<int, 4>{}, integral_constant<int, BM / 16>{});
     }
 }
 
